@@ -185,6 +185,14 @@ int tcfft_query_split(int dims, int n_or_nx, int ny, int n_batch, int *desc, int
 int tcfft_plan_create_r2c_1d(tcfft_plan *plan, int n, int n_batch);
 int tcfft_exec_r2c(tcfft_plan plan, const void *in, void *out, void *stream);
 int tcfft_exec_c2r(tcfft_plan plan, const void *in, void *out, void *stream);
+/* Their adjoints as real-linear maps (the gradients of the two transforms),
+ * with the buffers, sizes and rules of the call of the same shape:
+ *   tcfft_exec_r2c_adjoint: bins -> reals, tcfft_exec_c2r of the bins with
+ *     bins 1..n/2-1 halved (in FP32);
+ *   tcfft_exec_c2r_adjoint: reals -> bins, tcfft_exec_r2c with bins
+ *     1..n/2-1 of the result doubled (before the rounding to FP16). */
+int tcfft_exec_r2c_adjoint(tcfft_plan plan, const void *in, void *out, void *stream);
+int tcfft_exec_c2r_adjoint(tcfft_plan plan, const void *in, void *out, void *stream);
 
 /* Natural-order input, spectrum output in the plan's digit-reversed order
  * (position p holds X[rev[p]], rev = tcfft_gen_rev of the plan's radices):

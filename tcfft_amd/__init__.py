@@ -46,6 +46,7 @@ EXPORTS = (
     "tcfft_plan_create_1d_split", "tcfft_plan_create_1d_tuned", "tcfft_query_1d_split",
     "tcfft_plan_create_r2c_1d", "tcfft_exec_r2c", "tcfft_exec_c2r", "tcfft_permute_to_dropin",
     "tcfft_exec_natural_noalloc", "tcfft_multi_exec_natural", "tcfft_plan_prepare_split", "tcfft_query_split",
+    "tcfft_exec_r2c_adjoint", "tcfft_exec_c2r_adjoint",
 )
 NOALLOC_SCRATCH_BYTES = 64 << 20  # TCFFT_NOALLOC_SCRATCH_BYTES
 OPT_SPLIT_CHUNK = 1
@@ -111,6 +112,8 @@ def lib():
         L.tcfft_exec_r2c.argtypes = [_vp, _vp, _vp, _vp]
         L.tcfft_permute_to_dropin.argtypes = [_vp, _vp, _vp, ctypes.c_int, _vp]
         L.tcfft_exec_c2r.argtypes = [_vp, _vp, _vp, _vp]
+        L.tcfft_exec_r2c_adjoint.argtypes = [_vp, _vp, _vp, _vp]
+        L.tcfft_exec_c2r_adjoint.argtypes = [_vp, _vp, _vp, _vp]
         L.tcfft_exec_dif.argtypes = [_vp, _vp, _vp, ctypes.c_int, _vp]
         L.tcfft_conv_exec.argtypes = [_vp, ctypes.c_int, _vp, _vp, _vp, ctypes.c_int, _vp, _vp]
         L.tcfft_conv_filter_grad.argtypes = [_vp, ctypes.c_int, _vp, _vp, _vp, _vp]
@@ -353,6 +356,14 @@ class PlanR2C(_Plan):
 
     def exec_c2r(self, in_ptr: int, out_ptr: int, stream: int = 0):
         _check(lib().tcfft_exec_c2r(self._h, _vp(in_ptr), _vp(out_ptr), _vp(stream)), "tcfft_exec_c2r")
+
+    def exec_r2c_adjoint(self, in_ptr: int, out_ptr: int, stream: int = 0):
+        """Gradient of exec_r2c: exec_c2r of the bins with bins 1..n/2-1 halved."""
+        _check(lib().tcfft_exec_r2c_adjoint(self._h, _vp(in_ptr), _vp(out_ptr), _vp(stream)), "tcfft_exec_r2c_adjoint")
+
+    def exec_c2r_adjoint(self, in_ptr: int, out_ptr: int, stream: int = 0):
+        """Gradient of exec_c2r: exec_r2c with bins 1..n/2-1 doubled."""
+        _check(lib().tcfft_exec_c2r_adjoint(self._h, _vp(in_ptr), _vp(out_ptr), _vp(stream)), "tcfft_exec_c2r_adjoint")
 
 
 class Plan2D(_Plan):

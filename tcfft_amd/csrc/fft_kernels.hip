@@ -548,6 +548,15 @@ __global__ __launch_bounds__(256) TCFFT_MFMA_BUDGET void k_rows_half_nat(const u
 // Complex side: L+1 FP16 complex words per signal, signal s at word s*(L+1).
 // W_N^k for k = 64j + lane is wn[lane] * wn[64]^j (wn = W_N^0..64, FP64-made
 // FP32 table; the recurrence runs at most 32 steps).
+//
+// ADJ: the adjoint of the other direction instead, viewed as real-linear maps
+// (the gradients of the two transforms).  The forward kernels then double the
+// bins 1..L-1 (the adjoint of c2r) and the inverse kernels halve them on
+// input (the adjoint of r2c), in FP32 at the place where the factors 1/2 of
+// the split stand anyway, so a gradient costs what the transform does (as
+// separate elementwise passes over FP32 copies of the bins it cost three
+// times the transform: 4099 signals of 8192 reals, forward and backward,
+// 169.5 -> 95.4 us).
 
 // k_r2c<T>: the k_rows_nat pass with its output kept in the wave's LDS slice
 // (natural order, same swizzle), then the pairwise untangle in FP32.  The
@@ -555,7 +564,7 @@ __global__ __launch_bounds__(256) TCFFT_MFMA_BUDGET void k_rows_half_nat(const u
 // offset, so each store instruction covers parts of three 128-byte lines,
 // which L2 merges into whole lines before writing back (non-temporal stores
 // of the same pattern: 16384 x 8192, 119.5 us instead of 110.8 us).
-template <int T>
+template <int T, bool ADJ>
 __global__ __launch_bounds__(256) TCFFT_MFMA_BUDGET void k_r2c(const u32* __restrict__ in, u32* __restrict__ out,
                                                              u32 n_tiles, const float2* __restrict__ w4096,
                                                              const float2* __restrict__ wn) {
@@ -581,15 +590,17 @@ __global__ __launch_bounds__(256) TCFFT_MFMA_BUDGET void k_r2c(const u32* __rest
     for (u32 i = 0; i < 16u / T; ++i) {
         if (i * T >= ntl) break;
         u32* const dst = out + (size_t)(line0 + i) * (L + 1u);
-        cf w = {0.5f * wb.x, 0.5f * wb.y};  // W_N^k / 2
+        constexpr float hf = ADJ ? 1.f : 0.5f;  // ADJ: every bin but 0 and L doubled
+        cf w = {hf * wb.x, hf * wb.y};          // W_N^k / 2
 #pragma unroll
         for (u32 j = 0; j < L / 128u; ++j) {
             const u32 k = 64u * j + (u32)lane;  // < L/2
             const cf a = unpack(wl[nat_lds_word(i * L + k)]);
             const cf b = unpack(wl[nat_lds_word(i * L + ((L - k) & (L - 1u)))]);
-            const cf hs = {0.5f * (a.x + b.x), 0.5f * (a.y - b.y)};  // S/2
-            const cf dif = {a.x - b.x, a.y + b.y};                   // D
-            const cf q = cmul(w, dif);                               // W D / 2;  P = i q
+            cf hs = {hf * (a.x + b.x), hf * (a.y - b.y)};  // S/2
+            const cf dif = {a.x - b.x, a.y + b.y};         // D
+            cf q = cmul(w, dif);                           // W D / 2;  P = i q
+            if (ADJ && j == 0 && lane == 0) hs = {0.5f * hs.x, 0.5f * hs.y}, q = {0.5f * q.x, 0.5f * q.y};
             dst[k] = pack(hs.x + q.y, hs.y - q.x);              // S/2 - P
             dst[L - k] = pack(hs.x - q.y, -(hs.y + q.x));       // conj(S/2 + P)
             w = cmul(w, step);
@@ -597,7 +608,7 @@ __global__ __launch_bounds__(256) TCFFT_MFMA_BUDGET void k_r2c(const u32* __rest
         if (lane == 0) {
             // k = L/2: W_N^{L/2} = -i, so X[L/2] = conj Z[L/2]
             const cf a = unpack(wl[nat_lds_word(i * L + L / 2u)]);
-            dst[L / 2u] = pack(a.x, -a.y);
+            dst[L / 2u] = ADJ ? pack(2.f * a.x, -2.f * a.y) : pack(a.x, -a.y);
         }
     }
 }
@@ -605,7 +616,7 @@ __global__ __launch_bounds__(256) TCFFT_MFMA_BUDGET void k_r2c(const u32* __rest
 // k_c2r<T>: Z' formed pairwise from bins read once from global memory (k
 // ascending and L-k descending across lanes), written to the LDS slice in
 // natural order, then the k_rows_nat inverse pass to the real output.
-template <int T>
+template <int T, bool ADJ>
 __global__ __launch_bounds__(256) TCFFT_MFMA_BUDGET void k_c2r(const u32* __restrict__ in, u32* __restrict__ out,
                                                              u32 n_tiles, const float2* __restrict__ w4096,
                                                              const float2* __restrict__ wn) {
@@ -634,15 +645,20 @@ __global__ __launch_bounds__(256) TCFFT_MFMA_BUDGET void k_c2r(const u32* __rest
                 vb[j] = __builtin_nontemporal_load(src + (L - 64u * j - (u32)lane));
             }
             const u32 vm = lane == 0 ? src[L / 2u] : 0u;
-            cf w = {wb.x, -wb.y};  // W_N^-k
+            constexpr float hf = ADJ ? 0.5f : 1.f;  // ADJ: every bin but 0 and L halved
+            cf w = {hf * wb.x, -hf * wb.y};         // W_N^-k
 #pragma unroll
             for (u32 j = 0; j < L / 128u; ++j) {
                 const u32 k = 64u * j + (u32)lane;  // < L/2
                 cf a = unpack(va[j]), b = unpack(vb[j]);
                 if (j == 0 && lane == 0) a.y = b.y = 0.f;  // bins 0 and L: real parts only
-                const cf sum = {a.x + b.x, a.y - b.y};   // S
-                const cf dif = {a.x - b.x, a.y + b.y};   // D
-                const cf q = cmul(w, dif);               // P = i q
+                cf sum = {a.x + b.x, a.y - b.y};           // S
+                const cf dif = {a.x - b.x, a.y + b.y};     // D
+                cf q = cmul(w, dif);                       // P = i q
+                if constexpr (ADJ) {
+                    if (j == 0 && lane == 0) q = {2.f * q.x, 2.f * q.y};
+                    else sum = {0.5f * sum.x, 0.5f * sum.y};
+                }
                 wl[nat_lds_word(i * L + k)] = pack(sum.x - q.y, sum.y + q.x);                  // S + P
                 if (k != 0) wl[nat_lds_word(i * L + (L - k))] = pack(sum.x + q.y, q.x - sum.y);  // conj(S - P)
                 w = cmul(w, step);
@@ -650,7 +666,7 @@ __global__ __launch_bounds__(256) TCFFT_MFMA_BUDGET void k_c2r(const u32* __rest
             if (lane == 0) {
                 // k = L/2: W_N^{-L/2} = i, so Z'[L/2] = 2 conj X[L/2]
                 const cf a = unpack(vm);
-                wl[nat_lds_word(i * L + L / 2u)] = pack(2.f * a.x, -2.f * a.y);
+                wl[nat_lds_word(i * L + L / 2u)] = pack(2.f * hf * a.x, -2.f * hf * a.y);
             }
         }
         __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
@@ -1498,7 +1514,7 @@ __global__ __launch_bounds__(64 * W) TCFFT_MFMA_BUDGET void k_big_nat(
 // two-level table of W_N (same formulas as k_r2c / k_c2r).
 //   SIGN -1: Z (natural, L words per signal) -> bins 0..L (L+1 words per signal)
 //   SIGN +1: bins 0..L -> Z' (L words per signal)
-template <int SIGN>
+template <int SIGN, bool ADJ>
 __global__ __launch_bounds__(256) void k_pairs(const u32* __restrict__ src, u32* __restrict__ dst, u32 l_log2,
                                                u32 n_pairs, const float2* __restrict__ hi,
                                                const float2* __restrict__ lo, u32 lo_bits) {
@@ -1512,30 +1528,32 @@ __global__ __launch_bounds__(256) void k_pairs(const u32* __restrict__ src, u32*
     if constexpr (SIGN < 0) {
         const u32* const z = src + s * L;
         u32* const x = dst + s * (L + 1u);
+        const float hf = ADJ && k != 0 ? 1.f : 0.5f;
         const cf a = unpack(z[k]);
         const cf b = unpack(z[(L - k) & (L - 1u)]);
-        const cf hs = {0.5f * (a.x + b.x), 0.5f * (a.y - b.y)};  // S/2
-        const cf dif = {a.x - b.x, a.y + b.y};                   // D
-        const cf q = cmul(cf{0.5f * w.x, 0.5f * w.y}, dif);      // P = i q
+        const cf hs = {hf * (a.x + b.x), hf * (a.y - b.y)};  // S/2
+        const cf dif = {a.x - b.x, a.y + b.y};               // D
+        const cf q = cmul(cf{hf * w.x, hf * w.y}, dif);      // P = i q
         x[k] = pack(hs.x + q.y, hs.y - q.x);
         x[L - k] = pack(hs.x - q.y, -(hs.y + q.x));
         if (k == 0) {
             const cf m = unpack(z[half]);
-            x[half] = pack(m.x, -m.y);
+            x[half] = ADJ ? pack(2.f * m.x, -2.f * m.y) : pack(m.x, -m.y);
         }
     } else {
         const u32* const x = src + s * (L + 1u);
         u32* const z = dst + s * L;
         cf a = unpack(x[k]), b = unpack(x[L - k]);
         if (k == 0) a.y = b.y = 0.f;  // bins 0 and L: real parts only
-        const cf sum = {a.x + b.x, a.y - b.y};
+        const float hf = ADJ && k != 0 ? 0.5f : 1.f;
+        const cf sum = {hf * (a.x + b.x), hf * (a.y - b.y)};
         const cf dif = {a.x - b.x, a.y + b.y};
-        const cf q = cmul(cf{w.x, -w.y}, dif);  // W_N^-k D; P = i q
+        const cf q = cmul(cf{hf * w.x, -hf * w.y}, dif);  // W_N^-k D; P = i q
         z[k] = pack(sum.x - q.y, sum.y + q.x);
         if (k != 0) z[L - k] = pack(sum.x + q.y, q.x - sum.y);
         if (k == 0) {
             const cf m = unpack(x[half]);
-            z[half] = pack(2.f * m.x, -2.f * m.y);
+            z[half] = ADJ ? pack(m.x, -m.y) : pack(2.f * m.x, -2.f * m.y);
         }
     }
 }
@@ -1550,7 +1568,7 @@ __global__ __launch_bounds__(256) void k_pairs(const u32* __restrict__ src, u32*
 // k_r2c_big<W>: the k_big_nat pass with the final results kept in registers
 // (big_phase2_regs), staged in natural order over the whole LDS (4096*W
 // words, lane-contiguous 16-byte writes), then the untangle.
-template <int W>
+template <int W, bool ADJ>
 __global__ __launch_bounds__(64 * W) TCFFT_MFMA_BUDGET void k_r2c_big(
     const u32* __restrict__ in, u32* __restrict__ out, const float2* __restrict__ w4096,
     const float2* __restrict__ wn_hi, const float2* __restrict__ wn_lo, u32 wn_lo_bits,
@@ -1600,28 +1618,30 @@ __global__ __launch_bounds__(64 * W) TCFFT_MFMA_BUDGET void k_r2c_big(
     __syncthreads();
     u32* const dst = out + (size_t)sig * (L + 1u);
     const cf step = {ws.x, ws.y};
-    cf tw = {0.5f * wb.x, 0.5f * wb.y};  // W_N^k / 2
+    constexpr float hf = ADJ ? 1.f : 0.5f;
+    cf tw = {hf * wb.x, hf * wb.y};  // W_N^k / 2
 #pragma unroll 8
     for (u32 j = 0; j < 32u; ++j) {
         const u32 k = 64u * (j * W + w) + (u32)lane;  // < L/2
         const cf a = unpack(lds[k]);
         const cf b = unpack(lds[(L - k) & (L - 1u)]);
-        const cf hs = {0.5f * (a.x + b.x), 0.5f * (a.y - b.y)};
+        cf hs = {hf * (a.x + b.x), hf * (a.y - b.y)};
         const cf dif = {a.x - b.x, a.y + b.y};
-        const cf q = cmul(tw, dif);
+        cf q = cmul(tw, dif);
+        if (ADJ && k == 0) hs = {0.5f * hs.x, 0.5f * hs.y}, q = {0.5f * q.x, 0.5f * q.y};
         dst[k] = pack(hs.x + q.y, hs.y - q.x);
         dst[L - k] = pack(hs.x - q.y, -(hs.y + q.x));
         tw = cmul(tw, step);
     }
     if (w == 0 && lane == 0) {
         const cf a = unpack(lds[L / 2u]);
-        dst[L / 2u] = pack(a.x, -a.y);
+        dst[L / 2u] = ADJ ? pack(2.f * a.x, -2.f * a.y) : pack(a.x, -a.y);
     }
 }
 
 // k_c2r_big<W>: Z' formed pairwise from the bins into the LDS staging of
 // k_big_nat (its swizzle), then the k_big_nat inverse pass to the real output.
-template <int W>
+template <int W, bool ADJ>
 __global__ __launch_bounds__(64 * W) TCFFT_MFMA_BUDGET void k_c2r_big(
     const u32* __restrict__ in, u32* __restrict__ out, const float2* __restrict__ w4096,
     const float2* __restrict__ wn_hi, const float2* __restrict__ wn_lo, u32 wn_lo_bits,
@@ -1648,22 +1668,27 @@ __global__ __launch_bounds__(64 * W) TCFFT_MFMA_BUDGET void k_c2r_big(
         }
         const u32 vm = (w == 0 && lane == 0) ? src[L / 2u] : 0u;
         const cf step = {ws.x, -ws.y};
-        cf tw = {wb.x, -wb.y};  // W_N^-k
+        constexpr float hf = ADJ ? 0.5f : 1.f;
+        cf tw = {hf * wb.x, -hf * wb.y};  // W_N^-k
 #pragma unroll
         for (u32 j = 0; j < 32u; ++j) {
             const u32 k = 64u * (j * W + w) + (u32)lane;
             cf a = unpack(va[j]), b = unpack(vb[j]);
             if (k == 0) a.y = b.y = 0.f;  // bins 0 and L: real parts only
-            const cf sum = {a.x + b.x, a.y - b.y};
+            cf sum = {a.x + b.x, a.y - b.y};
             const cf dif = {a.x - b.x, a.y + b.y};
-            const cf q = cmul(tw, dif);
+            cf q = cmul(tw, dif);
+            if constexpr (ADJ) {
+                if (k == 0) q = {2.f * q.x, 2.f * q.y};
+                else sum = {0.5f * sum.x, 0.5f * sum.y};
+            }
             lds[nat_big_word<W>(k)] = pack(sum.x - q.y, sum.y + q.x);
             if (k != 0) lds[nat_big_word<W>(L - k)] = pack(sum.x + q.y, q.x - sum.y);
             tw = cmul(tw, step);
         }
         if (w == 0 && lane == 0) {
             const cf a = unpack(vm);
-            lds[nat_big_word<W>(L / 2u)] = pack(2.f * a.x, -2.f * a.y);
+            lds[nat_big_word<W>(L / 2u)] = pack(2.f * hf * a.x, -2.f * hf * a.y);
         }
     }
     __syncthreads();
@@ -1924,9 +1949,9 @@ hipError_t launch_rows_nat(int T, const u32* in, u32* out, u32 n_tiles, int sign
 }
 
 template <int T>
-static hipError_t launch_r2c_t(int sign, const u32* in, u32* out, u32 n_tiles, const float2* w4096,
+static hipError_t launch_r2c_t(int sign, bool adjoint, const u32* in, u32* out, u32 n_tiles, const float2* w4096,
                                const float2* wn, hipStream_t st) {
-    auto k = sign < 0 ? k_r2c<T> : k_c2r<T>;
+    auto k = sign < 0 ? (adjoint ? k_r2c<T, true> : k_r2c<T, false>) : (adjoint ? k_c2r<T, true> : k_c2r<T, false>);
     const u32 waves = (n_tiles + 15) / 16;
     const u32 wg = slice_wg(k, waves);
     const size_t lds = wg * 4096 * sizeof(u32);  // 16 KiB per wave
@@ -1937,12 +1962,13 @@ static hipError_t launch_r2c_t(int sign, const u32* in, u32* out, u32 n_tiles, c
 }
 
 template <int W>
-static hipError_t launch_r2c_big_t(int sign, const u32* in, u32* out, u32 n_signals, const float2* w4096,
+static hipError_t launch_r2c_big_t(int sign, bool adjoint, const u32* in, u32* out, u32 n_signals, const float2* w4096,
                                    const float2* wn_hi, const float2* wn_lo, u32 lo_bits, const float2* wn,
                                    StartSched sched, hipStream_t st) {
     const size_t lds = 4096u * W * sizeof(u32);  // the whole half-size signal
     static_assert(4096u * W >= (size_t)BigCfg<W>::LDS_WORDS, "LDS covers the exchange");
-    auto k = sign < 0 ? k_r2c_big<W> : k_c2r_big<W>;
+    auto k = sign < 0 ? (adjoint ? k_r2c_big<W, true> : k_r2c_big<W, false>)
+                      : (adjoint ? k_c2r_big<W, true> : k_c2r_big<W, false>);
     const KernelInfo ki = kernel_info(k, 64 * W, lds);
     if (ki.lds_status != hipSuccess) return ki.lds_status;
     if (sched.groups == 0) sched.delay = 0;
@@ -1951,35 +1977,36 @@ static hipError_t launch_r2c_big_t(int sign, const u32* in, u32* out, u32 n_sign
     return hipGetLastError();
 }
 
-hipError_t launch_r2c_big(int W, int sign, const u32* in, u32* out, u32 n_signals, const float2* w4096,
+hipError_t launch_r2c_big(int W, int sign, bool adjoint, const u32* in, u32* out, u32 n_signals, const float2* w4096,
                           const float2* wn_hi, const float2* wn_lo, u32 lo_bits, const float2* wn, StartSched sched,
                           hipStream_t st) {
     switch (W) {
-    case 2: return launch_r2c_big_t<2>(sign, in, out, n_signals, w4096, wn_hi, wn_lo, lo_bits, wn, sched, st);
-    case 4: return launch_r2c_big_t<4>(sign, in, out, n_signals, w4096, wn_hi, wn_lo, lo_bits, wn, sched, st);
-    case 8: return launch_r2c_big_t<8>(sign, in, out, n_signals, w4096, wn_hi, wn_lo, lo_bits, wn, sched, st);
+    case 2: return launch_r2c_big_t<2>(sign, adjoint, in, out, n_signals, w4096, wn_hi, wn_lo, lo_bits, wn, sched, st);
+    case 4: return launch_r2c_big_t<4>(sign, adjoint, in, out, n_signals, w4096, wn_hi, wn_lo, lo_bits, wn, sched, st);
+    case 8: return launch_r2c_big_t<8>(sign, adjoint, in, out, n_signals, w4096, wn_hi, wn_lo, lo_bits, wn, sched, st);
     default: return hipErrorInvalidValue;
     }
 }
 
-hipError_t launch_real_pairs(int sign, const u32* in, u32* out, u32 l_log2, u32 n_signals, const float2* hi,
+hipError_t launch_real_pairs(int sign, bool adjoint, const u32* in, u32* out, u32 l_log2, u32 n_signals, const float2* hi,
                              const float2* lo, u32 lo_bits, hipStream_t st) {
     if (l_log2 < 2 || l_log2 > 26) return hipErrorInvalidValue;
     const u32 pairs = n_signals << (l_log2 - 1u);
     const u32 blocks = (pairs + 255u) / 256u;
-    if (sign < 0) hipLaunchKernelGGL(k_pairs<-1>, dim3(blocks), dim3(256), 0, st, in, out, l_log2, pairs, hi, lo, lo_bits);
-    else hipLaunchKernelGGL(k_pairs<+1>, dim3(blocks), dim3(256), 0, st, in, out, l_log2, pairs, hi, lo, lo_bits);
+    auto k = sign < 0 ? (adjoint ? k_pairs<-1, true> : k_pairs<-1, false>)
+                      : (adjoint ? k_pairs<+1, true> : k_pairs<+1, false>);
+    hipLaunchKernelGGL(k, dim3(blocks), dim3(256), 0, st, in, out, l_log2, pairs, hi, lo, lo_bits);
     return hipGetLastError();
 }
 
-hipError_t launch_r2c(int T, int sign, const u32* in, u32* out, u32 n_tiles, const float2* w4096, const float2* wn,
+hipError_t launch_r2c(int T, int sign, bool adjoint, const u32* in, u32* out, u32 n_tiles, const float2* w4096, const float2* wn,
                       hipStream_t st) {
     switch (T) {
-    case 1: return launch_r2c_t<1>(sign, in, out, n_tiles, w4096, wn, st);
-    case 2: return launch_r2c_t<2>(sign, in, out, n_tiles, w4096, wn, st);
-    case 4: return launch_r2c_t<4>(sign, in, out, n_tiles, w4096, wn, st);
-    case 8: return launch_r2c_t<8>(sign, in, out, n_tiles, w4096, wn, st);
-    case 16: return launch_r2c_t<16>(sign, in, out, n_tiles, w4096, wn, st);
+    case 1: return launch_r2c_t<1>(sign, adjoint, in, out, n_tiles, w4096, wn, st);
+    case 2: return launch_r2c_t<2>(sign, adjoint, in, out, n_tiles, w4096, wn, st);
+    case 4: return launch_r2c_t<4>(sign, adjoint, in, out, n_tiles, w4096, wn, st);
+    case 8: return launch_r2c_t<8>(sign, adjoint, in, out, n_tiles, w4096, wn, st);
+    case 16: return launch_r2c_t<16>(sign, adjoint, in, out, n_tiles, w4096, wn, st);
     default: return hipErrorInvalidValue;
     }
 }

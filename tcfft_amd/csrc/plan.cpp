@@ -897,15 +897,63 @@ namespace {
 // Real-input kernels of a real-input plan: the row kernels for n <= 8192, the
 // workgroup kernels (the half-size plan's 4096W-point first pass and its
 // twiddle tables) for n = 16384..65536.
-hipError_t launch_real(tcfft_plan_s* p, int sign, const void* in, void* out, hipStream_t st) {
+hipError_t launch_real(tcfft_plan_s* p, int sign, bool adjoint, const void* in, void* out, hipStream_t st) {
     const uint32_t half = (uint32_t)p->real_n / 2, batch = (uint32_t)p->lay.batch;
     if (half <= 4096)
-        return tcfft::launch_r2c((int)(half / 256), sign, (const uint32_t*)in, (uint32_t*)out, batch * (half / 256),
+        return tcfft::launch_r2c((int)(half / 256), sign, adjoint, (const uint32_t*)in, (uint32_t*)out, batch * (half / 256),
                                  p->w4096, p->w_real, st);
     const Pass& ps = p->lay.passes[0];
     if (ps.kind != 2 || ps.radix != (int)(half / 4096)) return hipErrorInvalidValue;
-    return tcfft::launch_r2c_big(ps.radix, sign, (const uint32_t*)in, (uint32_t*)out, batch, p->w4096, ps.big_hi,
+    return tcfft::launch_r2c_big(ps.radix, sign, adjoint, (const uint32_t*)in, (uint32_t*)out, batch, p->w4096, ps.big_hi,
                                  ps.big_lo, ps.big_M_log2 / 2, p->w_real, big_sched(p, ps.radix), st);
+}
+
+// n reals per signal to n/2 + 1 bins: the real-input transform or, with
+// `adjoint`, the adjoint of the inverse one.
+int exec_to_bins(tcfft_plan plan, bool adjoint, const void* in, void* out, void* stream) {
+    if (!valid(plan)) return TCFFT_INVALID_PLAN;
+    if (!plan->real_n) return TCFFT_INVALID_PLAN;
+    const size_t half = (size_t)plan->real_n / 2, batch = (size_t)plan->lay.batch;
+    const uintptr_t a = (uintptr_t)in, b = (uintptr_t)out;
+    if (!in || !out || (a & 15u) || (b & 3u)) return TCFFT_INVALID_POINTER;
+    if (a < b + (half + 1) * batch * 4u && b < a + half * batch * 4u) return TCFFT_INVALID_POINTER;  // overlap
+    DeviceGuard guard(plan->device);
+    if (plan->real_ws) {
+        // n > 65536: the n/2-point transform of z into the workspace, then the split
+        int rc = tcfft_exec_natural(plan, in, plan->real_ws, TCFFT_FORWARD, stream);
+        if (rc) return rc;
+        const hipError_t e = tcfft::launch_real_pairs(-1, adjoint, plan->real_ws, (uint32_t*)out,
+                                                      (uint32_t)ilog2((uint32_t)half), (uint32_t)batch,
+                                                      plan->w_real_pair.first, plan->w_real_pair.second,
+                                                      (uint32_t)ilog2((uint32_t)plan->real_n) / 2, (hipStream_t)stream);
+        return e == hipSuccess ? TCFFT_SUCCESS : hip_fail(e);
+    }
+    hipError_t e = launch_real(plan, -1, adjoint, in, out, (hipStream_t)stream);
+    if (e != hipSuccess) return hip_fail(e);
+    return TCFFT_SUCCESS;
+}
+
+// n/2 + 1 bins per signal to n reals, likewise.
+int exec_from_bins(tcfft_plan plan, bool adjoint, const void* in, void* out, void* stream) {
+    if (!valid(plan)) return TCFFT_INVALID_PLAN;
+    if (!plan->real_n) return TCFFT_INVALID_PLAN;
+    const size_t half = (size_t)plan->real_n / 2, batch = (size_t)plan->lay.batch;
+    const uintptr_t a = (uintptr_t)in, b = (uintptr_t)out;
+    if (!in || !out || (a & 3u) || (b & 15u)) return TCFFT_INVALID_POINTER;
+    if (a < b + half * batch * 4u && b < a + (half + 1) * batch * 4u) return TCFFT_INVALID_POINTER;  // overlap
+    DeviceGuard guard(plan->device);
+    if (plan->real_ws) {
+        // n > 65536: the split into the workspace, then the inverse n/2-point transform
+        const hipError_t e = tcfft::launch_real_pairs(+1, adjoint, (const uint32_t*)in, plan->real_ws,
+                                                      (uint32_t)ilog2((uint32_t)half), (uint32_t)batch,
+                                                      plan->w_real_pair.first, plan->w_real_pair.second,
+                                                      (uint32_t)ilog2((uint32_t)plan->real_n) / 2, (hipStream_t)stream);
+        if (e != hipSuccess) return hip_fail(e);
+        return tcfft_exec_natural(plan, plan->real_ws, out, TCFFT_INVERSE, stream);
+    }
+    hipError_t e = launch_real(plan, +1, adjoint, in, out, (hipStream_t)stream);
+    if (e != hipSuccess) return hip_fail(e);
+    return TCFFT_SUCCESS;
 }
 
 }  // namespace
@@ -951,48 +999,19 @@ int tcfft_plan_create_r2c_1d(tcfft_plan* plan, int n, int n_batch) {
 }
 
 int tcfft_exec_r2c(tcfft_plan plan, const void* in, void* out, void* stream) {
-    if (!valid(plan)) return TCFFT_INVALID_PLAN;
-    if (!plan->real_n) return TCFFT_INVALID_PLAN;
-    const size_t half = (size_t)plan->real_n / 2, batch = (size_t)plan->lay.batch;
-    const uintptr_t a = (uintptr_t)in, b = (uintptr_t)out;
-    if (!in || !out || (a & 15u) || (b & 3u)) return TCFFT_INVALID_POINTER;
-    if (a < b + (half + 1) * batch * 4u && b < a + half * batch * 4u) return TCFFT_INVALID_POINTER;  // overlap
-    DeviceGuard guard(plan->device);
-    if (plan->real_ws) {
-        // n > 65536: the n/2-point transform of z into the workspace, then the split
-        int rc = tcfft_exec_natural(plan, in, plan->real_ws, TCFFT_FORWARD, stream);
-        if (rc) return rc;
-        const hipError_t e = tcfft::launch_real_pairs(-1, plan->real_ws, (uint32_t*)out,
-                                                      (uint32_t)ilog2((uint32_t)half), (uint32_t)batch,
-                                                      plan->w_real_pair.first, plan->w_real_pair.second,
-                                                      (uint32_t)ilog2((uint32_t)plan->real_n) / 2, (hipStream_t)stream);
-        return e == hipSuccess ? TCFFT_SUCCESS : hip_fail(e);
-    }
-    hipError_t e = launch_real(plan, -1, in, out, (hipStream_t)stream);
-    if (e != hipSuccess) return hip_fail(e);
-    return TCFFT_SUCCESS;
+    return exec_to_bins(plan, false, in, out, stream);
 }
 
 int tcfft_exec_c2r(tcfft_plan plan, const void* in, void* out, void* stream) {
-    if (!valid(plan)) return TCFFT_INVALID_PLAN;
-    if (!plan->real_n) return TCFFT_INVALID_PLAN;
-    const size_t half = (size_t)plan->real_n / 2, batch = (size_t)plan->lay.batch;
-    const uintptr_t a = (uintptr_t)in, b = (uintptr_t)out;
-    if (!in || !out || (a & 3u) || (b & 15u)) return TCFFT_INVALID_POINTER;
-    if (a < b + half * batch * 4u && b < a + (half + 1) * batch * 4u) return TCFFT_INVALID_POINTER;  // overlap
-    DeviceGuard guard(plan->device);
-    if (plan->real_ws) {
-        // n > 65536: the split into the workspace, then the inverse n/2-point transform
-        const hipError_t e = tcfft::launch_real_pairs(+1, (const uint32_t*)in, plan->real_ws,
-                                                      (uint32_t)ilog2((uint32_t)half), (uint32_t)batch,
-                                                      plan->w_real_pair.first, plan->w_real_pair.second,
-                                                      (uint32_t)ilog2((uint32_t)plan->real_n) / 2, (hipStream_t)stream);
-        if (e != hipSuccess) return hip_fail(e);
-        return tcfft_exec_natural(plan, plan->real_ws, out, TCFFT_INVERSE, stream);
-    }
-    hipError_t e = launch_real(plan, +1, in, out, (hipStream_t)stream);
-    if (e != hipSuccess) return hip_fail(e);
-    return TCFFT_SUCCESS;
+    return exec_from_bins(plan, false, in, out, stream);
+}
+
+int tcfft_exec_c2r_adjoint(tcfft_plan plan, const void* in, void* out, void* stream) {
+    return exec_to_bins(plan, true, in, out, stream);
+}
+
+int tcfft_exec_r2c_adjoint(tcfft_plan plan, const void* in, void* out, void* stream) {
+    return exec_from_bins(plan, true, in, out, stream);
 }
 
 int tcfft_plan_prepare_split(tcfft_plan plan) {

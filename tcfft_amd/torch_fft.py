@@ -204,32 +204,34 @@ def _rplan(n: int, batch: int, device: torch.device) -> PlanR2C:
     return _cached(_RPLANS, (n, batch, device.index), make)
 
 
-def _r2c(x: torch.Tensor) -> torch.Tensor:
+def _r2c(x: torch.Tensor, adjoint: bool = False) -> torch.Tensor:
+    """rfft of real x or, with adjoint, the adjoint of c2r (bins 1..n/2-1
+    doubled, inside the kernel)."""
     if x.device.type != "cuda" or x.dtype != torch.float16 or x.dim() < 1:
         raise RuntimeError("expected a real fp16 CUDA (HIP) tensor of shape [..., n]")
     x = x.contiguous()
     n = x.shape[-1]
     batch = x.numel() // n
     out = torch.empty(x.shape[:-1] + (n // 2 + 1, 2), dtype=torch.float16, device=x.device)
-    _rplan(n, batch, x.device).exec_r2c(x.data_ptr(), out.data_ptr(), torch.cuda.current_stream(x.device).cuda_stream)
+    plan = _rplan(n, batch, x.device)
+    call = plan.exec_c2r_adjoint if adjoint else plan.exec_r2c
+    call(x.data_ptr(), out.data_ptr(), torch.cuda.current_stream(x.device).cuda_stream)
     return out
 
 
-def _c2r(X: torch.Tensor, n: int) -> torch.Tensor:
+def _c2r(X: torch.Tensor, n: int, adjoint: bool = False) -> torch.Tensor:
+    """c2r of the bins X or, with adjoint, the adjoint of rfft (bins 1..n/2-1
+    halved, inside the kernel)."""
     _check(X)
     if X.shape[-2] != n // 2 + 1:
         raise RuntimeError(f"expected {n // 2 + 1} bins for n = {n}, got {X.shape[-2]}")
     X = X.contiguous()
     batch = X.numel() // (2 * (n // 2 + 1))
     out = torch.empty(X.shape[:-2] + (n,), dtype=torch.float16, device=X.device)
-    _rplan(n, batch, X.device).exec_c2r(X.data_ptr(), out.data_ptr(), torch.cuda.current_stream(X.device).cuda_stream)
+    plan = _rplan(n, batch, X.device)
+    call = plan.exec_r2c_adjoint if adjoint else plan.exec_c2r
+    call(X.data_ptr(), out.data_ptr(), torch.cuda.current_stream(X.device).cuda_stream)
     return out
-
-
-def _scale_interior(t: torch.Tensor, f: float) -> torch.Tensor:
-    v = t.float()
-    v[..., 1:-1, :] *= f
-    return v.half()
 
 
 class _RFFT(torch.autograd.Function):
@@ -240,7 +242,7 @@ class _RFFT(torch.autograd.Function):
 
     @staticmethod
     def backward(ctx, g):
-        return _c2r(_scale_interior(g, 0.5), ctx.n)
+        return _c2r(g.half(), ctx.n, adjoint=True)
 
 
 class _C2R(torch.autograd.Function):
@@ -250,7 +252,7 @@ class _C2R(torch.autograd.Function):
 
     @staticmethod
     def backward(ctx, g):
-        return _scale_interior(_r2c(g), 2.0), None
+        return _r2c(g, adjoint=True), None
 
 
 def rfft(x: torch.Tensor) -> torch.Tensor:
