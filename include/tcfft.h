@@ -142,16 +142,18 @@ int tcfft_exec_split(tcfft_plan plan, const void *in, void *out, int direction, 
 
 /* Prepares a complex plan for tcfft_exec_split at its size: builds the
  * pass list (1D n = 65536 as two 256 x 256 passes; other shapes as passes
- * of 16..256 rows, 2..4 per axis), uploads their twiddle tables and
- * allocates a workspace of 8 bytes per element, so that tcfft_exec_split
- * allocates nothing (graph-capturable) and runs in place.  One workspace per
+ * of 16..256 rows, 2..4 per axis, of which the passes over contiguous lines
+ * of at most 4096 points run as one kernel), uploads their twiddle tables and
+ * allocates a workspace of 8 bytes per element where a pass needs one, so that
+ * tcfft_exec_split allocates nothing (graph-capturable) and runs in place.
+ * One workspace per
  * plan: split calls on one plan must not overlap (out-of-place calls on a 1D
  * plan of at most 65536 points do not use it and may), and this call must not
  * run concurrently with any other call on the plan.  Idempotent.  No
  * counterpart in the reference. */
 int tcfft_plan_prepare_split(tcfft_plan plan);
 
-/* The split-precision pass list tcfft_plan_prepare_split builds for a shape
+/* The split-precision pass list tcfft_plan_prepare_split starts from for a shape
  * (dims 1: n_or_nx = n, ny ignored; dims 2: nx x ny), computed on the host
  * without a device.  Pass i fills desc[5i .. 5i+4] = {R, log2 Q, log2 Qlo,
  * log2 M or 0, units}: each signal seen as R rows x Q columns, the R-point

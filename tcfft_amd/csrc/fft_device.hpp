@@ -325,4 +325,37 @@ __device__ __forceinline__ void small_dft<8>(cf* v, int sign) {
     v[7] = csub(e[3], w3);
 }
 
+template <>
+__device__ __forceinline__ void small_dft<16>(cf* v, int sign) {
+    // 4 x 4: n = 4 n2 + n1, X[k1 + 4 k2] = sum_n1 W_4^{n1 k2} W_16^{n1 k1} (DFT-4 over n2)[k1]
+    const float h = 0.70710678118654752f, c = 0.92387953251128674f, s = 0.38268343236508977f;
+    cf y[4][4];
+#pragma unroll
+    for (int n1 = 0; n1 < 4; ++n1) {
+#pragma unroll
+        for (int n2 = 0; n2 < 4; ++n2) y[n1][n2] = v[4 * n2 + n1];
+        small_dft<4>(y[n1], sign);
+    }
+    auto rot8 = [&](cf a, float re) -> cf {  // times (re, sign) * h, re = +-1
+        const cf b = {re * a.x - sign * a.y, re * a.y + sign * a.x};
+        return {h * b.x, h * b.y};
+    };
+    y[1][1] = cmul(y[1][1], cf{c, sign * s});
+    y[1][2] = rot8(y[1][2], 1.f);
+    y[1][3] = cmul(y[1][3], cf{s, sign * c});
+    y[2][1] = rot8(y[2][1], 1.f);
+    y[2][2] = mul_si(y[2][2], sign);
+    y[2][3] = rot8(y[2][3], -1.f);
+    y[3][1] = cmul(y[3][1], cf{s, sign * c});
+    y[3][2] = rot8(y[3][2], -1.f);
+    y[3][3] = cmul(y[3][3], cf{-c, sign * -s});
+#pragma unroll
+    for (int k1 = 0; k1 < 4; ++k1) {
+        cf x[4] = {y[0][k1], y[1][k1], y[2][k1], y[3][k1]};
+        small_dft<4>(x, sign);
+#pragma unroll
+        for (int k2 = 0; k2 < 4; ++k2) v[k1 + 4 * k2] = x[k2];
+    }
+}
+
 }  // namespace tcfft

@@ -83,6 +83,12 @@ struct SplitPassArgs {
 hipError_t launch_split_pass(int R, bool row, const float2* src, float2* dst, const SplitPassArgs& a, int sign,
                              const float2* w4096, StartSched sched, hipStream_t st);
 
+// Split precision over contiguous lines of 256*T points (T = 1, 2, 4, 8, 16)
+// in one pass, natural order in and out, in place or out of place; cus = the
+// device's compute units.
+hipError_t launch_split_rows(int T, const float2* src, float2* dst, uint32_t n_lines, int sign, const float2* w4096,
+                             StartSched sched, uint32_t cus, hipStream_t st);
+
 // Uneven batch: one task = signals [first, first + count) of one size class.
 struct MultiTask {
     uint32_t size_log2;

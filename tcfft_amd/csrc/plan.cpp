@@ -235,6 +235,7 @@ struct tcfft_plan_s {
     // for the passes whose transposed store cannot go in place.
     struct SplitStep {
         int R;
+        int row_tiles;     // > 0: one pass over contiguous lines of 256*row_tiles points (k_split_rows), a.units lines
         bool row;          // Qlo = 1 (transposed row store)
         bool transposing;  // not the last pass of its axis: src != dst
         tcfft::SplitPassArgs a;
@@ -390,6 +391,28 @@ int split_steps_of(int dims, int n_or_nx, int ny, int batch, std::vector<tcfft_p
     // axis with the ny columns of each image
     const int rc = split_axis(ilog2((uint32_t)ny), 0, (uint32_t)batch * (uint32_t)n_or_nx, steps);
     return rc ? rc : split_axis(ilog2((uint32_t)n_or_nx), ilog2((uint32_t)ny), (uint32_t)batch, steps);
+}
+
+// The passes tcfft_exec_split runs for that list: the passes of a contiguous
+// axis of 256..4096 points are one kernel over whole lines (k_split_rows, one
+// HBM round trip instead of one per pass), the others as listed.
+int split_exec_steps_of(int dims, int n_or_nx, int ny, int batch, std::vector<tcfft_plan_s::SplitStep>& steps) {
+    std::vector<tcfft_plan_s::SplitStep> list;
+    const int rc = split_steps_of(dims, n_or_nx, ny, batch, list);
+    if (rc) return rc;
+    const int line = dims == 1 ? n_or_nx : ny;
+    size_t i = 0;
+    if (line <= 4096) {
+        while (list[i].transposing) ++i;  // the contiguous axis's passes end with the first one without a twiddle
+        ++i;
+        tcfft_plan_s::SplitStep s{};
+        s.R = line;
+        s.row_tiles = line / 256;
+        s.a.units = (uint32_t)batch * (dims == 1 ? 1u : (uint32_t)n_or_nx);
+        steps.push_back(s);
+    }
+    steps.insert(steps.end(), list.begin() + (long)i, list.end());
+    return TCFFT_SUCCESS;
 }
 
 int finish_plan(tcfft_plan_s* p) {
@@ -1021,7 +1044,7 @@ int tcfft_plan_prepare_split(tcfft_plan plan) {
     DeviceGuard guard(plan->device);
     const Layout& L = plan->lay;
     std::vector<tcfft_plan_s::SplitStep> steps;
-    int rc = split_steps_of(L.dims, L.dims == 1 ? L.n : L.nx, L.ny, L.batch, steps);
+    int rc = split_exec_steps_of(L.dims, L.dims == 1 ? L.n : L.nx, L.ny, L.batch, steps);
     if (rc) return rc;
     if (L.dims == 1 && L.n == 65536) {
         std::pair<float2*, float2*> t;
@@ -1036,11 +1059,16 @@ int tcfft_plan_prepare_split(tcfft_plan plan) {
         s.a.hi = t.first;
         s.a.lo = t.second;
     }
-    void* ws = nullptr;
-    const hipError_t e = hipMalloc(&ws, plan->total * 8u);
-    if (e != hipSuccess) return hip_fail(e);
-    plan->allocs.push_back(ws);
-    plan->split_ws = (float2*)ws;
+    // a workspace only where some pass cannot go in place
+    bool need = L.dims == 1 && L.n == 65536;
+    for (const auto& s : steps) need |= s.transposing;
+    if (need) {
+        void* ws = nullptr;
+        const hipError_t e = hipMalloc(&ws, plan->total * 8u);
+        if (e != hipSuccess) return hip_fail(e);
+        plan->allocs.push_back(ws);
+        plan->split_ws = (float2*)ws;
+    }
     plan->split_steps = std::move(steps);
     plan->split_ready = true;
     return TCFFT_SUCCESS;
@@ -1100,7 +1128,10 @@ int tcfft_exec_split(tcfft_plan plan, const void* in, void* out, int direction, 
     const float2* src = (const float2*)in;
     for (int j = 0; j < P; ++j) {
         const hipError_t e =
-            tcfft::launch_split_pass(S[j].R, S[j].row, src, dst[j], S[j].a, direction, plan->w4096, sched, st);
+            S[j].row_tiles
+                ? tcfft::launch_split_rows(S[j].row_tiles, src, dst[j], S[j].a.units, direction, plan->w4096, sched,
+                                           (uint32_t)plan->cus, st)
+                : tcfft::launch_split_pass(S[j].R, S[j].row, src, dst[j], S[j].a, direction, plan->w4096, sched, st);
         if (e != hipSuccess) return hip_fail(e);
         src = dst[j];
     }

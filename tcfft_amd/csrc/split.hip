@@ -54,23 +54,30 @@ __device__ __forceinline__ Dft16Split make_dft16_split(int lane, int sign) {
     return s;
 }
 
-// B-form DFT-16 of the four (scaled) points (re[j], im[j]) * s of this lane
-// (column lane%16, rows 4g+j): FP32 results for rows 4g+i in (ore, oim).
+// The FP16 hi/lo operands of this lane's four points (re[j], im[j]) * s:
+// hi = fp16(x*s), lo = fp16(x*s - hi) (the difference is exact in FP32);
+// without SCALE, s = 1.
 template <bool SCALE>
-__device__ __forceinline__ void dft16_split_b(const float* re, const float* im, float s, const Dft16Split& F,
-                                              f32x4& ore, f32x4& oim) {
+__device__ __forceinline__ void split_operand(const float* re, const float* im, float s, f16x8& h, f16x8& l) {
     u32 hi[4], lo[4];
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
-        // hi = fp16(x*s); lo = fp16(x*s - hi) (the difference is exact in
-        // FP32); without SCALE, s = 1
         const float xr = SCALE ? re[j] * s : re[j], xi = SCALE ? im[j] * s : im[j];
         hi[j] = pack(xr, xi);
-        const cf h = unpack(hi[j]);
-        lo[j] = pack(xr - h.x, xi - h.y);
+        const cf v = unpack(hi[j]);
+        lo[j] = pack(xr - v.x, xi - v.y);
     }
-    const f16x8 bh = as_operand(hi[0], hi[1], hi[2], hi[3]);
-    const f16x8 bl = as_operand(lo[0], lo[1], lo[2], lo[3]);
+    h = as_operand(hi[0], hi[1], hi[2], hi[3]);
+    l = as_operand(lo[0], lo[1], lo[2], lo[3]);
+}
+
+// B-form DFT-16 of the four (scaled) points of this lane (column lane%16,
+// rows 4g+j): FP32 results for rows 4g+i in (ore, oim).
+template <bool SCALE>
+__device__ __forceinline__ void dft16_split_b(const float* re, const float* im, float s, const Dft16Split& F,
+                                              f32x4& ore, f32x4& oim) {
+    f16x8 bh, bl;
+    split_operand<SCALE>(re, im, s, bh, bl);
     const f32x4 z = {0.f, 0.f, 0.f, 0.f};
     ore = __builtin_amdgcn_mfma_f32_16x16x32_f16(F.h.re, bh, z, 0, 0, 0);
     ore = __builtin_amdgcn_mfma_f32_16x16x32_f16(F.h.re, bl, ore, 0, 0, 0);
@@ -78,6 +85,21 @@ __device__ __forceinline__ void dft16_split_b(const float* re, const float* im, 
     oim = __builtin_amdgcn_mfma_f32_16x16x32_f16(F.h.im, bh, z, 0, 0, 0);
     oim = __builtin_amdgcn_mfma_f32_16x16x32_f16(F.h.im, bl, oim, 0, 0, 0);
     oim = __builtin_amdgcn_mfma_f32_16x16x32_f16(F.l.im, bh, oim, 0, 0, 0);
+}
+
+// The same in the A-form: the frequency goes to lane%16, the column to rows 4g+i.
+template <bool SCALE>
+__device__ __forceinline__ void dft16_split_a(const float* re, const float* im, float s, const Dft16Split& F,
+                                              f32x4& ore, f32x4& oim) {
+    f16x8 ah, al;
+    split_operand<SCALE>(re, im, s, ah, al);
+    const f32x4 z = {0.f, 0.f, 0.f, 0.f};
+    ore = __builtin_amdgcn_mfma_f32_16x16x32_f16(ah, F.h.re, z, 0, 0, 0);
+    ore = __builtin_amdgcn_mfma_f32_16x16x32_f16(al, F.h.re, ore, 0, 0, 0);
+    ore = __builtin_amdgcn_mfma_f32_16x16x32_f16(ah, F.l.re, ore, 0, 0, 0);
+    oim = __builtin_amdgcn_mfma_f32_16x16x32_f16(ah, F.h.im, z, 0, 0, 0);
+    oim = __builtin_amdgcn_mfma_f32_16x16x32_f16(al, F.h.im, oim, 0, 0, 0);
+    oim = __builtin_amdgcn_mfma_f32_16x16x32_f16(ah, F.l.im, oim, 0, 0, 0);
 }
 
 // 2^(13 - e) for the wave-wide largest magnitude m = f * 2^e (f in [0.5, 1)),
@@ -285,13 +307,13 @@ __global__ __launch_bounds__(256, 2) void k_split_col(const float2* src, float2*
     split_col_body<PASS, SIGN>(src, dst, blockIdx.x, w4096, wn_hi, wn_lo);
 }
 
-// Workgroups of 256 threads of kernel k resident at once on the current device.
+// Workgroups of kernel k resident at once on the current device.
 template <class K>
-static u32 split_resident(K k) {
+static u32 split_resident(K k, int threads = 256) {
     int dev = 0, cus = 0, per_cu = 0;
     if (hipGetDevice(&dev) != hipSuccess ||
         hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess ||
-        hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k, 256, 0) != hipSuccess)
+        hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k, threads, 0) != hipSuccess)
         return 0;  // no schedule rather than a wrong one
     return (u32)(cus * per_cu);
 }
@@ -677,6 +699,270 @@ __global__ __launch_bounds__(256) void k_split_small(const float2* src, float2* 
     for (int k = 0; k < R; ++k) {
         const f32x2 x = {v[k].x, v[k].y};
         __builtin_nontemporal_store(x, reinterpret_cast<f32x2*>(dst + base + ((size_t)k << q_log2)));
+    }
+}
+
+// ---------------------------------------------------------------------------
+// k_split_rows<T>: contiguous lines of L = 256*T points (T = 1..16), the whole
+// line transform in one HBM round trip, natural order in and out, in place or
+// out of place.  Bound by HBM; what it replaces is the two column passes of
+// split_axis over the same lines (16 B per element each).  Measured, those
+// passes -> this kernel: 256 x 32000 55.8 -> 28.4 us, 512 x 16000 53.1 -> 28.0,
+// 1024 x 8000 50.6 -> 30.5, 2048 x 4000 50.2 -> 31.0, 4096 x 4096 96.9 ->
+// 63.7 (4.2 TB/s; a copy of 1 GiB reaches 5.1), 256 x 400 9.9 (two passes)
+// -> 4.5.  What is left is the latency of two waves per SIMD (a wave's 4096
+// points take 128 registers).
+//
+// A wave holds 4096 points (16/T lines, tile t = line*T + d2) in registers,
+// no LDS.  Natural index of a line m = d2 + T*(d1 + 16*d0): lane (c16 = d1, g)
+// word j holds d0 = 4g + j.  T <= 4 loads that directly (a lane's points with
+// the same d0 are T adjacent elements); T = 8 and 16 load four adjacent
+// elements per lane (so that a wave instruction covers whole 128-byte lines)
+// and swap lane bits 4 (and 5) with the register bits of d0.
+//   stage 0: split DFT-16 over d0 (A-form) -> lane%16 = k0, (g,i) = d1, times
+//            W_256^{k0*d1} / 16;
+//   stage 1: split DFT-16 over d1 (A-form) -> lane%16 = k1, (g,i) = k0;
+//   then radix T over the line's tiles in FP32 on VALU (FP32 rather than a
+//   third split stage: no rounding to hi/lo, no register transpose), with
+//   W_{256T}^{(k0+16*k1)*d2} and the inverse scale in one factor: X[k0 +
+//   16*k1 + 256*k2], four adjacent elements per lane.
+// Every line has its own power-of-two scale, so lines of different size do
+// not share one.
+template <int T, int NT>
+__device__ __forceinline__ void split_rows_load(const float2* src, u32 line0, u32 n_lines, int lane,
+                                                float (&dr)[NT][4], float (&di)[NT][4]) {
+    const u32 c16 = (u32)lane & 15u, g = (u32)lane >> 4;
+    // a ragged wave re-reads the last line
+    auto base = [&](int l) { return src + (size_t)min(line0 + (u32)l, n_lines - 1u) * (256u * T); };
+    if constexpr (T == 1) {
+#pragma unroll
+        for (int l = 0; l < NT; ++l) {
+            const float2* b = base(l);
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                const f32x2 v = ld_at_nt<f32x2>(b + 16 * j, 8u * (c16 + 64u * g));
+                dr[l][j] = v[0];
+                di[l][j] = v[1];
+            }
+        }
+    } else if constexpr (T <= 4) {
+#pragma unroll
+        for (int l = 0; l < NT / T; ++l) {
+            const float2* b = base(l);
+#pragma unroll
+            for (int j = 0; j < 4; ++j)
+#pragma unroll
+                for (int h = 0; h < T / 2; ++h) {
+                    const f32x4 v = ld_at_nt<f32x4>(b + 16 * T * j + 2 * h, 8u * T * (c16 + 64u * g));
+                    dr[l * T + 2 * h][j] = v[0];
+                    di[l * T + 2 * h][j] = v[1];
+                    dr[l * T + 2 * h + 1][j] = v[2];
+                    di[l * T + 2 * h + 1][j] = v[3];
+                }
+        }
+    } else {
+        // words i = d2 bits 0-1; lane bit 4 = d2 bit 2; lane bit 5 = d2 bit 3
+        // (T = 16) or d0 bit 3 (T = 8); x = the other bits of d0
+        constexpr int X = T == 8 ? 8 : 16;
+#pragma unroll
+        for (int l = 0; l < NT / T; ++l) {
+            const float2* b = base(l);
+            const u32 off = 8u * (T == 8 ? 4u * (g & 1u) + 8u * (c16 + 128u * (g >> 1)) : 4u * g + 16u * c16);
+            u32 wr[X][4], wi[X][4];
+#pragma unroll
+            for (int x = 0; x < X; ++x)
+#pragma unroll
+                for (int h = 0; h < 2; ++h) {
+                    const f32x4 v = ld_at_nt<f32x4>(b + 16 * T * x + 2 * h, off);
+                    wr[x][2 * h] = __float_as_uint(v[0]);
+                    wi[x][2 * h] = __float_as_uint(v[1]);
+                    wr[x][2 * h + 1] = __float_as_uint(v[2]);
+                    wi[x][2 * h + 1] = __float_as_uint(v[3]);
+                }
+#pragma unroll
+            for (int x = 0; x < X; ++x)
+                if (!(x & 4))
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) {
+                        swap_l4(wr[x][i], wr[x | 4][i]);
+                        swap_l4(wi[x][i], wi[x | 4][i]);
+                    }
+            if constexpr (T == 16) {
+#pragma unroll
+                for (int x = 0; x < X; ++x)
+                    if (!(x & 8))
+#pragma unroll
+                        for (int i = 0; i < 4; ++i) {
+                            swap_l5(wr[x][i], wr[x | 8][i]);
+                            swap_l5(wi[x][i], wi[x | 8][i]);
+                        }
+            }
+#pragma unroll
+            for (int x = 0; x < X; ++x)
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    dr[l * T + i + 4 * (x >> 2)][x & 3] = __uint_as_float(wr[x][i]);
+                    di[l * T + i + 4 * (x >> 2)][x & 3] = __uint_as_float(wi[x][i]);
+                }
+        }
+    }
+}
+
+// cos and sin of the small angle 2*pi*k/n (at most 0.07) by their Taylor
+// series in FP64, for compile-time constants.
+__host__ __device__ constexpr float small_cos(int k, int n) {
+    const double a = 6.283185307179586477 * k / n, q = a * a;
+    return (float)(1 - q / 2 * (1 - q / 12 * (1 - q / 30 * (1 - q / 56))));
+}
+__host__ __device__ constexpr float small_sin(int k, int n) {
+    const double a = 6.283185307179586477 * k / n, q = a * a;
+    return (float)(a * (1 - q / 6 * (1 - q / 20 * (1 - q / 42 * (1 - q / 72)))));
+}
+
+template <int T, int SIGN, int NT>
+__global__ __launch_bounds__(256, 2) void k_split_rows(const float2* src, float2* dst, u32 n_lines,
+                                                     const float2* __restrict__ w4096, StartSched sched) {
+    constexpr int LPW = NT / T;
+    constexpr float sg = SIGN < 0 ? 1.f : -1.f;
+    const int lane = lane_id(), c16 = lane & 15, g = lane >> 4;
+    const u32 wave = blockIdx.x * (blockDim.x >> 6) + (u32)__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+    const u32 line0 = wave * LPW;
+    if (line0 >= n_lines) return;
+    split_start_delay(sched);
+    // table values before the data (global loads complete in issue order)
+    // W_{256T}^{e*(16*c16 + 4*g)}, e = 1, 2, 3, 4, 8, 12
+    constexpr int NE = T == 1 ? 0 : T == 2 ? 1 : T == 4 ? 3 : T == 8 ? 4 : 6;
+    float2 t_w1[4], t_e[NE + 1];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) t_w1[i] = w4096[((c16 * (4 * g + i)) & 255) * 16];
+    auto load_e = [&] {
+#pragma unroll
+        for (int k = 0; k < NE; ++k) t_e[k] = w4096[(k < 4 ? k + 1 : 4 * k - 8) * (16 * c16 + 4 * g) * (16 / T)];
+    };
+    if constexpr (T < 16) load_e();
+    __builtin_amdgcn_sched_barrier(0);
+    float dr[NT][4], di[NT][4];
+    split_rows_load<T, NT>(src, line0, n_lines, lane, dr, di);
+    __builtin_amdgcn_sched_barrier(0);
+    cf w1[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) w1[i] = cf{0.0625f * t_w1[i].x, 0.0625f * sg * t_w1[i].y};
+    const Dft16Split F = make_dft16_split(lane, SIGN);
+#pragma unroll
+    for (int l = 0; l < LPW; ++l) {
+        float m = 0.f;
+#pragma unroll
+        for (int t = l * T; t < l * T + T; ++t)
+#pragma unroll
+            for (int j = 0; j < 4; ++j) m = fmaxf(m, fmaxf(fabsf(dr[t][j]), fabsf(di[t][j])));
+        float s, inv;
+        wave_scale(m, s, inv);
+        s = __int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(s)));
+        inv = 16.f * __int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(inv)));
+#pragma unroll
+        for (int t = l * T; t < l * T + T; ++t) {
+            f32x4 ore, oim;
+            dft16_split_a<true>(dr[t], di[t], s, F, ore, oim);
+            float sr[4], si[4];
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const cf v = cmul(cf{ore[i], oim[i]}, w1[i]);
+                sr[i] = v.x;
+                si[i] = v.y;
+            }
+            dft16_split_a<false>(sr, si, 1.f, F, ore, oim);
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                dr[t][i] = ore[i];
+                di[t][i] = oim[i];
+            }
+        }
+        // W_{256T}^{c*d2}, c = (16*c16 + 4*g) + i: e[d2] of the lane, at most
+        // two table values (powers of one rounded root would carry its error
+        // d2-fold), times a constant
+        if constexpr (T == 16) load_e();  // during the stages they would spill
+        cf e[T];
+#pragma unroll
+        for (int d = 1; d < T; ++d) {
+            if (d < 4) e[d] = cf{inv * t_e[d - 1].x, inv * sg * t_e[d - 1].y};
+            else if (d % 4 == 0) e[d] = cf{inv * t_e[d / 4 + 2].x, inv * sg * t_e[d / 4 + 2].y};
+            else e[d] = cmul(e[d & ~3], cf{t_e[d % 4 - 1].x, sg * t_e[d % 4 - 1].y});
+        }
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            cf v[T];
+            v[0] = cf{dr[l * T][i] * inv, di[l * T][i] * inv};
+            if constexpr (T > 1) {
+#pragma unroll
+                for (int d = 1; d < T; ++d) {
+                    const cf p = i ? cmul(e[d], cf{small_cos(d * i, 256 * T), -sg * small_sin(d * i, 256 * T)}) : e[d];
+                    v[d] = cmul(cf{dr[l * T + d][i], di[l * T + d][i]}, p);
+                }
+                small_dft<T>(v, SIGN);
+            }
+#pragma unroll
+            for (int d = 0; d < T; ++d) {
+                dr[l * T + d][i] = v[d].x;
+                di[l * T + d][i] = v[d].y;
+            }
+        }
+        if (line0 + l < n_lines) {  // wave-uniform
+            float2* o = dst + (size_t)(line0 + l) * (256u * T);
+            const u32 off = 8u * (16u * c16 + 4u * g);
+#pragma unroll
+            for (int d = 0; d < T; ++d) {
+                const int t = l * T + d;
+                const f32x4 o0 = {dr[t][0], di[t][0], dr[t][1], di[t][1]}, o1 = {dr[t][2], di[t][2], dr[t][3], di[t][3]};
+                st_at<f32x4>(o + 256 * d, off, o0);
+                st_at<f32x4>(o + 256 * d + 2, off, o1);
+            }
+        }
+    }
+}
+
+template <int T, int SIGN, int NT>
+static hipError_t launch_split_rows_nt(const float2* src, float2* dst, u32 n_lines, const float2* w4096,
+                                       StartSched sched, hipStream_t st) {
+    static const u32 res = split_resident(k_split_rows<T, SIGN, NT>, 64);
+    const u32 waves = (n_lines * T + NT - 1u) / NT;
+    if (sched.groups == 0 || waves <= res) sched.delay = 0;
+    const u32 wg = waves > res ? 4u : 1u;
+    sched.resident = res / wg;
+    hipLaunchKernelGGL((k_split_rows<T, SIGN, NT>), dim3((waves + wg - 1) / wg), dim3(64 * wg), 0, st, src, dst, n_lines, w4096, sched);
+    return hipGetLastError();
+}
+
+// Tiles per wave: 16, or the fewest that hold a line (4 at least) when 16
+// would leave fewer than two waves per SIMD: such a call takes one wave's
+// time (256 x 400: 9.9 -> 4.5 us, 1024 x 700: 8.5 -> 5.5), while a full chip
+// wants the bytes in flight (1024 x 32000: 110.8 us against 120.3 with 4).
+// Four waves per workgroup, and the start delay, when the grid is more than
+// one round of waves (1024 x 8000: 32.6 -> 30.5 us); else one, so that a
+// small grid spreads over the chip (4096 x 300: 16.4 -> 12.5 us).
+template <int T, int SIGN>
+static hipError_t launch_split_rows_t(const float2* src, float2* dst, u32 n_lines, const float2* w4096,
+                                      StartSched sched, u32 cus, hipStream_t st) {
+    if constexpr (T < 16) {
+        if ((n_lines * T + 15u) / 16u < 8u * cus)
+            return launch_split_rows_nt<T, SIGN, (T < 4 ? 4 : T)>(src, dst, n_lines, w4096, sched, st);
+    }
+    return launch_split_rows_nt<T, SIGN, 16>(src, dst, n_lines, w4096, sched, st);
+}
+
+hipError_t launch_split_rows(int T, const float2* src, float2* dst, u32 n_lines, int sign, const float2* w4096,
+                             StartSched sched, uint32_t cus, hipStream_t st) {
+    switch (T * 2 + (sign < 0 ? 0 : 1)) {
+    case 2: return launch_split_rows_t<1, -1>(src, dst, n_lines, w4096, sched, cus, st);
+    case 3: return launch_split_rows_t<1, +1>(src, dst, n_lines, w4096, sched, cus, st);
+    case 4: return launch_split_rows_t<2, -1>(src, dst, n_lines, w4096, sched, cus, st);
+    case 5: return launch_split_rows_t<2, +1>(src, dst, n_lines, w4096, sched, cus, st);
+    case 8: return launch_split_rows_t<4, -1>(src, dst, n_lines, w4096, sched, cus, st);
+    case 9: return launch_split_rows_t<4, +1>(src, dst, n_lines, w4096, sched, cus, st);
+    case 16: return launch_split_rows_t<8, -1>(src, dst, n_lines, w4096, sched, cus, st);
+    case 17: return launch_split_rows_t<8, +1>(src, dst, n_lines, w4096, sched, cus, st);
+    case 32: return launch_split_rows_t<16, -1>(src, dst, n_lines, w4096, sched, cus, st);
+    case 33: return launch_split_rows_t<16, +1>(src, dst, n_lines, w4096, sched, cus, st);
+    default: return hipErrorInvalidValue;
     }
 }
 
