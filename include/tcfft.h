@@ -142,8 +142,9 @@ int tcfft_exec_split(tcfft_plan plan, const void *in, void *out, int direction, 
 
 /* Prepares a complex plan for tcfft_exec_split at its size: builds the
  * pass list (1D n = 65536 as two 256 x 256 passes; other shapes as passes
- * of 16..256 rows, 2..4 per axis, of which the passes over contiguous lines
- * of at most 4096 points run as one kernel), uploads their twiddle tables and
+ * of 16..256 rows, 2..4 per axis; contiguous lines of at most 4096 points and
+ * strided axes of 512..2048 run as one pass each, 1D lines of 2^17..2^22
+ * points as two), uploads their twiddle tables and
  * allocates a workspace of 8 bytes per element where a pass needs one, so that
  * tcfft_exec_split allocates nothing (graph-capturable) and runs in place.
  * One workspace per

@@ -393,25 +393,52 @@ int split_steps_of(int dims, int n_or_nx, int ny, int batch, std::vector<tcfft_p
     return rc ? rc : split_axis(ilog2((uint32_t)n_or_nx), ilog2((uint32_t)ny), (uint32_t)batch, steps);
 }
 
-// The passes tcfft_exec_split runs for that list: the passes of a contiguous
-// axis of 256..4096 points are one kernel over whole lines (k_split_rows, one
-// HBM round trip instead of one per pass), the others as listed.
+// The passes tcfft_exec_split runs for that list.  Fewer round trips where a
+// kernel holds more than a pass of the list:
+//   a contiguous axis of 256..4096 points: whole lines (k_split_rows);
+//   1D 2^17..2^22 points: two passes of radix 256..2048 instead of three;
+//   a strided axis of 512..2048 points: one pass (k_split_colsw).
 int split_exec_steps_of(int dims, int n_or_nx, int ny, int batch, std::vector<tcfft_plan_s::SplitStep>& steps) {
     std::vector<tcfft_plan_s::SplitStep> list;
     const int rc = split_steps_of(dims, n_or_nx, ny, batch, list);
     if (rc) return rc;
     const int line = dims == 1 ? n_or_nx : ny;
+    const uint32_t lines = (uint32_t)batch * (dims == 1 ? 1u : (uint32_t)n_or_nx);
     size_t i = 0;
+    while (i < list.size() && list[i].transposing) ++i;  // an axis's passes end with the first one without a twiddle
+    ++i;
+    tcfft_plan_s::SplitStep s{};
     if (line <= 4096) {
-        while (list[i].transposing) ++i;  // the contiguous axis's passes end with the first one without a twiddle
-        ++i;
-        tcfft_plan_s::SplitStep s{};
         s.R = line;
         s.row_tiles = line / 256;
-        s.a.units = (uint32_t)batch * (dims == 1 ? 1u : (uint32_t)n_or_nx);
+        s.a.units = lines;
         steps.push_back(s);
+    } else if (dims == 1 && line >= (1 << 17) && line <= (1 << 22)) {
+        const int m = ilog2((uint32_t)line), b = m == 17 ? 9 : m / 2;  // R = 2^b rows, then 2^(m-b)
+        s.R = 1 << b;
+        s.row = s.transposing = true;
+        s.a.q_log2 = (uint32_t)(m - b);
+        s.a.units = lines << (s.a.q_log2 - 4);
+        s.a.m_mask = (uint32_t)line - 1u;
+        s.a.lo_bits = (uint32_t)m / 2u;  // the split of table_pair
+        steps.push_back(s);
+        s = {};
+        s.R = 1 << (m - b);
+        s.a.q_log2 = s.a.qlo_log2 = (uint32_t)b;
+        s.a.units = lines << (b - 4);
+        steps.push_back(s);
+    } else {
+        steps.insert(steps.end(), list.begin(), list.begin() + (long)std::min(i, list.size()));
     }
-    steps.insert(steps.end(), list.begin() + (long)i, list.end());
+    if (dims == 2 && n_or_nx >= 512 && n_or_nx <= 2048) {
+        s = {};
+        s.R = n_or_nx;
+        s.a.q_log2 = s.a.qlo_log2 = (uint32_t)ilog2((uint32_t)ny);
+        s.a.units = (uint32_t)batch << (s.a.q_log2 - 4);
+        steps.push_back(s);
+    } else if (dims == 2) {
+        steps.insert(steps.end(), list.begin() + (long)i, list.end());
+    }
     return TCFFT_SUCCESS;
 }
 

@@ -54,6 +54,45 @@ __device__ __forceinline__ Dft16Split make_dft16_split(int lane, int sign) {
     return s;
 }
 
+// The same with output row f multiplied by scale (this lane's, f = lane%16;
+// the B-form, where the constant's row is the output frequency): the FP32
+// product is split, so the factor costs nothing per point.
+__device__ __forceinline__ Dft16Split make_dft16_split_scaled(int lane, int sign, cf scale) {
+    const int f = lane & 15, g = lane >> 4;
+    Dft16Split s;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+        const int m = ((4 * g + j) * f) & 15;
+        const cf v = cmul(scale, cf{cos16_exact(m), sign < 0 ? -sin16_exact(m) : sin16_exact(m)});
+        const _Float16 frh = (_Float16)v.x, fih = (_Float16)v.y;
+        const _Float16 frl = (_Float16)(v.x - (float)frh), fil = (_Float16)(v.y - (float)fih);
+        s.h.re[2 * j] = frh;
+        s.h.re[2 * j + 1] = -fih;
+        s.h.im[2 * j] = fih;
+        s.h.im[2 * j + 1] = frh;
+        s.l.re[2 * j] = frl;
+        s.l.re[2 * j + 1] = -fil;
+        s.l.im[2 * j] = fil;
+        s.l.im[2 * j + 1] = frl;
+    }
+    return s;
+}
+
+// cos and sin of the angle 2*pi*k/n (at most 1.2) by their Taylor series in
+// FP64, for compile-time twiddle constants.
+__host__ __device__ constexpr float cos_of(int k, int n) {
+    const double a = 6.283185307179586477 * k / n, q = a * a;
+    double v = 1;
+    for (int j = 20; j > 0; j -= 2) v = 1 - v * q / (j * (j - 1));
+    return (float)v;
+}
+__host__ __device__ constexpr float sin_of(int k, int n) {
+    const double a = 6.283185307179586477 * k / n, q = a * a;
+    double v = 1;
+    for (int j = 21; j > 1; j -= 2) v = 1 - v * q / (j * (j - 1));
+    return (float)(a * v);
+}
+
 // The FP16 hi/lo operands of this lane's four points (re[j], im[j]) * s:
 // hi = fp16(x*s), lo = fp16(x*s - hi) (the difference is exact in FP32);
 // without SCALE, s = 1.
@@ -309,11 +348,11 @@ __global__ __launch_bounds__(256, 2) void k_split_col(const float2* src, float2*
 
 // Workgroups of kernel k resident at once on the current device.
 template <class K>
-static u32 split_resident(K k, int threads = 256) {
+static u32 split_resident(K k, int threads = 256, size_t lds = 0) {
     int dev = 0, cus = 0, per_cu = 0;
     if (hipGetDevice(&dev) != hipSuccess ||
         hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess ||
-        hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k, threads, 0) != hipSuccess)
+        hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k, threads, lds) != hipSuccess)
         return 0;  // no schedule rather than a wrong one
     return (u32)(cus * per_cu);
 }
@@ -373,6 +412,26 @@ __device__ __forceinline__ cf split_tw(const SplitPassArgs& a, u32 e, float sg) 
     e &= a.m_mask;
     const float2 h = a.hi[e >> a.lo_bits], l = a.lo[e & ((1u << a.lo_bits) - 1u)];
     return cmul(cf{h.x, sg * h.y}, cf{l.x, sg * l.y});
+}
+
+// W_256^{t*(4g + i)} * scale for tile t, word i of a wave's 256-point column
+// DFT: a lane value of at most two table entries times a constant (a
+// recurrence over the tiles would carry its root's rounding 15-fold).
+struct Tw256 {
+    float2 e[6];  // W_256^{k*4g}, k = 1, 2, 3, 4, 8, 12
+};
+__device__ __forceinline__ void tw256_load(Tw256& tw, int g, const float2* __restrict__ w4096) {
+#pragma unroll
+    for (int k = 0; k < 6; ++k) tw.e[k] = w4096[(k < 4 ? k + 1 : 4 * k - 8) * (64 * g)];
+}
+__device__ __forceinline__ cf tw256_tile(const Tw256& tw, int t, float sg, float scale) {
+    auto at = [&](int k, float f) { return cf{f * tw.e[k].x, f * sg * tw.e[k].y}; };
+    if (t == 0) return cf{scale, 0.f};
+    if (t < 4) return at(t - 1, scale);
+    return t % 4 ? cmul(at(t / 4 + 2, scale), at(t % 4 - 1, 1.f)) : at(t / 4 + 2, scale);
+}
+__device__ __forceinline__ cf tw256_word(cf tile, int t, int i, float sg) {
+    return t * i ? cmul(tile, cf{cos_of(t * i, 256), -sg * sin_of(t * i, 256)}) : tile;
 }
 
 __device__ __forceinline__ float uniform_f(float v) {
@@ -532,9 +591,8 @@ __device__ __forceinline__ void split_pass_256(const float2* src, float2* dst, c
     const u32 q = ((u & ((1u << upq) - 1u)) << 4) + c16;
     const size_t sbase = (size_t)(u >> upq) << (a.q_log2 + 8);
 
-    float2 t_step[4];
-#pragma unroll
-    for (int i = 0; i < 4; ++i) t_step[i] = w4096[16 * (4 * g + i)];
+    Tw256 tw256;
+    tw256_load(tw256, g, w4096);
     __builtin_amdgcn_sched_barrier(0);
     // rows r = r0 + 16 (4g + j): tile r0, word j
     float dr[16][4], di[16][4];
@@ -564,20 +622,14 @@ __device__ __forceinline__ void split_pass_256(const float2* src, float2* dst, c
     inv = uniform_f(inv);
     {
         const Dft16Split F = make_dft16_split(lane, SIGN);
-        cf step[4], rec[4];
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            step[i] = cf{t_step[i].x, sg * t_step[i].y};
-            rec[i] = cf{0.0625f, 0.f};
-        }
 #pragma unroll
         for (int t = 0; t < 16; ++t) {
             f32x4 ore, oim;
             dft16_split_b<true>(dr[t], di[t], s, F, ore, oim);
+            const cf e = tw256_tile(tw256, t, sg, 0.0625f);
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
-                const cf v = cmul(cf{ore[i], oim[i]}, rec[i]);
-                if (t < 15) rec[i] = cmul(rec[i], step[i]);
+                const cf v = cmul(cf{ore[i], oim[i]}, tw256_word(e, t, i, sg));
                 dr[t][i] = v.x;
                 di[t][i] = v.y;
             }
@@ -808,17 +860,6 @@ __device__ __forceinline__ void split_rows_load(const float2* src, u32 line0, u3
     }
 }
 
-// cos and sin of the small angle 2*pi*k/n (at most 0.07) by their Taylor
-// series in FP64, for compile-time constants.
-__host__ __device__ constexpr float small_cos(int k, int n) {
-    const double a = 6.283185307179586477 * k / n, q = a * a;
-    return (float)(1 - q / 2 * (1 - q / 12 * (1 - q / 30 * (1 - q / 56))));
-}
-__host__ __device__ constexpr float small_sin(int k, int n) {
-    const double a = 6.283185307179586477 * k / n, q = a * a;
-    return (float)(a * (1 - q / 6 * (1 - q / 20 * (1 - q / 42 * (1 - q / 72)))));
-}
-
 template <int T, int SIGN, int NT>
 __global__ __launch_bounds__(256, 2) void k_split_rows(const float2* src, float2* dst, u32 n_lines,
                                                      const float2* __restrict__ w4096, StartSched sched) {
@@ -895,7 +936,7 @@ __global__ __launch_bounds__(256, 2) void k_split_rows(const float2* src, float2
             if constexpr (T > 1) {
 #pragma unroll
                 for (int d = 1; d < T; ++d) {
-                    const cf p = i ? cmul(e[d], cf{small_cos(d * i, 256 * T), -sg * small_sin(d * i, 256 * T)}) : e[d];
+                    const cf p = i ? cmul(e[d], cf{cos_of(d * i, 256 * T), -sg * sin_of(d * i, 256 * T)}) : e[d];
                     v[d] = cmul(cf{dr[l * T + d][i], di[l * T + d][i]}, p);
                 }
                 small_dft<T>(v, SIGN);
@@ -966,6 +1007,226 @@ hipError_t launch_split_rows(int T, const float2* src, float2* dst, u32 n_lines,
     }
 }
 
+// ---------------------------------------------------------------------------
+// k_split_colsw<W>: a column pass (as k_split_pass) of radix R = 256*W, W = 2,
+// 4, 8, in one HBM round trip: the two passes of such an axis in one.  Bound
+// by HBM.  Measured per exec, radices <= 256 -> this kernel (and k_split_rows
+// for 2D rows): 2D 512 x 512 x 32 107.7 -> 55.3 us, 1024 x 1024 x 8 100.5 ->
+// 57.8, 2048 x 1024 x 4 99.8 -> 59.2; 1D, three passes -> two: 2^17 x 64 75.5
+// -> 57.3, 2^20 x 16 151 -> 113, 2^22 x 4 161 -> 117.
+//
+// A workgroup of W waves owns 16 adjacent columns of one signal.  Wave w
+// takes the rows r = w + W*(r0 + 16*r1) (tile r0, r1 = 4g + j) and runs
+// their 256-point DFT in registers; output m = k0 + 16*k1 also gets the
+// radix-W stage's twiddle W_R^{w*m}, which rides on the rows of the two
+// stages' operands (W_R^{w*k0} and W_R^{16*w*k1}).  Each wave has its own
+// scale, undone before the exchange: the radix-W stage over the waves runs in
+// FP32 on the exchanged values, output k = m + 256*k2.
+// The FP32 data takes W*32 KiB, so it is exchanged in two rounds (W = 4: two
+// workgroups per CU):
+//   column store (no twiddle): round = half of the tiles k0, LDS [source]
+//     [tile][lane][4] for the real and the imaginary parts, b128 both ways;
+//   row store (twiddle W_M^{q k}, transposed): round = half of the columns,
+//     LDS [source][column][m], so that a lane then holds two adjacent k and
+//     a wave stores 1 KiB runs.  Element of (column c, m): 258 c + (m ^
+//     16*((m >> 6) & 1)): the 16 writing lanes of a half wave (8 columns, two
+//     g) fall on different banks, the b128 reads are contiguous.
+template <int W, bool ROW, int SIGN>
+__global__ __launch_bounds__(64 * W) TCFFT_MFMA_BUDGET void k_split_colsw(const float2* src, float2* dst,
+                                                                        SplitPassArgs a,
+                                                                        const float2* __restrict__ w4096,
+                                                                        StartSched sched) {
+    constexpr float sg = SIGN < 0 ? 1.f : -1.f;
+    constexpr int LR = W == 2 ? 9 : W == 4 ? 10 : 11;  // log2 R
+    extern __shared__ __attribute__((aligned(16))) float xch[];
+    split_start_delay(sched);
+    const int lane = lane_id(), c16 = lane & 15, g = lane >> 4;
+    const u32 w = (u32)__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+    const u32 u = blockIdx.x;
+    const u32 upq = a.q_log2 - 4u;
+    const u32 q0 = (u & ((1u << upq) - 1u)) << 4;  // first column
+    const size_t sbase = (size_t)(u >> upq) << (a.q_log2 + LR);
+    // table values before the data (global loads complete in issue order)
+    Tw256 tw;
+    tw256_load(tw, g, w4096);
+    const float2 t_v1 = w4096[((u32)c16 * w * (16u / W)) & 4095u];   // W_R^{w*f}
+    const float2 t_v2 = w4096[((u32)c16 * w * (256u / W)) & 4095u];  // W_R^{16*w*f}
+    __builtin_amdgcn_sched_barrier(0);
+    float dr[16][4], di[16][4];
+    {
+        // wave-uniform row bases and a 32-bit lane offset (at most 2^30 bytes)
+        const float2* ub = src + sbase + q0 + ((size_t)w << a.q_log2);
+        const u32 off = ((u32)c16 + ((64u * W * (u32)g) << a.q_log2)) * 8u;
+#pragma unroll
+        for (int r0 = 0; r0 < 16; ++r0)
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                const f32x2 v = ld_at_nt<f32x2>(ub + ((size_t)(W * (r0 + 16 * j)) << a.q_log2), off);
+                dr[r0][j] = v[0];
+                di[r0][j] = v[1];
+            }
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    float m = 0.f;
+#pragma unroll
+    for (int t = 0; t < 16; ++t)
+#pragma unroll
+        for (int j = 0; j < 4; ++j) m = fmaxf(m, fmaxf(fabsf(dr[t][j]), fabsf(di[t][j])));
+    float s, inv;
+    wave_scale(m, s, inv);
+    s = uniform_f(s);
+    inv = 16.f * uniform_f(inv);  // undoes the scale and the 1/16 of stage 1
+    {
+        const Dft16Split F = make_dft16_split_scaled(lane, SIGN, cf{t_v1.x, sg * t_v1.y});
+#pragma unroll
+        for (int t = 0; t < 16; ++t) {
+            f32x4 ore, oim;
+            dft16_split_b<true>(dr[t], di[t], s, F, ore, oim);
+            const cf e = tw256_tile(tw, t, sg, 0.0625f);
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const cf p = tw256_word(e, t, i, sg);
+                const cf v = cmul(cf{ore[i], oim[i]}, p);
+                dr[t][i] = v.x;
+                di[t][i] = v.y;
+            }
+        }
+    }
+    {
+        float tr[16][4], ti[16][4];
+        transpose_gi_tile(dr, tr);
+        transpose_gi_tile(di, ti);
+        const Dft16Split F2 = make_dft16_split_scaled(lane_id(), SIGN, cf{t_v2.x, sg * t_v2.y});
+#pragma unroll
+        for (int t = 0; t < 16; ++t) {
+            f32x4 ore, oim;
+            dft16_split_b<false>(tr[t], ti[t], 1.f, F2, ore, oim);
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                dr[t][i] = ore[i] * inv;
+                di[t][i] = oim[i] * inv;
+            }
+        }
+    }
+    // tile t = k0, (g,i) = k1, column c16
+    if constexpr (!ROW) {
+        constexpr u32 TPW = 8 / W;
+        f32x4* const xr = reinterpret_cast<f32x4*>(xch);
+        f32x4* const xi = xr + W * 8 * 64;
+        const u32 off = ((u32)c16 + ((64u * (u32)g) << a.qlo_log2)) * 8u;
+        float2* const ob = dst + sbase + q0;
+#pragma unroll
+        for (int r = 0; r < 2; ++r) {
+            if (r) __syncthreads();  // round 0's reads are done
+#pragma unroll
+            for (int tt = 0; tt < 8; ++tt) {
+                const int t = 8 * r + tt;
+                xr[(w * 8 + tt) * 64 + lane] = f32x4{dr[t][0], dr[t][1], dr[t][2], dr[t][3]};
+                xi[(w * 8 + tt) * 64 + lane] = f32x4{di[t][0], di[t][1], di[t][2], di[t][3]};
+            }
+            __syncthreads();
+#pragma unroll
+            for (u32 ti = 0; ti < TPW; ++ti) {
+                const u32 tt = w * TPW + ti;
+                f32x4 vr[W], vi[W];
+#pragma unroll
+                for (int k = 0; k < W; ++k) {
+                    vr[k] = xr[(k * 8 + tt) * 64 + lane];
+                    vi[k] = xi[(k * 8 + tt) * 64 + lane];
+                }
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    cf v[W];
+#pragma unroll
+                    for (int k = 0; k < W; ++k) v[k] = cf{vr[k][i], vi[k][i]};
+                    small_dft<W>(v, SIGN);
+                    // row k0 + 16 (4g + i) + 256 k2 (the 64 g part is the lane's)
+#pragma unroll
+                    for (int k2 = 0; k2 < W; ++k2)
+                        st_at_nt<f32x2>(ob + ((size_t)(8u * r + tt + 16u * i + 256u * k2) << a.qlo_log2), off,
+                                        f32x2{v[k2].x, v[k2].y});
+                }
+            }
+        }
+    } else {
+        constexpr u32 CPW = 8 / W;
+        float2* const xc = reinterpret_cast<float2*>(xch);
+#pragma unroll
+        for (int r = 0; r < 2; ++r) {
+            if (r) __syncthreads();  // round 0's reads are done
+            if ((c16 >> 3) == r) {
+                float2* const xw = xc + (w * 8 + (c16 & 7)) * 258;
+#pragma unroll
+                for (int t = 0; t < 16; ++t)
+#pragma unroll
+                    for (int i = 0; i < 4; ++i)
+                        xw[(t + 16 * i + 64 * g) ^ (16 * (g & 1))] = make_float2(dr[t][i], di[t][i]);
+            }
+            // twiddles W_M^{q m} of m = 2 lane + 128 h (m + 1 and k2 below)
+            cf ta[CPW][2];
+#pragma unroll
+            for (u32 ci = 0; ci < CPW; ++ci)
+#pragma unroll
+                for (u32 h = 0; h < 2; ++h)
+                    ta[ci][h] = split_tw(a, (q0 + 8u * r + w * CPW + ci) * (2u * (u32)lane + 128u * h), sg);
+            __syncthreads();
+#pragma unroll
+            for (u32 ci = 0; ci < CPW; ++ci) {
+                const u32 cc = w * CPW + ci, q = q0 + 8u * r + cc;
+                float2* const ob = dst + sbase + ((size_t)q << LR);
+#pragma unroll
+                for (int h = 0; h < 2; ++h) {
+                    const u32 mm = 2u * (u32)lane + 128u * h;
+                    f32x4 x[W];
+#pragma unroll
+                    for (int k = 0; k < W; ++k)
+                        x[k] = *reinterpret_cast<const f32x4*>(xc + (k * 8 + cc) * 258 + (mm ^ (16u * ((mm >> 6) & 1u))));
+                    cf v0[W], v1[W];
+#pragma unroll
+                    for (int k = 0; k < W; ++k) {
+                        v0[k] = cf{x[k][0], x[k][1]};
+                        v1[k] = cf{x[k][2], x[k][3]};
+                    }
+                    small_dft<W>(v0, SIGN);
+                    small_dft<W>(v1, SIGN);
+                    const cf b0 = ta[ci][h], b1 = split_tw(a, q * (2u * (u32)lane + 128u * h + 1u), sg);
+#pragma unroll
+                    for (int k2 = 0; k2 < W; ++k2) {
+                        const cf uk = split_tw(a, 256u * k2 * q, sg);
+                        const cf o0 = cmul(v0[k2], k2 ? cmul(b0, uk) : b0), o1 = cmul(v1[k2], k2 ? cmul(b1, uk) : b1);
+                        st_at<f32x4>(ob + 128 * h + 256 * k2, 16u * (u32)lane, f32x4{o0.x, o0.y, o1.x, o1.y});
+                    }
+                }
+            }
+        }
+    }
+}
+
+template <int W, bool ROW, int SIGN>
+static hipError_t launch_colsw_t(const float2* src, float2* dst, const SplitPassArgs& a, const float2* w4096,
+                                 StartSched sched, hipStream_t st) {
+    constexpr size_t lds = (ROW ? W * 8 * 258 : W * 8 * 256) * sizeof(float2);
+    auto k = k_split_colsw<W, ROW, SIGN>;
+    static const hipError_t attr =
+        hipFuncSetAttribute((const void*)k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+    if (attr != hipSuccess) return attr;
+    static const u32 res = split_resident(k, 64 * W, lds);
+    // a grid that does not fill the chip has nothing to stagger (2^20 x 1:
+    // 34.1 us with the delay, 30.4 without)
+    if (sched.groups == 0 || a.units < res) sched.delay = 0;
+    sched.resident = res;
+    hipLaunchKernelGGL(k, dim3(a.units), dim3(64 * W), lds, st, src, dst, a, w4096, sched);
+    return hipGetLastError();
+}
+
+template <int W, int SIGN>
+static hipError_t launch_colsw(bool row, const float2* src, float2* dst, const SplitPassArgs& a, const float2* w4096,
+                               StartSched sched, hipStream_t st) {
+    if (!row && a.m_mask) return hipErrorInvalidValue;  // the column store has no twiddle
+    return row ? launch_colsw_t<W, true, SIGN>(src, dst, a, w4096, sched, st)
+               : launch_colsw_t<W, false, SIGN>(src, dst, a, w4096, sched, st);
+}
+
 template <int R, bool ROW, int SIGN>
 static hipError_t launch_pass_t(const float2* src, float2* dst, const SplitPassArgs& a, const float2* w4096,
                                 StartSched sched, hipStream_t st) {
@@ -1008,6 +1269,9 @@ static hipError_t launch_pass_s(int R, bool row, const float2* src, float2* dst,
     case 256:
         return row ? launch_pass_t<256, true, SIGN>(src, dst, a, w4096, sched, st)
                    : launch_pass_t<256, false, SIGN>(src, dst, a, w4096, sched, st);
+    case 512: return launch_colsw<2, SIGN>(row, src, dst, a, w4096, sched, st);
+    case 1024: return launch_colsw<4, SIGN>(row, src, dst, a, w4096, sched, st);
+    case 2048: return launch_colsw<8, SIGN>(row, src, dst, a, w4096, sched, st);
     default: return hipErrorInvalidValue;
     }
 }
