@@ -135,6 +135,68 @@ __device__ __forceinline__ void dit4096(u32 (&d)[16][4], int sign, const Dit4096
 }
 
 // ----------------------------------------------------------------------------
+// Natural-order input of the row passes, straight into the digit-reversed
+// register layout (tile t = line*T + d2, lane (c16 = d1, g), word j: d0 = 4g
+// + j) without LDS.  Natural index of a line: m = d2 + T*(d1 + 16*d0), so a
+// lane's points with the same d0 are T adjacent words.  T = 2 and 4 load them
+// as they stand; T = 8 and 16 load four adjacent words per lane, so that a
+// wave instruction covers whole 128-byte lines, and swap lane bit 4 (and 5),
+// which then holds d2 bit 2 (and 3), with the register bits of d0.  Measured
+// against 16-byte writes and 4-byte reads of 16 KiB of LDS per wave: 1024 x
+// 32768 56.1 -> 50.1 us, 2048 x 2000 11.3 -> 9.1, 4096 x 4096 27.2 -> 22.7.
+// line_ptr(l): the wave's l-th line (absent lines: any readable line).
+template <int T, int NT, class LinePtr>
+__device__ __forceinline__ void nat_direct_load(u32 (&d)[NT][4], LinePtr line_ptr, int lane) {
+    static_assert(T >= 2 && NT % T == 0, "whole lines of at least 512 points");
+    const u32 c16 = (u32)lane & 15u, g = (u32)lane >> 4;
+#pragma unroll
+    for (int l = 0; l < NT / T; ++l) {
+        const u32* const b = line_ptr(l);
+        if constexpr (T == 2) {
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                const u32x2 v = ld_at_nt<u32x2>(b + 32 * j, 4u * (2u * c16 + 128u * g));
+                d[2 * l][j] = v[0];
+                d[2 * l + 1][j] = v[1];
+            }
+        } else if constexpr (T == 4) {
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                const u32x4 v = ld_at_nt<u32x4>(b + 64 * j, 4u * (4u * c16 + 256u * g));
+#pragma unroll
+                for (int i = 0; i < 4; ++i) d[4 * l + i][j] = v[i];
+            }
+        } else if constexpr (T == 8) {
+            u32 v[8][4];
+#pragma unroll
+            for (int x = 0; x < 8; ++x) {
+                const u32x4 q = ld_at_nt<u32x4>(b + 128 * x, 4u * (4u * (g & 1u) + 8u * c16 + 1024u * (g >> 1)));
+#pragma unroll
+                for (int i = 0; i < 4; ++i) v[x][i] = q[i];
+            }
+#pragma unroll
+            for (int x = 0; x < 4; ++x)
+#pragma unroll
+                for (int i = 0; i < 4; ++i) swap_l4(v[x][i], v[x | 4][i]);
+#pragma unroll
+            for (int x = 0; x < 8; ++x)
+#pragma unroll
+                for (int i = 0; i < 4; ++i) d[8 * l + i + 4 * (x >> 2)][x & 3] = v[x][i];
+        } else {
+            static_assert(T == 16 && NT == 16, "one 4096-point line per wave");
+            u32 v[16][4];
+#pragma unroll
+            for (int x = 0; x < 16; ++x) {
+                const u32x4 q = ld_at_nt<u32x4>(b + 256 * x, 4u * (4u * g + 16u * c16));
+#pragma unroll
+                for (int i = 0; i < 4; ++i) v[x][i] = q[i];
+            }
+            transpose_gi_tile(v, d);
+        }
+    }
+}
+
+// ----------------------------------------------------------------------------
 // k_big<W>: one signal of N = 4096*W (W = 2, 4, 8, 16) per workgroup of W
 // waves, in a single HBM round trip.  Radix list [16, 16, 16, W]; position
 // p = d0 + 16*d1 + 256*d2 + 4096*w, wave w loads chunk w.
@@ -383,6 +445,129 @@ __device__ __forceinline__ void big_phase2_regs(u32 (&e)[16][4], int w, u32* lds
                 for (int s = 0; s < W; ++s) o[(r * QN + q) * W + s][j] = pack(x[s]);
             }
         }
+    }
+}
+
+// Natural-order input of the single-pass kernels: one signal of N = 4096*W
+// as W columns (index mod W = d3, the line of wave w) of 4096 rows rho = d2 +
+// 16*d1 + 256*d0, loaded with contiguous 16-byte accesses, through LDS once
+// (W = 16: in two rounds of 128 KiB) into the register layout of big_body.
+// LDS is column-major in quads of four rows, so that a reader takes four
+// adjacent d2 with one 16-byte access: 16 reads per lane, where 4-byte reads
+// of a row-major image took 64 (128 half-masked ones at W = 16).  The writers
+// scatter words (W = 2: pairs of rows), which move the same bytes.
+// Quad of (column c, row quad q): bits 0-1 ^= bits 4-5, and, for W >= 4, the
+// column's bits (W = 16: c/4) from bit 3 down: the 64 words of a write fall on
+// 64 banks (also those of 64 adjacent indices, W = 2 excepted, whose pair of
+// columns then shares one address computation), each 16 lanes of a read on 16
+// different quads.
+template <int W>
+__device__ __forceinline__ u32 nat_quad(u32 q, u32 c) {
+    return q ^ ((q >> 4) & 3u) ^ (W == 2 ? 0u : W == 4 ? c << 2 : W == 8 ? c << 1 : (c >> 2) << 2);
+}
+// LDS word of natural index m of a signal of W < 16 columns.
+template <int W>
+__device__ __forceinline__ u32 nat_big_word(u32 m) {
+    const u32 c = m % W, rho = m / W;
+    return 4096u * c + 4u * nat_quad<W>(rho >> 2, c) + (rho & 3u);
+}
+
+// The line of wave w from there, in the register layout of big_body.
+template <int W>
+__device__ __forceinline__ void big_nat_read(u32 (&d)[16][4], u32 w, const u32* lds, int lane) {
+    const u32 c16 = (u32)lane & 15u, g = (u32)lane >> 4;
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+#pragma unroll
+        for (int h = 0; h < 4; ++h) {
+            u32 r[4];
+            load4(r, lds + 4096u * w + 4u * nat_quad<W>((u32)h + 4u * (c16 + 16u * (4u * g + (u32)j)), w));
+#pragma unroll
+            for (int i = 0; i < 4; ++i) d[4 * h + i][j] = r[i];
+        }
+}
+
+// W = 2, 4, 8; the caller synchronises before reusing the LDS.
+template <int W>
+__device__ __forceinline__ void big_nat_load(u32 (&d)[16][4], const u32* __restrict__ src, u32 w, u32* lds, int lane) {
+    static_assert(W == 2 || W == 4 || W == 8, "whole signal in LDS");
+    u32 v[16][4];
+#pragma unroll
+    for (int x = 0; x < 16; ++x) load4_nt(v[x], src + 4096u * w + 256u * x + 4u * (u32)lane);
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int x = 0; x < 16; ++x) {
+        // row of this lane's first word (256/W rows per load)
+        const u32 rho = (4096u / W) * w + (256u / W) * x + 4u * (u32)lane / W;
+        if constexpr (W == 2) {  // rows rho, rho + 1 of both columns
+#pragma unroll
+            for (u32 c = 0; c < 2; ++c)
+                *reinterpret_cast<u32x2*>(lds + 4096u * c + 4u * nat_quad<W>(rho >> 2, c) + (rho & 3u)) =
+                    u32x2{v[x][c], v[x][2 + c]};
+        } else {  // four columns of row rho
+            const u32 col = W == 8 ? 4u * ((u32)lane & 1u) : 0u;
+#pragma unroll
+            for (u32 k = 0; k < 4; ++k)
+                lds[4096u * (col + k) + 4u * nat_quad<W>(rho >> 2, col + k) + (rho & 3u)] = v[x][k];
+        }
+    }
+    __syncthreads();
+    big_nat_read<W>(d, w, lds, lane);
+}
+
+// The same in two rounds through W*8 KiB, for W = 16 and for several signals
+// per workgroup; row rho at src + rho*row_words (W words of it).  A round
+// holds the rows with bit 9 (d0 bit 1) equal to its number, so that which
+// loads it writes and which words (j >> 1) it reads is fixed at compile time.
+// Every barrier is a workgroup barrier; the caller synchronises before reusing
+// the LDS.
+template <int W>
+__device__ __forceinline__ void big_nat_load2(u32 (&d)[16][4], const u32* __restrict__ src, u32 row_words, u32 w,
+                                              u32* lds, int lane) {
+    // load x = 8r + xx holds 256/W rows: the low LB row bits are the lane's
+    // (and, for W = 2, the word's), then xx, bit 9 = r, then the wave's bits
+    constexpr u32 LB = W == 2 ? 7 : W == 4 ? 6 : W == 8 ? 5 : 4;
+    const u32 L = (u32)lane, c16 = L & 15u, g = L >> 4;
+    auto above = [](u32 k) { return ((k & ((1u << (9 - LB)) - 1u)) << LB) | ((k >> (9 - LB)) << 10); };
+    u32 v[16][4];
+#pragma unroll
+    for (int x = 0; x < 16; ++x) {
+        const u32 row = above((u32)(x & 7) | (w << 3)) | ((u32)(x >> 3) << 9);
+        const u32x4 q = ld_at_nt<u32x4>(src + (size_t)row * row_words,
+                                        W <= 4 ? 16u * L : 4u * (4u * L / W * row_words + (4u * L & (W - 1u))));
+#pragma unroll
+        for (int i = 0; i < 4; ++i) v[x][i] = q[i];
+    }
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int r = 0; r < 2; ++r) {
+        if (r) __syncthreads();  // round 0's reads are done
+#pragma unroll
+        for (int xx = 0; xx < 8; ++xx) {
+            // row without bit 9
+            const u32 k = (u32)xx | (w << 3), rho = (k << LB) | (4u * L / W);
+            if constexpr (W == 2) {
+#pragma unroll
+                for (u32 c = 0; c < 2; ++c)
+                    *reinterpret_cast<u32x2*>(lds + 2048u * c + 4u * nat_quad<W>(rho >> 2, c) + (rho & 3u)) =
+                        u32x2{v[8 * r + xx][c], v[8 * r + xx][2 + c]};
+            } else {
+                const u32 col = 4u * L & (W - 1u);
+#pragma unroll
+                for (u32 i = 0; i < 4; ++i)
+                    lds[2048u * (col + i) + 4u * nat_quad<W>(rho >> 2, col + i) + (rho & 3u)] = v[8 * r + xx][i];
+            }
+        }
+        __syncthreads();
+#pragma unroll
+        for (int jj = 0; jj < 2; ++jj)
+#pragma unroll
+            for (int h = 0; h < 4; ++h) {
+                u32 t[4];
+                load4(t, lds + 2048u * w + 4u * nat_quad<W>((u32)h + 4u * (c16 + 16u * (2u * g + (u32)jj)), w));
+#pragma unroll
+                for (int i = 0; i < 4; ++i) d[4 * h + i][2 * r + jj] = t[i];
+            }
     }
 }
 

@@ -386,50 +386,73 @@ __device__ __forceinline__ u32 rev_pos_pow2(u32 x, const RevSpec& s) {
     return idx;
 }
 
-// Reads a wave's natural-order chunk (ntl tiles, whole lines of 256*T) from
-// its LDS slice into the digit-reversed register layout of k_rows.
-// The word of (t, j), nat_lds_word(m) with m = (t/T) L + (t%T) + T c16 +
-// 16T (4g + j), is (t/T) L + ((t%T) op y_j) with a per-lane y_j (the swizzle
-// depends on bits 6-7 of m, which t does not reach): op is + for T <= 4 (y_j
-// has no bits below 2) and ^ for T = 8, 16, so the per-element address is a
-// constant offset or one XOR.
+// For T >= 4 a reader wants four adjacent d2 = four adjacent words m of a
+// line, so the chunk is kept in quads: word m at quad m/4 with bits 0-1 ^=
+// bits 4-5 (16 reading lanes on 16 quads of the banks, the words of 64
+// adjacent indices on 64 banks).
+template <int T>
+__device__ __forceinline__ u32 nat_chunk_word(u32 m) {
+    if constexpr (T < 4) return nat_lds_word(m);
+    return m ^ (((m >> 6) & 3u) << 2);
+}
+
+// Reads a wave's natural-order chunk (ntl tiles, whole lines of 256*T, words
+// nat_chunk_word) from its LDS slice into the digit-reversed register layout
+// of k_rows.  T < 4: the word of (t, j) is (t/T) L + (t%T) + y_j with a
+// per-lane y_j (the swizzle depends on bits 6-7 of m, which t does not reach,
+// and y_j has no bits below 2).
 template <int T, int NT = 16>
 __device__ __forceinline__ void nat_rows_read(u32 (&d)[NT][4], const u32* wl, u32 ntl, int lane) {
     constexpr u32 L = 256u * T;
     const u32 c16 = (u32)lane & 15u, g = (u32)lane >> 4;
-    u32 y[4];
+    if constexpr (T >= 4) {
+        (void)ntl;  // absent tiles read what their slots hold: never stored
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
-        const u32 lp = T * c16 + 16u * T * (4u * g + (u32)j);
-        y[j] = lp ^ (((lp >> 6) & 3u) * 0x14u);
+        for (int l = 0; l < NT / T; ++l)
+#pragma unroll
+            for (int j = 0; j < 4; ++j)
+#pragma unroll
+                for (int h = 0; h < T / 4; ++h) {
+                    u32 r[4];
+                    load4(r, wl + nat_chunk_word<T>((u32)l * L + 4u * h + T * (c16 + 16u * (4u * g + (u32)j))));
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) d[l * T + 4 * h + i][j] = r[i];
+                }
+    } else {
+        u32 y[4];
+#pragma unroll
+        for (int j = 0; j < 4; ++j) y[j] = nat_lds_word(T * c16 + 16u * T * (4u * g + (u32)j));
+#pragma unroll
+        for (int t = 0; t < NT; ++t)
+#pragma unroll
+            for (int j = 0; j < 4; ++j) d[t][j] = (u32)t < ntl ? wl[(u32)(t / T) * L + (u32)(t % T) + y[j]] : 0u;
     }
-#pragma unroll
-    for (int t = 0; t < NT; ++t)
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            const u32 off = T <= 4 ? (u32)(t % T) + y[j] : (y[j] ^ (u32)(t % T));
-            d[t][j] = (u32)t < ntl ? wl[(u32)(t / T) * L + off] : 0u;
-        }
 }
 
-// 16-byte loads of ntl tiles at src (this wave's chunk) into the LDS slice,
-// then nat_rows_read.
-template <int T>
-__device__ __forceinline__ void nat_rows_load(u32 (&d)[16][4], const u32* __restrict__ src, u32* wl, u32 ntl,
+// Loads ntl tiles at src (this wave's chunk, NT tiles at most) into that
+// layout: T >= 2 straight into registers (nat_direct_load; absent lines load
+// the last present one), T = 1 with 16-byte loads through the LDS slice.
+template <int T, int NT = 16>
+__device__ __forceinline__ void nat_rows_load(u32 (&d)[NT][4], const u32* __restrict__ src, u32* wl, u32 ntl,
                                               int lane) {
-    src += 4u * lane;
-    u32 v[16][4];
+    if constexpr (T >= 2) {
+        nat_direct_load<T, NT>(
+            d, [&](int l) { return src + 256u * T * min((u32)l, ntl / T - 1u); }, lane);
+    } else {
+        src += 4u * lane;
+        u32 v[NT][4];
 #pragma unroll
-    for (int t = 0; t < 16; ++t)
-        if ((u32)t < ntl) load4_nt(v[t], src + 256u * t);
+        for (int t = 0; t < NT; ++t)
+            if ((u32)t < ntl) load4_nt(v[t], src + 256u * t);
 #pragma unroll
-    for (int t = 0; t < 16; ++t)
-        if ((u32)t < ntl) store4(wl + nat_lds_word(256u * t + 4u * lane), v[t]);
-    __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
-    nat_rows_read<T>(d, wl, ntl, lane);
+        for (int t = 0; t < NT; ++t)
+            if ((u32)t < ntl) store4(wl + nat_lds_word(256u * t + 4u * lane), v[t]);
+        __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+        nat_rows_read<T, NT>(d, wl, ntl, lane);
+    }
 }
 
-template <int T, int SIGN, bool CACHED = false>
+template <int T, int SIGN, bool CACHED = false, int NT = 16>
 __global__ __launch_bounds__(256) TCFFT_MFMA_BUDGET void k_rows_nat(const u32* in, u32* out,
                                                                   u32 n_tiles, const float2* __restrict__ w4096,
                                                                   u32 nx_log2, const u32* __restrict__ xpos,
@@ -439,17 +462,17 @@ __global__ __launch_bounds__(256) TCFFT_MFMA_BUDGET void k_rows_nat(const u32* i
     const int lane = threadIdx.x & 63;
     const u32 wib = (u32)__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
     const u32 wave = blockIdx.x * (blockDim.x >> 6) + wib;
-    const u32 tile0 = wave * 16u;
+    const u32 tile0 = wave * (u32)NT;
     if (tile0 >= n_tiles) return;
     start_delay(sched);
-    const u32 ntl = min(16u, n_tiles - tile0);
-    u32* const wl = lds + wib * 4096u;
+    const u32 ntl = min((u32)NT, n_tiles - tile0);
+    u32* const wl = lds + wib * (256u * NT);  // T = 1 only
     const int c16 = lane & 15, g = lane >> 4;
-    auto load = [&](u32 (&d)[16][4]) { nat_rows_load<T>(d, in + (size_t)tile0 * 256u, wl, ntl, lane); };
+    auto load = [&](u32 (&d)[NT][4]) { nat_rows_load<T, NT>(d, in + (size_t)tile0 * 256u, wl, ntl, lane); };
     const u32 lane_off = 16u * c16 + 4u * g;
-    // destination line of each of the wave's 16/T lines, once per line and
+    // destination line of each of the wave's NT/T lines, once per line and
     // wave-uniform (2D: the x position from the plan's table)
-    constexpr u32 LPW = 16u / T;
+    constexpr u32 LPW = NT / T;
     u32 dst_line[LPW];
 #pragma unroll
     for (u32 l = 0; l < LPW; ++l) {
@@ -462,25 +485,30 @@ __global__ __launch_bounds__(256) TCFFT_MFMA_BUDGET void k_rows_nat(const u32* i
         dst_line[l] = (u32)__builtin_amdgcn_readfirstlane((int)dst);
     }
     auto tile_ptr = [&](int t) -> u32* { return out + (size_t)dst_line[t / T] * L + 256u * ((u32)t % T) + lane_off; };
-    rows_body<T, false, SIGN, 16, CACHED>(tile_ptr, ntl, tile0, w4096, EpiParams{}, load);
+    rows_body<T, false, SIGN, NT, CACHED>(tile_ptr, ntl, tile0, w4096, EpiParams{}, load);
 }
 
 // k_rows_half on natural-order input (a 4096-point row pass of
-// tcfft_exec_natural, in -> out, in place allowed): the line's WPL waves
-// load its parts with 16-byte loads into 16 KiB of LDS (word nat_lds_word,
-// as k_rows_nat), and after a barrier part h reads tiles d2 = (16/WPL) h ..
-// of the digit-reversed layout (word y_j ^ d2, see nat_rows_read); the rest
-// is k_rows_half's, with the exchange rows in a second 16 KiB.  Every load
-// of a line precedes the barrier before its first store, so in place is
-// safe.  2D (nx_log2 > 0): input line img*nx + x goes to line img*nx +
-// xpos[x].  One line per workgroup.
-template <int SIGN, bool CACHED, int WPL>
+// tcfft_exec_natural, in -> out, in place allowed).  DIRECT: part h loads its
+// tiles d2 = (16/WPL) h .. straight into the digit-reversed layout as
+// nat_direct_load does, each lane four adjacent d2 (pieces of 32 or 16 bytes
+// of every 64; the other waves of the line read the rest of the same cache
+// lines).  Else (two waves only) the waves load whole lines into 16 KiB of
+// LDS (word nat_lds_word), and after a barrier part h reads its tiles (word
+// nat_lds_word(m) = y_j ^ d2 with a per-lane y_j): the pieces cost the caches more accesses, so
+// once many lines per CU stream from HBM whole lines are faster (4096 x 4096:
+// 22.7 us direct, 27.1 through LDS; 4096 x 8192 50.4 and 48.1; 4096 x 16384
+// 94.6 and 90.7).  The rest is k_rows_half's.  Every load of a line precedes
+// the exchange barrier and its first store, so in place is safe.  2D
+// (nx_log2 > 0): input line img*nx + x goes to line img*nx + xpos[x].  One
+// line per workgroup.
+template <int SIGN, bool CACHED, int WPL, bool DIRECT>
 __global__ __launch_bounds__(256) TCFFT_MFMA_BUDGET void k_rows_half_nat(const u32* in, u32* out, u32 n_lines,
                                                                        const float2* __restrict__ w4096,
                                                                        u32 nx_log2, const u32* __restrict__ xpos,
                                                                        StartSched sched) {
     constexpr int TPW = 16 / WPL;
-    extern __shared__ u32 lds[];
+    extern __shared__ u32 xl[];  // the exchange rows
     const int lane = lane_id();
     const u32 c16 = (u32)lane & 15u, g = (u32)lane >> 4;
     const u32 h = (u32)__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
@@ -494,24 +522,21 @@ __global__ __launch_bounds__(256) TCFFT_MFMA_BUDGET void k_rows_half_nat(const u
         dst_line = (src_line & ~mask) | xpos[src_line & mask];
     }
     dst_line = (u32)__builtin_amdgcn_readfirstlane((int)dst_line);
-    u32* const xin = lds;          // the natural-order line
-    u32* const xl = lds + 4096u;   // the exchange rows
 
     Dit4096Tw tw;
     dit4096_tw_load(tw, lane, w4096);
     __builtin_amdgcn_sched_barrier(0);
-    {
-        const u32 part = (4096u / WPL) * h;
-        const u32* const src = in + (size_t)src_line * 4096u + part + 4u * (u32)lane;
-        u32 v[TPW][4];
-#pragma unroll
-        for (int t = 0; t < TPW; ++t) load4_nt(v[t], src + 256u * t);
-#pragma unroll
-        for (int t = 0; t < TPW; ++t) store4(xin + nat_lds_word(part + 256u * t + 4u * (u32)lane), v[t]);
-    }
-    __syncthreads();
     u32 d[TPW][4];
-    {
+    const u32* const src = in + (size_t)src_line * 4096u + (DIRECT ? (u32)TPW * h : 2048u * h);
+    if constexpr (!DIRECT) {
+        static_assert(DIRECT || WPL == 2, "the LDS form is kept for two waves");
+        u32* const xin = xl + 4096u;  // the natural-order line
+        u32 v[8][4];
+#pragma unroll
+        for (int t = 0; t < 8; ++t) load4_nt(v[t], src + 256u * t + 4u * (u32)lane);
+#pragma unroll
+        for (int t = 0; t < 8; ++t) store4(xin + nat_lds_word(2048u * h + 256u * t + 4u * (u32)lane), v[t]);
+        __syncthreads();
         u32 y[4];
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
@@ -519,9 +544,29 @@ __global__ __launch_bounds__(256) TCFFT_MFMA_BUDGET void k_rows_half_nat(const u
             y[j] = lp ^ (((lp >> 6) & 3u) * 0x14u);
         }
 #pragma unroll
-        for (int t = 0; t < TPW; ++t)
+        for (int t = 0; t < 8; ++t)
 #pragma unroll
-            for (int j = 0; j < 4; ++j) d[t][j] = xin[y[j] ^ ((u32)TPW * h + (u32)t)];
+            for (int j = 0; j < 4; ++j) d[t][j] = xin[y[j] ^ (8u * h + (u32)t)];
+    } else if constexpr (WPL == 2) {
+        u32 v[8][4];  // lane bit 4 = d2 bit 2, lane bit 5 = d0 bit 3, x = d0 bits 0-2
+#pragma unroll
+        for (int x = 0; x < 8; ++x) load4(v[x], src + 256u * x + 16u * c16 + 4u * (g & 1u) + 2048u * (g >> 1));
+#pragma unroll
+        for (int x = 0; x < 4; ++x)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) swap_l4(v[x][i], v[x | 4][i]);
+#pragma unroll
+        for (int x = 0; x < 8; ++x)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) d[i + 4 * (x >> 2)][x & 3] = v[x][i];
+    } else {
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            u32 v[4];
+            load4(v, src + 256u * (4u * g + (u32)j) + 16u * c16);
+#pragma unroll
+            for (int i = 0; i < 4; ++i) d[i][j] = v[i];
+        }
     }
     const Dft16Op op = make_dft16(lane, SIGN);
     rows_split_part<SIGN, WPL>(h, d, tw, op, xl);
@@ -659,14 +704,14 @@ __global__ __launch_bounds__(256) TCFFT_MFMA_BUDGET void k_c2r(const u32* __rest
                     if (j == 0 && lane == 0) q = {2.f * q.x, 2.f * q.y};
                     else sum = {0.5f * sum.x, 0.5f * sum.y};
                 }
-                wl[nat_lds_word(i * L + k)] = pack(sum.x - q.y, sum.y + q.x);                  // S + P
-                if (k != 0) wl[nat_lds_word(i * L + (L - k))] = pack(sum.x + q.y, q.x - sum.y);  // conj(S - P)
+                wl[nat_chunk_word<T>(i * L + k)] = pack(sum.x - q.y, sum.y + q.x);                  // S + P
+                if (k != 0) wl[nat_chunk_word<T>(i * L + (L - k))] = pack(sum.x + q.y, q.x - sum.y);  // conj(S - P)
                 w = cmul(w, step);
             }
             if (lane == 0) {
                 // k = L/2: W_N^{-L/2} = i, so Z'[L/2] = 2 conj X[L/2]
                 const cf a = unpack(vm);
-                wl[nat_lds_word(i * L + L / 2u)] = pack(2.f * hf * a.x, -2.f * hf * a.y);
+                wl[nat_chunk_word<T>(i * L + L / 2u)] = pack(2.f * hf * a.x, -2.f * hf * a.y);
             }
         }
         __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
@@ -1366,63 +1411,14 @@ __global__ __launch_bounds__(64 * W) TCFFT_MFMA_BUDGET void k_big(u32* __restric
 // ----------------------------------------------------------------------------
 // k_big_nat<W>: k_big<W> (W = 2, 4, 8, 16) on natural-order input, in -> out (in
 // place allowed: a workgroup reads its whole signal before its first store).
-// Each wave loads its natural 4096-element chunk with 16-byte loads and stores
-// it to LDS (the signal, W*16 KiB, fits at once); after a barrier wave w reads
-// the chunk k_big loads in the drop-in order: register (t, lane (c16, g),
-// word j) = position 4096w + 256t + 16c16 + 4g + j, natural index
-// w + W*(t + 16*c16 + 256*(4g + j)).  The LDS word XORs two 2-bit fields of
-// the index into bits 2-3 and 4-5 (NatBigSwz): the 16-byte writes stay whole
-// and conflict-free, the b32 reads drop from 32..64-way to 4-way conflicts.
+// The waves load the signal with 16-byte accesses and exchange it through LDS
+// (big_nat_load, big_nat_load2), after which wave w holds the chunk k_big
+// loads in the drop-in order: register (t, lane (c16, g), word j) = position
+// 4096w + 256t + 16c16 + 4g + j, natural index w + W*(t + 16*c16 + 256*(4g + j)).
+// Measured, LDS read as 4-byte words -> in 16-byte quads: 65536 x 256 36.3 ->
+// 34.4 us, 32768 x 2000 148 -> 137.7, 16384 x 4096 99.1 -> 96.7, 8192 x 2048
+// 31.8 -> 31.4.
 // 2D (nx_log2 > 0, out of place): line img*nx + x goes to img*nx + pos(x).
-template <int W>
-struct NatBigSwz;
-template <>
-struct NatBigSwz<2> {
-    static constexpr u32 A = 7, B = 6;
-};
-template <>
-struct NatBigSwz<4> {
-    static constexpr u32 A = 6, B = 8;
-};
-template <>
-struct NatBigSwz<8> {
-    static constexpr u32 A = 7, B = 9;
-};
-
-template <int W>
-__device__ __forceinline__ u32 nat_big_word(u32 m) {
-    return m ^ (((m >> NatBigSwz<W>::A) & 3u) << 2) ^ (((m >> NatBigSwz<W>::B) & 3u) << 4);
-}
-
-// W = 16 (65536 points, 256 KiB per signal) goes through 128 KiB of LDS in
-// two rounds split by index bit 11: writer tile bit 3, reader lane bit
-// c16[3].  Round word: bit 11 removed, then bits 8-9 into 2-3 and 13-14 into
-// 4-5 (writes conflict-free, reads at most 2-way among the 32 active lanes).
-__device__ __forceinline__ u32 nat16_word(u32 n) {
-    const u32 m = (n & 2047u) | ((n >> 12) << 11);
-    return m ^ (((m >> 8) & 3u) << 2) ^ (((m >> 13) & 3u) << 4);
-}
-
-// Word of natural index n in a staging round that holds the indices with
-// bit B of n equal to the round number: bit B removed, then bits 8-9 into
-// 2-3 and 13-14 into 4-5 (a bijection that keeps 16-byte chunks whole).
-template <int B>
-__device__ __forceinline__ u32 nat_split_word(u32 n) {
-    const u32 m = (n & ((1u << B) - 1u)) | ((n >> (B + 1)) << B);
-    return m ^ (((m >> 8) & 3u) << 2) ^ (((m >> 13) & 3u) << 4);
-}
-
-// nat_split_word<B>(p + q) for p < 2^LW and a lane index q whose bits below
-// LW are zero (LW <= 8 <= B): the swizzle bits come from q alone, so the
-// word is base + (p ^ xlo) with base and xlo computed once per lane.
-template <int B, int LW>
-__device__ __forceinline__ void nat_split_lane(u32 q, u32& base, u32& xlo) {
-    const u32 m = (q & ((1u << B) - 1u)) | ((q >> (B + 1)) << B);
-    const u32 x = (((m >> 8) & 3u) << 2) ^ (((m >> 13) & 3u) << 4);
-    xlo = x & ((1u << LW) - 1u);
-    base = m ^ (x & ~((1u << LW) - 1u));
-}
-
 template <int W, int SIGN, bool CACHED = false>
 __global__ __launch_bounds__(64 * W) TCFFT_MFMA_BUDGET void k_big_nat(
     const u32* in, u32* out, const float2* __restrict__ w4096,
@@ -1440,57 +1436,11 @@ __global__ __launch_bounds__(64 * W) TCFFT_MFMA_BUDGET void k_big_nat(
     if constexpr (W < 16) {
         big_tw_load<W, false>(bt, lane, (int)w, sig, w4096, wn_hi, wn_lo, wn_lo_bits, EpiParams{});
         __builtin_amdgcn_sched_barrier(0);
-        {
-            u32 v[16][4];
-            const u32* src = in + (size_t)sig * N + 4096u * w + 4u * lane;
-#pragma unroll
-            for (int t = 0; t < 16; ++t) load4_nt(v[t], src + 256u * t);
-            __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-            for (int t = 0; t < 16; ++t) store4(lds + nat_big_word<W>(4096u * w + 256u * t + 4u * lane), v[t]);
-        }
-        __syncthreads();
-        // reader word of register (t, j): nat_big_word<W>(w + W (t + 16 c16 +
-        // 256 (4g + j))) = lane_base + ((w + W t) ^ xlo) + 256 W j: the swizzle
-        // bits come from the lane's part q = 16W c16 + 1024W g alone, its bits
-        // below log2(16W) (xlo) meet w + W t, the rest (q's) do not
-        constexpr u32 LW = W == 2 ? 5u : W == 4 ? 6u : 7u;  // log2(16W)
-        const u32 q = 16u * W * (u32)c16 + 1024u * W * (u32)g;
-        const u32 x = (((q >> NatBigSwz<W>::A) & 3u) << 2) ^ (((q >> NatBigSwz<W>::B) & 3u) << 4);
-        const u32 xlo = x & ((1u << LW) - 1u), lane_base = q ^ (x & ~((1u << LW) - 1u));
-#pragma unroll
-        for (int t = 0; t < 16; ++t) {
-            const u32* a = lds + lane_base + ((w + W * (u32)t) ^ xlo);
-#pragma unroll
-            for (int j = 0; j < 4; ++j) d[t][j] = a[256u * W * j];
-        }
+        big_nat_load<W>(d, in + (size_t)sig * N, w, lds, lane);
     } else {
         // data first, the twiddle tables after the exchange: the pending
         // half of the loaded data and the reader registers fit the budget
-        u32 v[16][4];
-        const u32* src = in + (size_t)sig * N + 4096u * w + 4u * lane;
-#pragma unroll
-        for (int t = 0; t < 16; ++t) load4_nt(v[t], src + 256u * t);
-        // reader word of register (t, j): nat16_word(w + 16 (t + 16 c16 +
-        // 256 (4g + j))) = lane_base + 16 (t ^ g) + 2048 j, computed once per
-        // lane (the per-element form cost about 1600 VALU instructions a wave)
-        const u32 lane_base = ((u32)w ^ (4u * ((u32)c16 & 3u))) + 256u * ((u32)c16 & 7u) + 8192u * (u32)g;
-#pragma unroll
-        for (int r = 0; r < 2; ++r) {
-            if (r) __syncthreads();  // round 0's reads are done
-#pragma unroll
-            for (int tt = 0; tt < 8; ++tt)
-                store4(lds + nat16_word(4096u * w + 256u * (8u * r + tt) + 4u * lane), v[8 * r + tt]);
-            __syncthreads();
-            if ((u32)(c16 >> 3) == (u32)r) {
-#pragma unroll
-                for (int t = 0; t < 16; ++t) {
-                    const u32* a = lds + lane_base + 16u * ((u32)t ^ (u32)g);
-#pragma unroll
-                    for (int j = 0; j < 4; ++j) d[t][j] = a[2048u * j];
-                }
-            }
-        }
+        big_nat_load2<16>(d, in + (size_t)sig * N, 16u, w, lds, lane);
         big_tw_load<W, false>(bt, lane_id(), (int)w, sig, w4096, wn_hi, wn_lo, wn_lo_bits, EpiParams{});
     }
     __syncthreads();  // every wave has read its chunk before the exchange reuses the LDS
@@ -1584,21 +1534,7 @@ __global__ __launch_bounds__(64 * W) TCFFT_MFMA_BUDGET void k_r2c_big(
     big_tw_load<W, false>(bt, lane, (int)w, sig, w4096, wn_hi, wn_lo, wn_lo_bits, EpiParams{});
     __builtin_amdgcn_sched_barrier(0);
     u32 d[16][4];
-    {
-        u32 v[16][4];
-        const u32* src = in + (size_t)sig * L + 4096u * w + 4u * lane;
-#pragma unroll
-        for (int t = 0; t < 16; ++t) load4_nt(v[t], src + 256u * t);
-        __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-        for (int t = 0; t < 16; ++t) store4(lds + nat_big_word<W>(4096u * w + 256u * t + 4u * lane), v[t]);
-    }
-    __syncthreads();
-#pragma unroll
-    for (int t = 0; t < 16; ++t)
-#pragma unroll
-        for (int j = 0; j < 4; ++j)
-            d[t][j] = lds[nat_big_word<W>(w + W * ((u32)t + 16u * c16 + 256u * (4u * g + j)))];
+    big_nat_load<W>(d, in + (size_t)sig * L, w, lds, lane);
     __syncthreads();
     const Dft16Op op = make_dft16(lane, -1);
     u32 e[16][4];
@@ -1693,11 +1629,7 @@ __global__ __launch_bounds__(64 * W) TCFFT_MFMA_BUDGET void k_c2r_big(
     }
     __syncthreads();
     u32 d[16][4];
-#pragma unroll
-    for (int t = 0; t < 16; ++t)
-#pragma unroll
-        for (int j = 0; j < 4; ++j)
-            d[t][j] = lds[nat_big_word<W>(w + W * ((u32)t + 16u * c16 + 256u * (4u * g + j)))];
+    big_nat_read<W>(d, w, lds, lane);
     __syncthreads();
     const Dft16Op op = make_dft16(lane, +1);
     u32 e[16][4];
@@ -1749,7 +1681,7 @@ static KernelInfo kernel_info(K kernel, int threads, size_t lds) {
 }
 
 // Waves per workgroup of the kernels whose waves each own a 16 KiB LDS slice
-// (k_rows_nat, k_r2c, k_c2r): four, or one when the grid has fewer than four
+// (k_r2c, k_c2r): four, or one when the grid has fewer than four
 // waves per CU, where four-wave workgroups would leave most CUs idle
 // (1024 x 1024 natural order: 64 workgroups on 256 CUs).
 template <class K>
@@ -1880,16 +1812,12 @@ static hipError_t launch_cols_t(u32* buf, u32 s_log2, u32 outer, int sign, const
     return hipGetLastError();
 }
 
-template <int T, int SIGN>
-static hipError_t launch_rows_nat_t(const u32* in, u32* out, u32 n_tiles, const float2* w4096, u32 nx_log2,
-                                    const u32* xpos, StartSched sched, hipStream_t st) {
-    // cached output stores switch only for 4096-point lines (as launch_rows_t)
-    auto k = k_rows_nat<T, SIGN, false>;
-    if constexpr (T == 16)
-        if (sched.cached_out) k = k_rows_nat<T, SIGN, true>;
-    const u32 waves = (n_tiles + 15) / 16;
-    const u32 wg = slice_wg(k, waves);
-    const size_t lds = wg * 4096 * sizeof(u32);  // 16 KiB per wave
+template <int T, int SIGN, bool CACHED, int NT>
+static hipError_t launch_rows_nat_nt(const u32* in, u32* out, u32 n_tiles, const float2* w4096, u32 nx_log2,
+                                     const u32* xpos, StartSched sched, u32 wg, hipStream_t st) {
+    auto k = k_rows_nat<T, SIGN, CACHED, NT>;
+    const u32 waves = (n_tiles + NT - 1) / NT;
+    const size_t lds = T == 1 ? wg * NT * 256 * sizeof(u32) : 0;
     const KernelInfo ki = kernel_info(k, (int)(64 * wg), lds);
     if (ki.lds_status != hipSuccess) return ki.lds_status;
     if (sched.groups == 0) sched.delay = 0;
@@ -1899,15 +1827,38 @@ static hipError_t launch_rows_nat_t(const u32* in, u32* out, u32 n_tiles, const 
     return hipGetLastError();
 }
 
-// k_rows_half_nat<WPL> over n_tiles / 16 lines, one line (WPL waves,
-// 32 KiB of LDS) per workgroup.
-template <int SIGN, bool CACHED, int WPL>
+template <int T, int SIGN>
+static hipError_t launch_rows_nat_t(const u32* in, u32* out, u32 n_tiles, const float2* w4096, u32 nx_log2,
+                                    const u32* xpos, StartSched sched, u32 tiles, u32 wg, hipStream_t st) {
+    // cached output stores switch only for 4096-point lines (as launch_rows_t)
+    if constexpr (T == 16) {
+        if (sched.cached_out)
+            return launch_rows_nat_nt<T, SIGN, true, 16>(in, out, n_tiles, w4096, nx_log2, xpos, sched, wg, st);
+    } else {
+        if (tiles == 8)
+            return launch_rows_nat_nt<T, SIGN, false, 8>(in, out, n_tiles, w4096, nx_log2, xpos, sched, wg, st);
+        if constexpr (T <= 4)
+            if (tiles == 4)
+                return launch_rows_nat_nt<T, SIGN, false, 4>(in, out, n_tiles, w4096, nx_log2, xpos, sched, wg, st);
+    }
+    if (tiles != 16) return hipErrorInvalidValue;
+    return launch_rows_nat_nt<T, SIGN, false, 16>(in, out, n_tiles, w4096, nx_log2, xpos, sched, wg, st);
+}
+
+// k_rows_half_nat<WPL> over n_tiles / 16 lines, one line (WPL waves, 16 KiB
+// of LDS, 32 when not DIRECT) per workgroup.
+template <int SIGN, bool CACHED, int WPL, bool DIRECT = true>
 static hipError_t launch_rows_half_nat_t(const u32* in, u32* out, u32 n_tiles, const float2* w4096, u32 nx_log2,
                                          const u32* xpos, StartSched sched, hipStream_t st) {
     const u32 lines = n_tiles / 16u;
-    const size_t lds = 8192u * sizeof(u32);
-    auto k = k_rows_half_nat<SIGN, CACHED, WPL>;
+    const size_t lds = (DIRECT ? 4096u : 8192u) * sizeof(u32);
+    auto k = k_rows_half_nat<SIGN, CACHED, WPL, DIRECT>;
     const KernelInfo ki = kernel_info(k, 64 * WPL, lds);
+    // whole lines through LDS above 16 lines per CU (see the kernel)
+    if constexpr (WPL == 2 && DIRECT) {
+        if (lines > 16u * ki.cus)
+            return launch_rows_half_nat_t<SIGN, CACHED, WPL, false>(in, out, n_tiles, w4096, nx_log2, xpos, sched, st);
+    }
     if (ki.lds_status != hipSuccess) return ki.lds_status;
     if (sched.groups == 0) sched.delay = 0;
     if (sched.delay) sched.resident = ki.resident;
@@ -1926,24 +1877,24 @@ static hipError_t launch_rows_half_nat_w(const u32* in, u32* out, u32 n_tiles, i
 }
 
 hipError_t launch_rows_nat(int T, const u32* in, u32* out, u32 n_tiles, int sign, const float2* w4096, u32 nx_log2,
-                           const u32* xpos, StartSched sched, u32 tiles_per_wave, hipStream_t st) {
+                           const u32* xpos, StartSched sched, u32 tiles_per_wave, u32 wg_waves, hipStream_t st) {
     if (nx_log2 && !xpos) return hipErrorInvalidValue;
     if ((tiles_per_wave == 8 || tiles_per_wave == 4) && T == 16)
         return tiles_per_wave == 8
                    ? launch_rows_half_nat_w<2>(in, out, n_tiles, sign, w4096, nx_log2, xpos, sched, st)
                    : launch_rows_half_nat_w<4>(in, out, n_tiles, sign, w4096, nx_log2, xpos, sched, st);
-    if (tiles_per_wave != 16) return hipErrorInvalidValue;
+    if (wg_waves != 1 && wg_waves != 2 && wg_waves != 4) return hipErrorInvalidValue;
     switch (T * 2 + (sign < 0 ? 0 : 1)) {
-    case 2: return launch_rows_nat_t<1, -1>(in, out, n_tiles, w4096, nx_log2, xpos, sched, st);
-    case 3: return launch_rows_nat_t<1, +1>(in, out, n_tiles, w4096, nx_log2, xpos, sched, st);
-    case 4: return launch_rows_nat_t<2, -1>(in, out, n_tiles, w4096, nx_log2, xpos, sched, st);
-    case 5: return launch_rows_nat_t<2, +1>(in, out, n_tiles, w4096, nx_log2, xpos, sched, st);
-    case 8: return launch_rows_nat_t<4, -1>(in, out, n_tiles, w4096, nx_log2, xpos, sched, st);
-    case 9: return launch_rows_nat_t<4, +1>(in, out, n_tiles, w4096, nx_log2, xpos, sched, st);
-    case 16: return launch_rows_nat_t<8, -1>(in, out, n_tiles, w4096, nx_log2, xpos, sched, st);
-    case 17: return launch_rows_nat_t<8, +1>(in, out, n_tiles, w4096, nx_log2, xpos, sched, st);
-    case 32: return launch_rows_nat_t<16, -1>(in, out, n_tiles, w4096, nx_log2, xpos, sched, st);
-    case 33: return launch_rows_nat_t<16, +1>(in, out, n_tiles, w4096, nx_log2, xpos, sched, st);
+    case 2: return launch_rows_nat_t<1, -1>(in, out, n_tiles, w4096, nx_log2, xpos, sched, tiles_per_wave, wg_waves, st);
+    case 3: return launch_rows_nat_t<1, +1>(in, out, n_tiles, w4096, nx_log2, xpos, sched, tiles_per_wave, wg_waves, st);
+    case 4: return launch_rows_nat_t<2, -1>(in, out, n_tiles, w4096, nx_log2, xpos, sched, tiles_per_wave, wg_waves, st);
+    case 5: return launch_rows_nat_t<2, +1>(in, out, n_tiles, w4096, nx_log2, xpos, sched, tiles_per_wave, wg_waves, st);
+    case 8: return launch_rows_nat_t<4, -1>(in, out, n_tiles, w4096, nx_log2, xpos, sched, tiles_per_wave, wg_waves, st);
+    case 9: return launch_rows_nat_t<4, +1>(in, out, n_tiles, w4096, nx_log2, xpos, sched, tiles_per_wave, wg_waves, st);
+    case 16: return launch_rows_nat_t<8, -1>(in, out, n_tiles, w4096, nx_log2, xpos, sched, tiles_per_wave, wg_waves, st);
+    case 17: return launch_rows_nat_t<8, +1>(in, out, n_tiles, w4096, nx_log2, xpos, sched, tiles_per_wave, wg_waves, st);
+    case 32: return launch_rows_nat_t<16, -1>(in, out, n_tiles, w4096, nx_log2, xpos, sched, tiles_per_wave, wg_waves, st);
+    case 33: return launch_rows_nat_t<16, +1>(in, out, n_tiles, w4096, nx_log2, xpos, sched, tiles_per_wave, wg_waves, st);
     default: return hipErrorInvalidValue;
     }
 }
@@ -2242,12 +2193,12 @@ __global__ __launch_bounds__(1024) void k_multi(u32* __restrict__ buf, const Mul
 // Natural-order uneven batch (k_multi_nat): the tasks of k_multi on
 // natural-order input, in -> out (in place allowed: each signal belongs to
 // one wave or group, which reads it completely before its first store).
-// Row classes of 256..2048 points pass each wave's lines through the wave's
-// own 8 KiB of LDS (words k*L + natural index for the k-th line of a call)
-// and read them back in the digit-reversed register layout (nat_rows_read's
-// formula); a 4096-point line passes in two rounds split by index bit 8.
-// Big classes stage every group's signal in two rounds split by index bit
-// 9 or 11 (W * 8 KiB per group per round, 128 KiB in all).
+// Row classes load their lines straight into the digit-reversed register
+// layout (nat_direct_load), the 256-point class through the wave's own 8 KiB
+// of LDS; big classes exchange every group's signal in two rounds
+// (big_nat_load2, W * 8 KiB per group per round, 128 KiB in all).  Measured
+// against staging every class through LDS with 4-byte reads: 4096 signals of
+// 2^U{8..16} 153 -> 134.7 us, 2048 80.4 -> 70.8, 100 33.5 -> 24.1.
 
 template <int T, int SIGN>
 __device__ __forceinline__ void multi_rows_nat(const u32* in, u32* out, const MultiTask& tk,
@@ -2260,59 +2211,32 @@ __device__ __forceinline__ void multi_rows_nat(const u32* in, u32* out, const Mu
     const int c16 = lane & 15, g = lane >> 4;
     const u32 lane_off = 16u * c16 + 4u * g;
     const u32* offs = offsets + tk.first + first_line;
+    if (lines <= 0) return;
     if constexpr (T == 16) {
-        if (lines <= 0) return;
-        // one 4096-point line per wave through the wave's 2048-word slice in
-        // two rounds: round r holds the natural indices with bit 8 = r, i.e.
-        // the loaded tiles with t & 1 = r and the read words with j & 1 = r
-        // (reader index t + 16*c16 + 256*(4g + j)), so that which registers
-        // each round writes and reads is fixed at compile time
-        u32* const wl = lds + (u32)wave * 2048u;
-        auto load = [&](u32 (&d)[16][4]) {
-            u32 v[16][4];
-            const u32* src = in + offs[0] + 4u * lane;
-#pragma unroll
-            for (int t = 0; t < 16; ++t) load4_nt(v[t], src + 256u * t);
-            // reader word of (t, j): base_j + (t ^ xlo_j) (nat_split_lane)
-            u32 base[4], xlo[4];
-#pragma unroll
-            for (int j = 0; j < 4; ++j) nat_split_lane<8, 4>(16u * c16 + 256u * (4u * g + j), base[j], xlo[j]);
-#pragma unroll
-            for (int r = 0; r < 2; ++r) {
-#pragma unroll
-                for (int tt = 0; tt < 8; ++tt)
-                    store4(wl + nat_split_word<8>(256u * (2u * tt + r) + 4u * lane), v[2 * tt + r]);
-                __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
-#pragma unroll
-                for (int t = 0; t < 16; ++t)
-#pragma unroll
-                    for (int j = r; j < 4; j += 2) d[t][j] = wl[base[j] + ((u32)t ^ xlo[j])];
-                __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
-            }
-        };
+        auto load = [&](u32 (&d)[16][4]) { nat_direct_load<16, 16>(d, [&](int) { return in + offs[0]; }, lane); };
         rows_body<16, false, SIGN>([&](int t) { return out + offs[0] + 256u * t + lane_off; }, 16u, 0u, w4096,
                                    EpiParams{}, load);
     } else {
-        if (lines <= 0) return;
-        u32* const wl = lds + (u32)wave * 2048u;  // 8 KiB per wave: NT * 256 words
         constexpr int NT = (T == 1 || T == 8) ? 8 : 4;  // as multi_rows
         for (int t0 = 0; t0 < lines * T; t0 += NT) {
             const u32 ntl = (u32)min(lines * T - t0, NT);
             auto load = [&](u32 (&d)[NT][4]) {
+                if constexpr (T > 1) {
+                    nat_direct_load<T, NT>(
+                        d, [&](int l) { return in + offs[t0 / T + (int)min((u32)l, ntl / T - 1u)]; }, lane);
+                } else {
+                    u32* const wl = lds + (u32)wave * 2048u;  // 8 KiB per wave: NT * 256 words
 #pragma unroll
-                for (int k = 0; k < NT / T; ++k)
-                    if ((u32)(k * T) < ntl) {
-                        const u32* src = in + offs[t0 / T + k] + 4u * lane;
-#pragma unroll
-                        for (int tt = 0; tt < T; ++tt) {
+                    for (int k = 0; k < NT; ++k)
+                        if ((u32)k < ntl) {
                             u32 v[4];
-                            load4_nt(v, src + 256u * tt);
-                            store4(wl + nat_lds_word((u32)k * L + 256u * tt + 4u * lane), v);
+                            load4_nt(v, in + offs[t0 + k] + 4u * lane);
+                            store4(wl + nat_lds_word((u32)k * L + 4u * lane), v);
                         }
-                    }
-                __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
-                nat_rows_read<T, NT>(d, wl, ntl, lane);
-                __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+                    __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+                    nat_rows_read<T, NT>(d, wl, ntl, lane);
+                    __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+                }
             };
             rows_body<T, false, SIGN, NT>(
                 [&](int t) { return out + offs[(t0 + t) / T] + 256u * ((t0 + t) % T) + lane_off; }, ntl, 0u, w4096,
@@ -2334,49 +2258,8 @@ __device__ __forceinline__ void multi_big_nat(const u32* in, u32* out, const Mul
     // signal, so that every load stays in bounds, and stores nothing
     const bool active = grp < (int)tk.count;
     const u32 off = offsets[tk.first + (active ? grp : 0)];
-    u32 v[16][4];
-    {
-        const u32* src = in + off + 4096u * (u32)w + 4u * lane;
-#pragma unroll
-        for (int t = 0; t < 16; ++t) load4_nt(v[t], src + 256u * t);
-    }
-    // Two rounds over every group at once: round r stages the natural
-    // indices n with bit B of n = r at word nat_split_word<B>(n) of the
-    // group's W * 2048 words.  B is chosen so that the writer's half is a
-    // set of its loaded tiles (n = 4096w + 256t + ...: tile bit B - 8) and,
-    // for W = 2, 4, 8, the reader's half a set of its registers (reader
-    // n = w + W*(t + 16*c16 + 256*(4g + j)): bit 9 = j & 1 for W = 2, bit
-    // 11 = j >> 1 for W = 4 and j & 1 for W = 8); for W = 16 bit 11 is
-    // c16 >> 3, a lane predicate.
-    constexpr int B = W == 2 ? 9 : 11;
-    constexpr int LW = W == 2 ? 5 : W == 4 ? 6 : W == 8 ? 7 : 8;  // log2(16W)
-    // reader word of (t, j): base_j + ((w + W t) ^ xlo_j) (nat_split_lane)
-    u32 base[4], xlo[4];
-#pragma unroll
-    for (int j = 0; j < 4; ++j)
-        nat_split_lane<B, LW>(16u * W * (u32)c16 + 256u * W * (4u * g + (u32)j), base[j], xlo[j]);
     u32 d[16][4];
-    u32* const region = lds + (u32)grp * (2048u * W);
-#pragma unroll
-    for (int r = 0; r < 2; ++r) {
-        if (r) __syncthreads();  // round 0's reads are done
-#pragma unroll
-        for (int t = 0; t < 16; ++t)
-            if (((t >> (B - 8)) & 1) == r)
-                store4(region + nat_split_word<B>(4096u * (u32)w + 256u * t + 4u * lane), v[t]);
-        __syncthreads();
-#pragma unroll
-        for (int t = 0; t < 16; ++t)
-#pragma unroll
-            for (int j = 0; j < 4; ++j) {
-                const u32 word = base[j] + (((u32)w + W * (u32)t) ^ xlo[j]);
-                if constexpr (W == 16) {
-                    if ((c16 >> 3) == r) d[t][j] = region[word];
-                } else {
-                    if ((W == 4 ? (j >> 1) : (j & 1)) == r) d[t][j] = region[word];
-                }
-            }
-    }
+    big_nat_load2<W>(d, in + off, W, (u32)w, lds + (u32)grp * (2048u * W), lane);
     __syncthreads();  // every wave has read its data before the exchange reuses the LDS
     BigTw bt;
     big_tw_load<W, false>(bt, lane_id(), w, 0u, w4096, tb.hi[M - 13], tb.lo[M - 13], (u32)(M / 2), EpiParams{});

@@ -505,8 +505,11 @@ bool valid(tcfft_plan p) { return p && p->magic == kMagic; }
 // delay 2 27.60 us, delay 3 27.43, 5 groups delay 1 27.46, 7 groups delay 1
 // 27.66, no stagger 28.13; natural order 5 groups delay 3 37.40 us, 7 groups
 // delay 2 37.11, 3 groups delay 2 38.59.
-tcfft::StartSched big_sched(const tcfft_plan_s* p, int W) {
-    const int delay = p->big_delay >= 0 ? p->big_delay : (W == 4 || W == 8 ? 1 : 2);
+// A grid of less than one wave per SIMD has nothing to stagger (natural order,
+// 8192 x 100: 8.9 us with the delay, 7.1 without; 16384 x 64 10.6 and 9.8).
+tcfft::StartSched big_sched(const tcfft_plan_s* p, int W, uint32_t lines) {
+    const bool small = (uint64_t)lines * (uint32_t)W < 4u * (uint64_t)p->cus;
+    const int delay = p->big_delay >= 0 ? p->big_delay : small ? 0 : (W == 4 || W == 8 ? 1 : 2);
     return tcfft::StartSched{(uint32_t)delay, (uint32_t)p->big_groups, 0u};
 }
 
@@ -517,8 +520,9 @@ tcfft::StartSched big_sched(const tcfft_plan_s* p, int W) {
 // delays 2, 3, 4, 5: 38.6-38.8, 38.2-38.4, 37.9-38.4, 37.1-37.4 us; 5 groups
 // with delay 2: 37.5-37.9, delay 3: 36.7-37.1; 7 groups with delay 2:
 // 36.8-37.0); for W = 2, 4, 8 the drop-in defaults stay within 2% of the best.
-tcfft::StartSched nat_big_sched(const tcfft_plan_s* p, int W) {
-    if (p->big_delay >= 0 || W != 16) return big_sched(p, W);
+tcfft::StartSched nat_big_sched(const tcfft_plan_s* p, int W, uint32_t lines) {
+    const tcfft::StartSched s = big_sched(p, W, lines);
+    if (p->big_delay >= 0 || W != 16 || s.delay == 0) return s;
     return tcfft::StartSched{3u, 5u, 0u};
 }
 
@@ -570,23 +574,33 @@ uint32_t rows_nt(const tcfft_plan_s* p, const Pass& ps) {
     return lo;
 }
 
-// The same for the natural-order pass of 4096-point lines (k_rows_nat<16>
-// or k_rows_half_nat), whose lines go through LDS whole before any compute:
-// four waves per line up to one line per CU, one wave from 4 to 8 lines
-// per CU, two otherwise.  Measured (out of place, random input; one / two
-// / four waves per line): 4096 x 256 7.96 / 5.76 / 5.33 us, 4096 x 1024
-// 10.3 / 8.0 / 8.8, 4096 x 1536 13.1 / 13.7 / -, 4096 x 2048 15.0 / 16.0
-// / 16.4, 4096 x 4096 30.2 / 27.1 / 29.2, 4096 x 16384 101 / 93 / -; 2D 4 x
-// 4096 x 256 22.5 / 20.4 / -, 8 x 4096 x 256 32.3 / 31.3 / -.
+// The same for the natural-order pass.  4096-point lines: four waves per line
+// up to two lines per CU, two above (out of place, random input; one / two /
+// four waves per line: 4096 x 256 6.7 / 5.4 / 5.0 us, 4096 x 512 7.5 / 6.2 /
+// 5.4, 4096 x 1024 8.4 / 7.8 / 8.2, 4096 x 2048 12.9 / 12.0 / 13.9, 4096 x
+// 4096 27.3 / 22.7 / 24.0, 4096 x 16384 95.6 / 90.7 / 107).  256-point lines:
+// 16 or 4, never 8 (256 x 16384 9.5 us with 4, 10.7 with 8; 256 x 65536 27.4
+// with 4, 26.9 with 16).  Else as rows_nt (1024 x 1024 5.8 / 4.7 / 4.6 us with
+// 16 / 8 / 4 tiles, 1024 x 4096 9.5 / 8.7 / 9.9, 1024 x 16384 26.1 / 25.9 /
+// 28.7).
 uint32_t rows_nt_nat(const tcfft_plan_s* p, const Pass& ps) {
+    if (ps.radix < 16) {
+        const uint32_t nt = rows_nt(p, ps);
+        return ps.radix == 1 && nt == 8u && !p->rows_tiles ? 4u : nt;
+    }
     if (p->rows_tiles > 0) return (uint32_t)p->rows_tiles;
-    const uint32_t lines = ps.n_tiles / 16u, cus = (uint32_t)p->cus;
-    if (lines <= cus) return 4u;
-    return lines > 4u * cus && lines <= 8u * cus ? 16u : 8u;
+    return ps.n_tiles / 16u <= 2u * (uint32_t)p->cus ? 4u : 8u;
 }
 
-// Start schedule of a contiguous-row first pass run with nt tiles per wave
-// (the natural-order kernel k_rows_nat always runs 16).
+// Waves per workgroup of the natural-order pass: as rows_wg, but four for 2D
+// rows that fill the chip, whose stores go to permuted lines (2D 1024 x 1024
+// x 8 29.4 us against 30.7 with one; 1D 1024 x 16384 26.7 against 26.1).
+uint32_t rows_wg_nat(const tcfft_plan_s* p, const Pass& ps) {
+    if (p->rows_waves > 0) return (uint32_t)p->rows_waves;
+    return p->lay.dims == 2 && (ps.n_tiles + 15u) / 16u >= 4u * (uint32_t)p->cus ? 4u : rows_wg(p, ps);
+}
+
+// Start schedule of a contiguous-row first pass run with nt tiles per wave.
 tcfft::StartSched rows_sched(const tcfft_plan_s* p, const Pass& ps, uint32_t nt) {
     const uint32_t waves = (ps.n_tiles + nt - 1u) / nt;  // at most one wave per SIMD: a delay of 1
     const int delay = p->big_delay >= 0 ? p->big_delay : (waves <= 4u * (uint32_t)p->cus ? 1 : 0);
@@ -651,7 +665,7 @@ int run_passes(tcfft_plan_s* p, uint32_t* buf, int sign, hipStream_t st, size_t 
             e = tcfft::launch_rows(ps.radix, buf, ps.n_tiles, sign, p->w4096, epi, sc, rows_wg(p, ps), rows_nt(p, ps),
                                    st);
         } else if (ps.kind == 2) {
-            tcfft::StartSched sc = big_sched(p, ps.radix);
+            tcfft::StartSched sc = big_sched(p, ps.radix, ps.n_tiles);
             sc.cached_out = cached_out(p, i, nsig);
             e = tcfft::launch_big(ps.radix, buf, ps.n_tiles, sign, p->w4096, ps.big_hi, ps.big_lo, ps.big_M_log2 / 2,
                                   epi, sc, st);
@@ -955,7 +969,7 @@ hipError_t launch_real(tcfft_plan_s* p, int sign, bool adjoint, const void* in, 
     const Pass& ps = p->lay.passes[0];
     if (ps.kind != 2 || ps.radix != (int)(half / 4096)) return hipErrorInvalidValue;
     return tcfft::launch_r2c_big(ps.radix, sign, adjoint, (const uint32_t*)in, (uint32_t*)out, batch, p->w4096, ps.big_hi,
-                                 ps.big_lo, ps.big_M_log2 / 2, p->w_real, big_sched(p, ps.radix), st);
+                                 ps.big_lo, ps.big_M_log2 / 2, p->w_real, big_sched(p, ps.radix, batch), st);
 }
 
 // n reals per signal to n/2 + 1 bins: the real-input transform or, with
@@ -1527,15 +1541,13 @@ int exec_natural_staged(tcfft_plan plan, const void* in, void* out, int directio
         return for_chunks(plan, [&](uint32_t s0, uint32_t ns) -> int {
             Pass fp = first;
             fp.n_tiles = (uint32_t)((uint64_t)first.n_tiles / B * ns);
-            // 4096-point lines: one or two waves per line (rows_nt_nat);
-            // shorter lines 16 tiles per wave
-            const uint32_t nt = fused_rows && fp.radix == 16 ? rows_nt_nat(plan, fp) : 16u;
-            tcfft::StartSched sc = fused_rows ? rows_sched(plan, fp, nt) : nat_big_sched(plan, fp.radix);
+            const uint32_t nt = fused_rows ? rows_nt_nat(plan, fp) : 16u;
+            tcfft::StartSched sc = fused_rows ? rows_sched(plan, fp, nt) : nat_big_sched(plan, fp.radix, fp.n_tiles);
             sc.cached_out = cached_out(plan, 0, ns);
             const uint32_t* ci = rsrc + per * s0;
             uint32_t* co = (uint32_t*)out + per * s0;
             hipError_t e = fused_rows ? tcfft::launch_rows_nat(fp.radix, ci, co, fp.n_tiles, direction, plan->w4096,
-                                                               nx_log2, plan->xpos, sc, nt, st)
+                                                               nx_log2, plan->xpos, sc, nt, rows_wg_nat(plan, fp), st)
                                       : tcfft::launch_big_nat(fp.radix, ci, co, fp.n_tiles, direction, plan->w4096,
                                                               fp.big_hi, fp.big_lo, fp.big_M_log2 / 2, nx_log2, x_pos,
                                                               sc, st);
