@@ -271,6 +271,23 @@ __device__ __forceinline__ void big_tw_load(BigTw& bt, int lane, int w, u32 sig,
     bt.s3 = wq_load(4096u * rj * (u32)c16);
 }
 
+// The phase-1 values of a single line with exponent e (twiddle W_Q^{c*e}) from
+// the two-level table of W_Q: what big_tw_load gives wave w of chunk j under
+// the epilogue for e = w*R + rev(j).
+__device__ __forceinline__ void line_tw_load(BigTw& bt, int lane, u32 e, const float2* __restrict__ w4096,
+                                             const float2* __restrict__ q_hi, const float2* __restrict__ q_lo,
+                                             u32 q_bits, u32 q_mask) {
+    const int c16 = lane & 15, g = lane >> 4;
+    auto wq_load = [&](u32 m) -> RawQ {
+        m &= q_mask;
+        return RawQ{q_hi[m >> q_bits], q_lo[m & ((1u << q_bits) - 1u)]};
+    };
+    dit4096_tw_load(bt.tw, lane, w4096);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) bt.rec0[i] = wq_load(e * (4u * g + i + 16u * c16));
+    bt.s2 = wq_load(256u * e * (u32)c16);
+}
+
 template <int SIGN>
 __device__ __forceinline__ cf raw_q(const RawQ& r) {
     constexpr float sg = SIGN < 0 ? 1.f : -1.f;

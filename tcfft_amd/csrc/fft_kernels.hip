@@ -1457,6 +1457,189 @@ __global__ __launch_bounds__(64 * W) TCFFT_MFMA_BUDGET void k_big_nat(
 }
 
 // ----------------------------------------------------------------------------
+// Natural-order lines of N = 65536*R points, R = 2, 4, 8, 16 (2^17..2^20), in
+// two passes without a reversal pass.  The drop-in plan of these sizes is
+// k_big<16> on R chunks of 65536 points and a radix-R pass; its arithmetic is
+// kept, bit for bit, but the passes are cut one stage earlier: with n = q +
+// 16R*rho (q = d4 + R*d3 the lowest digits) the natural signal is a matrix of
+// 4096 rows x 16R columns whose columns are the 4096-point lines of k_big's
+// phase 1, and columns can be read from natural order directly.
+//
+// k_lines_nat: a workgroup of 16 waves loads 16 adjacent columns (64-byte
+// pieces of every row, big_nat_load2), runs phase 1 on one column per wave
+// with the twiddle W_N^{q c} that k_big folds for chunk d4 and wave d3, and
+// stores line q as row q of an intermediate [16R][4096].  Workgroups are
+// mapped so that those on one XCD take adjacent column groups, whose pieces
+// share 128-byte lines.
+// Against the reversal pass + k_big + radix-R pass, per exec: 2^17 x 128 76.1 ->
+// 51.6 us, 2^18 x 64 77.2 -> 51.8, 2^19 x 32 77.9 -> 56.2, 2^20 x 16 77.8 ->
+// 60.4, 2^20 x 200 902 -> 735 (2^20: 33.9 us here, 27.4 in k_rows16r).
+template <int SIGN, bool CACHED>
+__global__ __launch_bounds__(1024) TCFFT_MFMA_BUDGET void k_lines_nat(const u32* __restrict__ in,
+                                                                    u32* __restrict__ out, u32 r_log2, u32 n_groups,
+                                                                    const float2* __restrict__ w4096, EpiParams epi,
+                                                                    StartSched sched) {
+    extern __shared__ u32 lds[];
+    start_delay(sched);
+    const int lane = lane_id();
+    const u32 w = (u32)__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+    u32 grp = blockIdx.x;
+    if ((n_groups & 7u) == 0u) grp = (blockIdx.x & 7u) * (n_groups >> 3) + (blockIdx.x >> 3);
+    const u32 q0 = (grp & ((1u << r_log2) - 1u)) * 16u;
+    const size_t sig = (size_t)(grp >> r_log2) << (16u + r_log2);
+    u32 d[16][4];
+    big_nat_load2<16>(d, in + sig + q0, 16u << r_log2, w, lds, lane);
+    BigTw bt;
+    line_tw_load(bt, lane_id(), q0 + w, w4096, epi.hi, epi.lo, epi.lo_bits, epi.m_mask);
+    const Dft16Op op = make_dft16(lane, SIGN);
+    u32 e[16][4];
+    big_phase1<SIGN>(d, e, bt, op);
+    // (g,i) = k0, tile = k2, lane%16 = k1: four adjacent c = k0 + 16*k1 + 256*k2
+    u32* const row = out + sig + (size_t)(q0 + w) * 4096u;
+    const u32 off = 4u * (16u * ((u32)lane & 15u) + 4u * ((u32)lane >> 4));
+#pragma unroll
+    for (int t = 0; t < 16; ++t) {
+        const u32x4 v = {e[t][0], e[t][1], e[t][2], e[t][3]};
+        if constexpr (CACHED)
+            st_at<u32x4>(row + 256 * t, off, v);
+        else
+            st_at_nt<u32x4>(row + 256 * t, off, v);
+    }
+}
+
+// k_rows16r<R>: the rest of those transforms, in place on the intermediate
+// rows q = d4 + R*d3 of 4096 columns c: k_big's phase 2 over d3 (radix 16, the
+// operand of chunk d4 with rows k3 scaled by W_N^{4096 d4 k3}), the rounding
+// that ends its pass, then radix R over d4 -> X[c + 4096*(k3 + 16*k4)].
+// Bound by memory (the intermediate is in the MALL while a batch chunk fits).
+// R = 2, 4: four adjacent columns per lane and 64 per wave, as k_cols_q.
+// R = 8, 16: 64 columns per workgroup of 4 waves through an LDS tile, as
+// k_cols_w; its word with bits 5-6 (R = 8) or 6-7 of the row, so that the four
+// lane groups' rows 4R apart fall on different banks.
+template <int R>
+__device__ __forceinline__ u32 rows16r_word(u32 r, u32 c) {
+    return 64u * r + (c ^ ((((r >> 2) ^ (r >> (R == 16 ? 6 : 5))) & 3u) << 4));
+}
+
+template <int R, int SIGN>
+__global__ __launch_bounds__(256) TCFFT_MFMA_BUDGET void k_rows16r(u32* __restrict__ buf, u32 n_waves, EpiParams epi) {
+    constexpr int RL = R == 2 ? 1 : R == 4 ? 2 : R == 8 ? 3 : 4;
+    const int lane = lane_id();
+    const int c16 = lane & 15, g = lane >> 4;
+    const u32 wib = (u32)__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+    // row scales W_N^{4096 d4 k3} (k3 = lane%16) first: a table entry each
+    // (the low table's index is 0)
+    RawQ s3[R];
+#pragma unroll
+    for (int t = 0; t < R; ++t) {
+        const u32 m = (4096u * (u32)t * (u32)c16) & epi.m_mask;
+        s3[t] = RawQ{epi.hi[m >> epi.lo_bits], epi.lo[m & ((1u << epi.lo_bits) - 1u)]};
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    if constexpr (R <= 4) {
+        const u32 wave = blockIdx.x * (blockDim.x >> 6) + wib;
+        if (wave >= n_waves) return;
+        u32* const base = buf + ((size_t)(wave >> 6) << (16 + RL)) + (wave & 63u) * 64u + 4u * (u32)c16;
+        u32 d[R][4][4];  // [d4][word i: d3 = 4g + i][column]
+#pragma unroll
+        for (int t = 0; t < R; ++t)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) load4(d[t][i], base + 4096u * ((u32)t + R * (4u * g + i)));
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int t = 0; t < R; ++t) {
+            const Dft16Op op3 = make_dft16_scaled(lane, SIGN, raw_q<SIGN>(s3[t]));
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                const u32 a[4] = {d[t][0][q], d[t][1][q], d[t][2][q], d[t][3][q]};
+                f32x4 re, im;
+                dft16_b(a, op3, re, im);
+#pragma unroll
+                for (int i = 0; i < 4; ++i) d[t][i][q] = pack(cf{re[i], im[i]});
+            }
+        }
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                cf v[R];
+#pragma unroll
+                for (int t = 0; t < R; ++t) v[t] = unpack(d[t][i][q]);
+                small_dft<R>(v, SIGN);
+#pragma unroll
+                for (int t = 0; t < R; ++t) d[t][i][q] = pack(v[t]);
+            }
+#pragma unroll
+        for (int t = 0; t < R; ++t)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) store4_nt(base + 4096u * (4u * g + i + 16u * t), d[t][i]);
+    } else {
+        extern __shared__ u32 lds[];
+        const u32 grp = blockIdx.x;
+        u32* const base = buf + ((size_t)(grp >> 6) << (16 + RL)) + (grp & 63u) * 64u;
+        const u32 rr = threadIdx.x >> 4, cq = threadIdx.x & 15u;
+        {
+            u32 v[R][4];
+#pragma unroll
+            for (int k = 0; k < R; ++k) load4(v[k], base + 4096u * (rr + 16u * k) + 4u * cq);
+#pragma unroll
+            for (int k = 0; k < R; ++k) store4(lds + rows16r_word<R>(rr + 16u * k, 4u * cq), v[k]);
+        }
+        __syncthreads();
+        u32 d[R][4];
+#pragma unroll
+        for (int t = 0; t < R; ++t)
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+                d[t][i] = lds[rows16r_word<R>((u32)t + R * (4u * g + i), 16u * wib + c16)];
+#pragma unroll
+        for (int t = 0; t < R; ++t) {
+            const Dft16Op op3 = make_dft16_scaled(lane, SIGN, raw_q<SIGN>(s3[t]));
+            f32x4 re, im;
+            dft16_b(d[t], op3, re, im);
+#pragma unroll
+            for (int i = 0; i < 4; ++i) d[t][i] = pack(cf{re[i], im[i]});
+        }
+        __syncthreads();  // every wave has read its columns
+        if constexpr (R == 16) {
+            u32 e[16][4];
+            transpose_gi_tile(d, e);  // (g,i) = d4, tile = k3
+            const Dft16Op op = make_dft16(lane, SIGN);
+#pragma unroll
+            for (int t = 0; t < 16; ++t) {
+                f32x4 re, im;
+                dft16_b(e[t], op, re, im);
+#pragma unroll
+                for (int i = 0; i < 4; ++i)
+                    lds[rows16r_word<R>((u32)t + 16u * (4u * g + i), 16u * wib + c16)] = pack(cf{re[i], im[i]});
+            }
+        } else {
+            // the sign as a run-time value, as in k_cols_small: with a constant
+            // the compiler contracts the products by (1 +- i)/sqrt(2) into
+            // other FMAs, and last bits differ
+            int sign = SIGN;
+            asm volatile("" : "+s"(sign));
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                cf v[R];
+#pragma unroll
+                for (int t = 0; t < R; ++t) v[t] = unpack(d[t][i]);
+                small_dft<R>(v, sign);
+#pragma unroll
+                for (int t = 0; t < R; ++t) lds[rows16r_word<R>(4u * g + i + 16u * t, 16u * wib + c16)] = pack(v[t]);
+            }
+        }
+        __syncthreads();
+#pragma unroll
+        for (int k = 0; k < R; ++k) {
+            u32 v[4];
+            load4(v, lds + rows16r_word<R>(rr + 16u * k, 4u * cq));
+            store4_nt(base + 4096u * (rr + 16u * k) + 4u * cq, v);
+        }
+    }
+}
+
+// ----------------------------------------------------------------------------
 // Real-input transforms above 65536 points: the L = N/2-point complex
 // transform runs as its own passes and k_pairs<SIGN> is the even/odd split by
 // itself, one lane per bin pair (k, L-k), k < L/2 (the lane with k = 0 also
@@ -1993,6 +2176,56 @@ hipError_t launch_big_nat(int W, const u32* in, u32* out, u32 n_signals, int sig
     case 32: return launch_big_nat_t<16, -1>(in, out, n_signals, w4096, wn_hi, wn_lo, lo_bits, nx_log2, x_pos, sched, st);
     case 33: return launch_big_nat_t<16, +1>(in, out, n_signals, w4096, wn_hi, wn_lo, lo_bits, nx_log2, x_pos, sched, st);
     default: return hipErrorInvalidValue;
+    }
+}
+
+template <int SIGN>
+static hipError_t launch_lines_nat_t(const u32* in, u32* out, u32 r_log2, u32 n_signals, const float2* w4096,
+                                     const EpiParams& epi, StartSched sched, hipStream_t st) {
+    const size_t lds = 32768u * sizeof(u32);
+    const u32 groups = n_signals << r_log2;
+    auto k = sched.cached_out ? k_lines_nat<SIGN, true> : k_lines_nat<SIGN, false>;
+    const KernelInfo ki = kernel_info(k, 1024, lds);
+    if (ki.lds_status != hipSuccess) return ki.lds_status;
+    if (sched.groups == 0) sched.delay = 0;
+    if (sched.delay) sched.resident = ki.resident;
+    hipLaunchKernelGGL(k, dim3(groups), dim3(1024), lds, st, in, out, r_log2, groups, w4096, epi, sched);
+    return hipGetLastError();
+}
+
+template <int R, int SIGN>
+static hipError_t launch_rows16r_t(u32* buf, u32 n_signals, const EpiParams& epi, hipStream_t st) {
+    auto k = k_rows16r<R, SIGN>;
+    const u32 groups = n_signals * 64u;  // of 64 columns
+    if constexpr (R <= 4) {
+        hipLaunchKernelGGL(k, dim3(groups / 4u), dim3(256), 0, st, buf, groups, epi);
+    } else {
+        const size_t lds = 16u * R * 64u * sizeof(u32);
+        const KernelInfo ki = kernel_info(k, 256, lds);
+        if (ki.lds_status != hipSuccess) return ki.lds_status;
+        hipLaunchKernelGGL(k, dim3(groups), dim3(256), lds, st, buf, groups, epi);
+    }
+    return hipGetLastError();
+}
+
+hipError_t launch_nat_two_pass(int R, const u32* in, u32* out, u32 n_signals, int sign, const float2* w4096,
+                               const EpiParams& epi, StartSched sched, hipStream_t st) {
+    // the folded epilogue of a 65536-point first pass: W_N, N = 65536*R
+    if (epi.shift != 0 || epi.s_log2 != 16 || (R != 2 && R != 4 && R != 8 && R != 16) || (1 << epi.r_log2) != R ||
+        epi.lo_bits > 12)
+        return hipErrorInvalidValue;
+    hipError_t e = sign < 0 ? launch_lines_nat_t<-1>(in, out, epi.r_log2, n_signals, w4096, epi, sched, st)
+                            : launch_lines_nat_t<+1>(in, out, epi.r_log2, n_signals, w4096, epi, sched, st);
+    if (e != hipSuccess) return e;
+    switch (R * 2 + (sign < 0 ? 0 : 1)) {
+    case 4: return launch_rows16r_t<2, -1>(out, n_signals, epi, st);
+    case 5: return launch_rows16r_t<2, +1>(out, n_signals, epi, st);
+    case 8: return launch_rows16r_t<4, -1>(out, n_signals, epi, st);
+    case 9: return launch_rows16r_t<4, +1>(out, n_signals, epi, st);
+    case 16: return launch_rows16r_t<8, -1>(out, n_signals, epi, st);
+    case 17: return launch_rows16r_t<8, +1>(out, n_signals, epi, st);
+    case 32: return launch_rows16r_t<16, -1>(out, n_signals, epi, st);
+    default: return launch_rows16r_t<16, +1>(out, n_signals, epi, st);
     }
 }
 

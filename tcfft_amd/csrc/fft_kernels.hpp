@@ -181,4 +181,10 @@ hipError_t launch_big_nat(int W, const uint32_t* in, uint32_t* out, uint32_t n_s
                           const float2* wn_hi, const float2* wn_lo, uint32_t lo_bits, uint32_t nx_log2,
                           const RevSpec& x_pos, StartSched sched, hipStream_t st);
 
+// Natural-order transform of N = 65536*R points (R = 2, 4, 8, 16), in -> out
+// out of place, bit-identical to launch_big<16> with the epilogue epi and a
+// radix-R pass on the reversed input; two passes, the intermediate in out.
+hipError_t launch_nat_two_pass(int R, const uint32_t* in, uint32_t* out, uint32_t n_signals, int sign,
+                               const float2* w4096, const EpiParams& epi, StartSched sched, hipStream_t st);
+
 }  // namespace tcfft

@@ -1567,6 +1567,20 @@ int exec_natural_staged(tcfft_plan plan, const void* in, void* out, int directio
         int rc = stage(src);
         if (rc) return rc;
     }
+    // 2^17..2^20 points: two passes that read natural order themselves
+    if (L.passes.size() == 2 && first.kind == 2 && first.radix == 16 && first.has_epi && L.passes[1].kind == 1 &&
+        L.passes[1].radix <= 16) {
+        return for_chunks(plan, [&](uint32_t s0, uint32_t ns) -> int {
+            const size_t off = (size_t)L.n * s0;
+            // no stagger by default: 2^20 x 16 66 us with the 65536-point
+            // kernel's schedule, 59 without, 2^17 x 128 59 and 53
+            tcfft::StartSched sc{plan->big_delay > 0 ? (uint32_t)plan->big_delay : 0u, (uint32_t)plan->big_groups, 0u};
+            sc.cached_out = cached_out(plan, 0, ns);
+            const hipError_t e = tcfft::launch_nat_two_pass(L.passes[1].radix, src + off, (uint32_t*)out + off, ns,
+                                                            direction, plan->w4096, first.epi, sc, st);
+            return e == hipSuccess ? TCFFT_SUCCESS : hip_fail(e);
+        });
+    }
     // per batch chunk (chunk_signals): the reversal, then the passes
     const tcfft::RevSpec spec = rev_spec(L.rad_y);
     return for_chunks(plan, [&](uint32_t s0, uint32_t ns) -> int {
