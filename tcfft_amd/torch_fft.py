@@ -86,6 +86,13 @@ def _check(x: torch.Tensor):
         raise RuntimeError("expected an fp16 tensor of shape [..., n, 2] (interleaved complex)")
 
 
+def _stream(device: torch.device) -> int:
+    """The current HIP stream's handle.  The raw getter takes 0.1 us where
+    torch.cuda.current_stream(device).cuda_stream builds a Stream object in
+    2.0, a fifth of a short call (fft of 8 x 1024: 10.2 us of host time)."""
+    return torch._C._cuda_getCurrentRawStream(device.index)
+
+
 def _exec(x: torch.Tensor, direction: int) -> torch.Tensor:
     _check(x)
     x = x.contiguous()
@@ -93,7 +100,7 @@ def _exec(x: torch.Tensor, direction: int) -> torch.Tensor:
     batch = x.numel() // (2 * n)
     out = torch.empty_like(x)
     plan = _plan(n, batch, x.device)
-    stream = torch.cuda.current_stream(x.device).cuda_stream
+    stream = _stream(x.device)
     plan.exec_natural(x.data_ptr(), out.data_ptr(), direction, stream)
     return out
 
@@ -160,7 +167,7 @@ def _exec_split(x: torch.Tensor, direction: int) -> torch.Tensor:
     batch = v.numel() // (2 * n)
     out = torch.empty_like(v)
     _splan(n, batch, v.device).exec_split(v.data_ptr(), out.data_ptr(), direction,
-                                          torch.cuda.current_stream(v.device).cuda_stream)
+                                          _stream(v.device))
     return torch.view_as_complex(out) if cplx else out
 
 
@@ -215,7 +222,7 @@ def _r2c(x: torch.Tensor, adjoint: bool = False) -> torch.Tensor:
     out = torch.empty(x.shape[:-1] + (n // 2 + 1, 2), dtype=torch.float16, device=x.device)
     plan = _rplan(n, batch, x.device)
     call = plan.exec_c2r_adjoint if adjoint else plan.exec_r2c
-    call(x.data_ptr(), out.data_ptr(), torch.cuda.current_stream(x.device).cuda_stream)
+    call(x.data_ptr(), out.data_ptr(), _stream(x.device))
     return out
 
 
@@ -230,7 +237,7 @@ def _c2r(X: torch.Tensor, n: int, adjoint: bool = False) -> torch.Tensor:
     out = torch.empty(X.shape[:-2] + (n,), dtype=torch.float16, device=X.device)
     plan = _rplan(n, batch, X.device)
     call = plan.exec_r2c_adjoint if adjoint else plan.exec_c2r
-    call(X.data_ptr(), out.data_ptr(), torch.cuda.current_stream(X.device).cuda_stream)
+    call(X.data_ptr(), out.data_ptr(), _stream(X.device))
     return out
 
 
@@ -312,7 +319,7 @@ class _FusedConv(torch.autograd.Function):
         n, C = x.shape[-2], weight.shape[0]
         signals = x.numel() // (2 * n)
         plan = _plan(n, signals, x.device)
-        stream = torch.cuda.current_stream(x.device).cuda_stream
+        stream = _stream(x.device)
         # the filter into the digit-reversed order on the device (LDS-tiled,
         # copy speed; a torch gather reads 16x the bytes for this permutation)
         h16 = weight.detach().half().contiguous()
@@ -334,7 +341,7 @@ class _FusedConv(torch.autograd.Function):
         n, C, signals, want_h = ctx.shape
         gy = gy.to(torch.float16).contiguous()
         plan = _plan(n, signals, gy.device)
-        stream = torch.cuda.current_stream(gy.device).cuda_stream
+        stream = _stream(gy.device)
         gx = torch.empty_like(gy)
         gspec = torch.empty_like(gy) if want_h else None
         plan.conv_exec(C, gy.data_ptr(), h_rev.data_ptr(), gx.data_ptr(), True,
