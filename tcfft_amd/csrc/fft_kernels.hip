@@ -2506,11 +2506,11 @@ template <int SIGN>
 __global__ __launch_bounds__(1024) void k_multi_nat(const u32* in, u32* out, const MultiTask* __restrict__ tasks,
                                                     u32 n_tasks, const u32* __restrict__ offsets,
                                                     const float2* __restrict__ w4096, MultiTables tb,
-                                                    StartSched sched) {
+                                                    u32 reverse, StartSched sched) {
     extern __shared__ u32 lds[];
     start_delay(sched);
     for (u32 ti = blockIdx.x; ti < n_tasks; ti += gridDim.x) {
-        const MultiTask tk = tasks[ti];
+        const MultiTask tk = tasks[reverse ? n_tasks - 1u - ti : ti];
         switch (tk.size_log2) {
         case 8: multi_rows_nat<1, SIGN>(in, out, tk, offsets, w4096, lds); break;
         case 9: multi_rows_nat<2, SIGN>(in, out, tk, offsets, w4096, lds); break;
@@ -2530,24 +2530,25 @@ __global__ __launch_bounds__(1024) void k_multi_nat(const u32* in, u32* out, con
 template <int SIGN>
 static hipError_t launch_multi_nat_t(const u32* in, u32* out, const MultiTask* tasks, u32 n_tasks,
                                      const u32* offsets, u32 grid, const float2* w4096, const MultiTables& tb,
-                                     StartSched sched, hipStream_t st) {
+                                     bool reverse, StartSched sched, hipStream_t st) {
     constexpr size_t lds = 16 * 2048 * sizeof(u32);  // 128 KiB
     auto k = k_multi_nat<SIGN>;
     const KernelInfo ki = kernel_info(k, 1024, lds);
     if (ki.lds_status != hipSuccess) return ki.lds_status;
     if (sched.groups == 0) sched.delay = 0;
     if (sched.delay) sched.resident = ki.resident;
-    hipLaunchKernelGGL(k, dim3(grid), dim3(1024), lds, st, in, out, tasks, n_tasks, offsets, w4096, tb, sched);
+    hipLaunchKernelGGL(k, dim3(grid), dim3(1024), lds, st, in, out, tasks, n_tasks, offsets, w4096, tb,
+                       reverse ? 1u : 0u, sched);
     return hipGetLastError();
 }
 
 hipError_t launch_multi_nat(const u32* in, u32* out, const MultiTask* tasks, u32 n_tasks, const u32* offsets,
-                            u32 grid, int sign, const float2* w4096, const MultiTables& tb, StartSched sched,
-                            hipStream_t st) {
+                            u32 grid, int sign, const float2* w4096, const MultiTables& tb, bool reverse,
+                            StartSched sched, hipStream_t st) {
     if (n_tasks == 0) return hipSuccess;
     if (grid == 0 || grid > n_tasks) grid = n_tasks;
-    return sign < 0 ? launch_multi_nat_t<-1>(in, out, tasks, n_tasks, offsets, grid, w4096, tb, sched, st)
-                    : launch_multi_nat_t<+1>(in, out, tasks, n_tasks, offsets, grid, w4096, tb, sched, st);
+    return sign < 0 ? launch_multi_nat_t<-1>(in, out, tasks, n_tasks, offsets, grid, w4096, tb, reverse, sched, st)
+                    : launch_multi_nat_t<+1>(in, out, tasks, n_tasks, offsets, grid, w4096, tb, reverse, sched, st);
 }
 
 template <int SIGN>

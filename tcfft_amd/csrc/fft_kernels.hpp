@@ -104,10 +104,11 @@ struct MultiTables {  // two-level W_N tables for N = 2^13 .. 2^16
 hipError_t launch_multi(uint32_t* buf, const MultiTask* tasks, uint32_t n_tasks, const uint32_t* offsets,
                         uint32_t grid, int sign, const float2* w4096, const MultiTables& tb, StartSched sched,
                         hipStream_t st);
-// The same tasks on natural-order input: in -> out (in == out allowed).
+// The same tasks on natural-order input: in -> out (in == out allowed);
+// reverse: from the end of the list.
 hipError_t launch_multi_nat(const uint32_t* in, uint32_t* out, const MultiTask* tasks, uint32_t n_tasks,
                             const uint32_t* offsets, uint32_t grid, int sign, const float2* w4096,
-                            const MultiTables& tb, StartSched sched, hipStream_t st);
+                            const MultiTables& tb, bool reverse, StartSched sched, hipStream_t st);
 
 // Natural-order transform of N = 4096*W (W = 1, 2, 4) per signal whose output
 // is the spectrum in the digit-reversed order the DIT kernels consume.
