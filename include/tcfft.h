@@ -226,6 +226,10 @@ int tcfft_conv_exec(tcfft_plan plan, int channels, const void *x, const void *h_
  * digit-reversed.  No reference counterpart. */
 int tcfft_conv_filter_grad(tcfft_plan plan, int channels, const void *x_spec, const void *g_spec, void *gh_rev,
                            void *stream);
+/* The same with the gradient in natural spectrum order: gh[c][rev[p]] as
+ * gh_rev[c][p] above.  Plans of n = 4096, 8192 or 16384. */
+int tcfft_conv_filter_grad_natural(tcfft_plan plan, int channels, const void *x_spec, const void *g_spec, void *gh,
+                                   void *stream);
 
 /* Plan options. TCFFT_OPT_SPLIT_CHUNK: signals per pass pair of
  * tcfft_exec_split (0 = whole batch, the default), which bounds the

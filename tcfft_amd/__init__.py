@@ -46,7 +46,7 @@ EXPORTS = (
     "tcfft_plan_create_1d_split", "tcfft_plan_create_1d_tuned", "tcfft_query_1d_split",
     "tcfft_plan_create_r2c_1d", "tcfft_exec_r2c", "tcfft_exec_c2r", "tcfft_permute_to_dropin",
     "tcfft_exec_natural_noalloc", "tcfft_multi_exec_natural", "tcfft_plan_prepare_split", "tcfft_query_split",
-    "tcfft_exec_r2c_adjoint", "tcfft_exec_c2r_adjoint",
+    "tcfft_exec_r2c_adjoint", "tcfft_exec_c2r_adjoint", "tcfft_conv_filter_grad_natural",
 )
 NOALLOC_SCRATCH_BYTES = 64 << 20  # TCFFT_NOALLOC_SCRATCH_BYTES
 OPT_SPLIT_CHUNK = 1
@@ -117,6 +117,7 @@ def lib():
         L.tcfft_exec_dif.argtypes = [_vp, _vp, _vp, ctypes.c_int, _vp]
         L.tcfft_conv_exec.argtypes = [_vp, ctypes.c_int, _vp, _vp, _vp, ctypes.c_int, _vp, _vp]
         L.tcfft_conv_filter_grad.argtypes = [_vp, ctypes.c_int, _vp, _vp, _vp, _vp]
+        L.tcfft_conv_filter_grad_natural.argtypes = [_vp, ctypes.c_int, _vp, _vp, _vp, _vp]
         L.tcfft_multi_create.argtypes = [ctypes.POINTER(_vp), ctypes.c_int, _i32p]
         L.tcfft_multi_destroy.argtypes = [_vp]
         L.tcfft_multi_info.argtypes = [_vp, _i32p, ctypes.POINTER(ctypes.c_longlong)]
@@ -264,6 +265,12 @@ class _Plan:
         """gh_rev[c] = (1/n) sum_b conj(X[b, c]) * G[b, c] (FP32, digit-reversed)."""
         _check(lib().tcfft_conv_filter_grad(self._h, channels, _vp(x_spec_ptr), _vp(g_spec_ptr), _vp(gh_rev_ptr),
                                             _vp(stream)), "tcfft_conv_filter_grad")
+
+    def conv_filter_grad_natural(self, channels: int, x_spec_ptr: int, g_spec_ptr: int, gh_ptr: int, stream: int = 0):
+        """conv_filter_grad with the gradient in natural spectrum order (n =
+        4096, 8192, 16384)."""
+        _check(lib().tcfft_conv_filter_grad_natural(self._h, channels, _vp(x_spec_ptr), _vp(g_spec_ptr), _vp(gh_ptr),
+                                                    _vp(stream)), "tcfft_conv_filter_grad_natural")
 
     def set_option(self, option: int, value: int):
         _check(lib().tcfft_plan_set_option(self._h, option, value), "tcfft_plan_set_option")

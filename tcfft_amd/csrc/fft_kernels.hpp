@@ -123,6 +123,9 @@ hipError_t launch_conv(int W, bool conj, const uint32_t* x, const uint32_t* h_re
 // gh_rev[c][p] = scale * sum_b conj(X[b][c][p]) G[b][c][p] (FP32 out).
 hipError_t launch_conv_wgrad(const uint32_t* xs, const uint32_t* gs, float2* gh, uint32_t n, uint32_t channels,
                              uint32_t batch, float scale, hipStream_t st);
+// The same for n = 4096*W (W = 1, 2, 4) with gh in natural spectrum order.
+hipError_t launch_conv_wgrad_nat(int W, const uint32_t* xs, const uint32_t* gs, float2* gh, uint32_t channels,
+                                 uint32_t batch, float scale, uint32_t cus, hipStream_t st);
 
 // Strided pass of radix R (2..256) at element step 2^s_log2 over `outer` blocks.
 hipError_t launch_cols(int R, uint32_t* buf, uint32_t s_log2, uint32_t outer, int sign, const float2* w4096,

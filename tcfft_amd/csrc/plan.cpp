@@ -1296,6 +1296,25 @@ int tcfft_conv_filter_grad(tcfft_plan plan, int channels, const void* x_spec, co
     return TCFFT_SUCCESS;
 }
 
+int tcfft_conv_filter_grad_natural(tcfft_plan plan, int channels, const void* x_spec, const void* g_spec, void* gh,
+                                   void* stream) {
+    if (!valid(plan)) return TCFFT_INVALID_PLAN;
+    if (!aligned16(x_spec) || !aligned16(g_spec) || !aligned16(gh)) return TCFFT_INVALID_POINTER;
+    int W = 0;
+    const float2 *hi = nullptr, *lo = nullptr;
+    uint32_t bits = 0;
+    int rc = dif_params(plan, W, hi, lo, bits);
+    if (rc) return rc;
+    const Layout& L = plan->lay;
+    if (channels < 1 || L.batch % channels) return TCFFT_INVALID_BATCH;
+    DeviceGuard guard(plan->device);
+    hipError_t e = tcfft::launch_conv_wgrad_nat(W, (const uint32_t*)x_spec, (const uint32_t*)g_spec, (float2*)gh,
+                                                (uint32_t)channels, (uint32_t)(L.batch / channels),
+                                                1.0f / (float)L.n, (uint32_t)plan->cus, (hipStream_t)stream);
+    if (e != hipSuccess) return hip_fail(e);
+    return TCFFT_SUCCESS;
+}
+
 int tcfft_plan_set_option(tcfft_plan plan, int option, int value) {
     if (!valid(plan)) return TCFFT_INVALID_PLAN;
     switch (option) {

@@ -44,7 +44,7 @@ from collections import OrderedDict
 
 import torch
 
-from . import FORWARD, INVERSE, Plan1D, PlanR2C, gen_rev
+from . import FORWARD, INVERSE, Plan1D, PlanR2C
 
 # Plans are cached per (n, batch, device), least recently used first out:
 # a plan holds device tables (and, for some layouts, a workspace as large as
@@ -287,19 +287,6 @@ def complex_mul(a: torch.Tensor, h: torch.Tensor) -> torch.Tensor:
 
 
 FUSED_N = (4096, 8192, 16384)
-_REV: dict = {}
-
-
-def _rev(n: int, device: torch.device):
-    """(rev, inverse rev) index tensors of the digit-reversed spectrum order."""
-    key = (n, device.index)
-    r = _REV.get(key)
-    if r is None:
-        plan = _plan(n, 1, device)
-        rev = torch.as_tensor(gen_rev(n, plan.radices).astype("int64"), device=device)
-        r = (rev, torch.argsort(rev))
-        _REV[key] = r
-    return r
 
 
 class _FusedConv(torch.autograd.Function):
@@ -348,9 +335,8 @@ class _FusedConv(torch.autograd.Function):
                        gspec.data_ptr() if gspec is not None else 0, stream)
         gw = None
         if want_h:
-            gh_rev = torch.empty(C, n, 2, dtype=torch.float32, device=gy.device)
-            plan.conv_filter_grad(C, spec.data_ptr(), gspec.data_ptr(), gh_rev.data_ptr(), stream)
-            gw = gh_rev.index_select(1, _rev(n, gy.device)[1])
+            gw = torch.empty(C, n, 2, dtype=torch.float32, device=gy.device)
+            plan.conv_filter_grad_natural(C, spec.data_ptr(), gspec.data_ptr(), gw.data_ptr(), stream)
         return gx, gw, None
 
 
