@@ -95,16 +95,22 @@ __host__ __device__ constexpr float sin_of(int k, int n) {
 
 // The FP16 hi/lo operands of this lane's four points (re[j], im[j]) * s:
 // hi = fp16(x*s), lo = fp16(x*s - hi) (the difference is exact in FP32);
-// without SCALE, s = 1.
+// without SCALE, s = 1.  The difference is written as hi*(-1) + x with a
+// factor the compiler does not see, so that it becomes one v_fma_mix_f32 that
+// reads the packed half where it stands (exact either way).  For the scaled
+// stage the compiler finds that by itself; with it here too a pass has 5% fewer
+// VALU instructions: 3000 x 4096 46.2 -> 45.6 us, 2D 1024 x 1024 x 8 55.3 -> 54.7.
 template <bool SCALE>
 __device__ __forceinline__ void split_operand(const float* re, const float* im, float s, f16x8& h, f16x8& l) {
     u32 hi[4], lo[4];
+    float minus_one;
+    asm("s_mov_b32 %0, -1.0" : "=s"(minus_one));
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
         const float xr = SCALE ? re[j] * s : re[j], xi = SCALE ? im[j] * s : im[j];
         hi[j] = pack(xr, xi);
         const cf v = unpack(hi[j]);
-        lo[j] = pack(xr - v.x, xi - v.y);
+        lo[j] = pack(__builtin_fmaf(v.x, minus_one, xr), __builtin_fmaf(v.y, minus_one, xi));
     }
     h = as_operand(hi[0], hi[1], hi[2], hi[3]);
     l = as_operand(lo[0], lo[1], lo[2], lo[3]);
