@@ -197,10 +197,11 @@ __device__ __forceinline__ void stepa_exchange(u32 (&v)[16][4], int w, int lane,
                 lds[zp] = hadd2(v[s * W][q], v[s * W + 1][q]);
                 lds[4096u + zp] = hsub2(v[s * W][q], v[s * W + 1][q]);
             } else {
-                cf x[W];
+                u32 xw[W];
 #pragma unroll
-                for (int n2 = 0; n2 < W; ++n2) x[n2] = unpack(v[s * W + n2][q]);
-                if constexpr (W > 1) small_dft<W>(x, SIGN);
+                for (int n2 = 0; n2 < W; ++n2) xw[n2] = v[s * W + n2][q];
+                cf x[W];
+                small_dft_words<W>(xw, x, SIGN);
 #pragma unroll
                 for (int k = 0; k < W; ++k) lds[4096u * k + zp] = pack(x[k]);
             }

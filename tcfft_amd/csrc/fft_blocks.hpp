@@ -401,10 +401,11 @@ __device__ __forceinline__ void big_phase2(u32 (&e)[16][4], int w, u32* lds, u32
                         o[0][j] = hadd2(v[0][j], v[1][j]);
                         o[1][j] = hsub2(v[0][j], v[1][j]);
                     } else {
-                        cf x[W];
+                        u32 xw[W];
 #pragma unroll
-                        for (int s = 0; s < W; ++s) x[s] = unpack(v[s][j]);
-                        small_dft<W>(x, sign);
+                        for (int s = 0; s < W; ++s) xw[s] = v[s][j];
+                        cf x[W];
+                        small_dft_words<W>(xw, x, sign);
 #pragma unroll
                         for (int s = 0; s < W; ++s)
                             o[s][j] = SCALE ? pack(x[s].x * scale, x[s].y * scale) : pack(x[s]);
@@ -454,10 +455,11 @@ __device__ __forceinline__ void big_phase2_regs(u32 (&e)[16][4], int w, u32* lds
                 load4(v[s], lds + (u32)s * C::COLS + lds_sigma(4u * lane + 256u * (q + QN * w)));
 #pragma unroll
             for (int j = 0; j < 4; ++j) {
-                cf x[W];
+                u32 xw[W];
 #pragma unroll
-                for (int s = 0; s < W; ++s) x[s] = unpack(v[s][j]);
-                small_dft<W>(x, SIGN);
+                for (int s = 0; s < W; ++s) xw[s] = v[s][j];
+                cf x[W];
+                small_dft_words<W>(xw, x, SIGN);
 #pragma unroll
                 for (int s = 0; s < W; ++s) o[(r * QN + q) * W + s][j] = pack(x[s]);
             }

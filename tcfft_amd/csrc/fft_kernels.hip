@@ -603,6 +603,16 @@ __global__ __launch_bounds__(256) TCFFT_MFMA_BUDGET void k_rows_half_nat(const u
 // times the transform: 4099 signals of 8192 reals, forward and backward,
 // 169.5 -> 95.4 us).
 
+// S and D of the words a = Z[k] and b = Z[L-k].  Their scales 1/2 (and those of
+// ADJ) are powers of two and ride on the last additions, exactly.
+struct RealPair {
+    cf sum, dif;
+};
+__device__ __forceinline__ RealPair real_pair(u32 a, u32 b) {
+    const cf s = hsum(a, b), d = hdif(a, b);
+    return {cf{s.x, d.y}, cf{d.x, s.y}};
+}
+
 // k_r2c<T>: the k_rows_nat pass with its output kept in the wave's LDS slice
 // (natural order, same swizzle), then the pairwise untangle in FP32.  The
 // bins go out with ordinary (cached) 4-byte stores: rows start at any 4-byte
@@ -640,14 +650,12 @@ __global__ __launch_bounds__(256) TCFFT_MFMA_BUDGET void k_r2c(const u32* __rest
 #pragma unroll
         for (u32 j = 0; j < L / 128u; ++j) {
             const u32 k = 64u * j + (u32)lane;  // < L/2
-            const cf a = unpack(wl[nat_lds_word(i * L + k)]);
-            const cf b = unpack(wl[nat_lds_word(i * L + ((L - k) & (L - 1u)))]);
-            cf hs = {hf * (a.x + b.x), hf * (a.y - b.y)};  // S/2
-            const cf dif = {a.x - b.x, a.y + b.y};         // D
-            cf q = cmul(w, dif);                           // W D / 2;  P = i q
-            if (ADJ && j == 0 && lane == 0) hs = {0.5f * hs.x, 0.5f * hs.y}, q = {0.5f * q.x, 0.5f * q.y};
-            dst[k] = pack(hs.x + q.y, hs.y - q.x);              // S/2 - P
-            dst[L - k] = pack(hs.x - q.y, -(hs.y + q.x));       // conj(S/2 + P)
+            const RealPair p = real_pair(wl[nat_lds_word(i * L + k)], wl[nat_lds_word(i * L + ((L - k) & (L - 1u)))]);
+            cf q = cmul(w, p.dif);  // W D / 2;  P = i q
+            float f = hf;
+            if (ADJ && j == 0 && lane == 0) f = 0.5f, q = {0.5f * q.x, 0.5f * q.y};
+            dst[k] = pack(__builtin_fmaf(f, p.sum.x, q.y), __builtin_fmaf(f, p.sum.y, -q.x));      // S/2 - P
+            dst[L - k] = pack(__builtin_fmaf(f, p.sum.x, -q.y), -__builtin_fmaf(f, p.sum.y, q.x));  // conj(S/2 + P)
             w = cmul(w, step);
         }
         if (lane == 0) {
@@ -695,17 +703,16 @@ __global__ __launch_bounds__(256) TCFFT_MFMA_BUDGET void k_c2r(const u32* __rest
 #pragma unroll
             for (u32 j = 0; j < L / 128u; ++j) {
                 const u32 k = 64u * j + (u32)lane;  // < L/2
-                cf a = unpack(va[j]), b = unpack(vb[j]);
-                if (j == 0 && lane == 0) a.y = b.y = 0.f;  // bins 0 and L: real parts only
-                cf sum = {a.x + b.x, a.y - b.y};           // S
-                const cf dif = {a.x - b.x, a.y + b.y};     // D
-                cf q = cmul(w, dif);                       // P = i q
-                if constexpr (ADJ) {
-                    if (j == 0 && lane == 0) q = {2.f * q.x, 2.f * q.y};
-                    else sum = {0.5f * sum.x, 0.5f * sum.y};
-                }
-                wl[nat_chunk_word<T>(i * L + k)] = pack(sum.x - q.y, sum.y + q.x);                  // S + P
-                if (k != 0) wl[nat_chunk_word<T>(i * L + (L - k))] = pack(sum.x + q.y, q.x - sum.y);  // conj(S - P)
+                if (j == 0 && lane == 0) va[j] &= 0xffffu, vb[j] &= 0xffffu;  // bins 0 and L: real parts only
+                const RealPair p = real_pair(va[j], vb[j]);
+                cf q = cmul(w, p.dif);  // P = i q
+                float f = hf;
+                if (ADJ && j == 0 && lane == 0) f = 1.f, q = {2.f * q.x, 2.f * q.y};
+                wl[nat_chunk_word<T>(i * L + k)] =
+                    pack(__builtin_fmaf(f, p.sum.x, -q.y), __builtin_fmaf(f, p.sum.y, q.x));  // S + P
+                if (k != 0)
+                    wl[nat_chunk_word<T>(i * L + (L - k))] =
+                        pack(__builtin_fmaf(f, p.sum.x, q.y), __builtin_fmaf(-f, p.sum.y, q.x));  // conj(S - P)
                 w = cmul(w, step);
             }
             if (lane == 0) {
@@ -1192,9 +1199,10 @@ __global__ __launch_bounds__(64 * W) TCFFT_MFMA_BUDGET void k_cols_big(u32* __re
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
                 cf x[W];
+                u32 xw[W];
 #pragma unroll
-                for (int src = 0; src < W; ++src) x[src] = unpack(v[src][i]);
-                small_dft<W>(x, SIGN);
+                for (int src = 0; src < W; ++src) xw[src] = v[src][i];
+                small_dft_words<W>(xw, x, SIGN);
                 // row k0 + 16 (4g + i) + 256 k2: the 64 g part is the lane's
 #pragma unroll
                 for (int k2 = 0; k2 < W; ++k2) {
@@ -1327,9 +1335,10 @@ __global__ __launch_bounds__(128 * W) TCFFT_MFMA_BUDGET void k_cols_bigw(u32* __
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
             cf x[W];
+            u32 xw[W];
 #pragma unroll
-            for (int src = 0; src < W; ++src) x[src] = unpack(v[src][i]);
-            small_dft<W>(x, SIGN);
+            for (int src = 0; src < W; ++src) xw[src] = v[src][i];
+            small_dft_words<W>(xw, x, SIGN);
 #pragma unroll
             for (int k2 = 0; k2 < W; ++k2) o[ti][i][k2] = pack(x[k2]);
         }
@@ -1381,9 +1390,10 @@ __global__ __launch_bounds__(256) void k_cols_small(u32* __restrict__ buf, u32 s
 #pragma unroll
     for (int q = 0; q < 4; ++q) {
         cf v[R];
+        u32 xw[R];
 #pragma unroll
-        for (int j = 0; j < R; ++j) v[j] = unpack(w[j][q]);
-        small_dft<R>(v, sign);
+        for (int j = 0; j < R; ++j) xw[j] = w[j][q];
+        small_dft_words<R>(xw, v, sign);
 #pragma unroll
         for (int j = 0; j < R; ++j) {
             cf o = v[j];
@@ -1563,9 +1573,10 @@ __global__ __launch_bounds__(256) TCFFT_MFMA_BUDGET void k_rows16r(u32* __restri
 #pragma unroll
             for (int q = 0; q < 4; ++q) {
                 cf v[R];
+                u32 xw[R];
 #pragma unroll
-                for (int t = 0; t < R; ++t) v[t] = unpack(d[t][i][q]);
-                small_dft<R>(v, SIGN);
+                for (int t = 0; t < R; ++t) xw[t] = d[t][i][q];
+                small_dft_words<R>(xw, v, SIGN);
 #pragma unroll
                 for (int t = 0; t < R; ++t) d[t][i][q] = pack(v[t]);
             }
@@ -1622,9 +1633,10 @@ __global__ __launch_bounds__(256) TCFFT_MFMA_BUDGET void k_rows16r(u32* __restri
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
                 cf v[R];
+                u32 xw[R];
 #pragma unroll
-                for (int t = 0; t < R; ++t) v[t] = unpack(d[t][i]);
-                small_dft<R>(v, sign);
+                for (int t = 0; t < R; ++t) xw[t] = d[t][i];
+                small_dft_words<R>(xw, v, sign);
 #pragma unroll
                 for (int t = 0; t < R; ++t) lds[rows16r_word<R>(4u * g + i + 16u * t, 16u * wib + c16)] = pack(v[t]);
             }
@@ -1742,14 +1754,12 @@ __global__ __launch_bounds__(64 * W) TCFFT_MFMA_BUDGET void k_r2c_big(
 #pragma unroll 8
     for (u32 j = 0; j < 32u; ++j) {
         const u32 k = 64u * (j * W + w) + (u32)lane;  // < L/2
-        const cf a = unpack(lds[k]);
-        const cf b = unpack(lds[(L - k) & (L - 1u)]);
-        cf hs = {hf * (a.x + b.x), hf * (a.y - b.y)};
-        const cf dif = {a.x - b.x, a.y + b.y};
-        cf q = cmul(tw, dif);
-        if (ADJ && k == 0) hs = {0.5f * hs.x, 0.5f * hs.y}, q = {0.5f * q.x, 0.5f * q.y};
-        dst[k] = pack(hs.x + q.y, hs.y - q.x);
-        dst[L - k] = pack(hs.x - q.y, -(hs.y + q.x));
+        const RealPair p = real_pair(lds[k], lds[(L - k) & (L - 1u)]);
+        cf q = cmul(tw, p.dif);
+        float f = hf;
+        if (ADJ && k == 0) f = 0.5f, q = {0.5f * q.x, 0.5f * q.y};
+        dst[k] = pack(__builtin_fmaf(f, p.sum.x, q.y), __builtin_fmaf(f, p.sum.y, -q.x));
+        dst[L - k] = pack(__builtin_fmaf(f, p.sum.x, -q.y), -__builtin_fmaf(f, p.sum.y, q.x));
         tw = cmul(tw, step);
     }
     if (w == 0 && lane == 0) {
@@ -1792,17 +1802,15 @@ __global__ __launch_bounds__(64 * W) TCFFT_MFMA_BUDGET void k_c2r_big(
 #pragma unroll
         for (u32 j = 0; j < 32u; ++j) {
             const u32 k = 64u * (j * W + w) + (u32)lane;
-            cf a = unpack(va[j]), b = unpack(vb[j]);
-            if (k == 0) a.y = b.y = 0.f;  // bins 0 and L: real parts only
-            cf sum = {a.x + b.x, a.y - b.y};
-            const cf dif = {a.x - b.x, a.y + b.y};
-            cf q = cmul(tw, dif);
-            if constexpr (ADJ) {
-                if (k == 0) q = {2.f * q.x, 2.f * q.y};
-                else sum = {0.5f * sum.x, 0.5f * sum.y};
-            }
-            lds[nat_big_word<W>(k)] = pack(sum.x - q.y, sum.y + q.x);
-            if (k != 0) lds[nat_big_word<W>(L - k)] = pack(sum.x + q.y, q.x - sum.y);
+            if (k == 0) va[j] &= 0xffffu, vb[j] &= 0xffffu;  // bins 0 and L: real parts only
+            const RealPair p = real_pair(va[j], vb[j]);
+            cf q = cmul(tw, p.dif);
+            float f = hf;
+            if (ADJ && k == 0) f = 1.f, q = {2.f * q.x, 2.f * q.y};
+            lds[nat_big_word<W>(k)] = pack(__builtin_fmaf(f, p.sum.x, -q.y), __builtin_fmaf(f, p.sum.y, q.x));
+            if (k != 0)
+                lds[nat_big_word<W>(L - k)] =
+                    pack(__builtin_fmaf(f, p.sum.x, q.y), __builtin_fmaf(-f, p.sum.y, q.x));
             tw = cmul(tw, step);
         }
         if (w == 0 && lane == 0) {
