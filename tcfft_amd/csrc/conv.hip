@@ -92,7 +92,7 @@ __device__ __forceinline__ Dft16Op make_dft16_colscaled(int lane, int sign, cons
 }
 
 template <int SIGN, int W, class Post>
-__device__ __forceinline__ void dif4096(u32 (&d)[16][4], const Dif4096Tw& tw, const Dft16Op& op, Post post) {
+__device__ __forceinline__ void dif4096(u32 (&d)[16][4], const Dif4096Tw& tw, const Dft16Op& op, int lane, Post post) {
     constexpr float sg = SIGN < 0 ? 1.f : -1.f;
     cf step[4], rec[4];
 #pragma unroll
@@ -104,7 +104,7 @@ __device__ __forceinline__ void dif4096(u32 (&d)[16][4], const Dif4096Tw& tw, co
         cf t[4];
 #pragma unroll
         for (int j = 0; j < 4; ++j) t[j] = cf{tw.col[j].x, sg * tw.col[j].y};
-        op1 = make_dft16_colscaled(lane_id(), SIGN, t);
+        op1 = make_dft16_colscaled(lane, SIGN, t);
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
             step[i] = cmul(step[i], s16);
@@ -230,7 +230,7 @@ __global__ __launch_bounds__(64 * W) TCFFT_MFMA_BUDGET void k_dif(const u32* in,
                                                 const float2* __restrict__ wn_lo, u32 wn_lo_bits) {
     extern __shared__ u32 lds[];
     constexpr u32 N = 4096u * W;
-    const int lane = lane_id(), w = threadIdx.x >> 6;
+    const int lane = lane_id(), w = W == 1 ? 0 : __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
     const int c16 = lane & 15, g = lane >> 4;
     Dif4096Tw dtw;
     dif4096_tw_load<W>(dtw, lane, w4096, (u32)w, wn_hi, wn_lo, wn_lo_bits);
@@ -242,7 +242,7 @@ __global__ __launch_bounds__(64 * W) TCFFT_MFMA_BUDGET void k_dif(const u32* in,
     __syncthreads();
     stepb_read(d, lds, w, lane);
     const Dft16Op op = make_dft16(lane, SIGN);
-    dif4096<SIGN, W>(d, dtw, op, [](int, int, cf v) -> cf { return v; });
+    dif4096<SIGN, W>(d, dtw, op, lane, [](int, int, cf v) -> cf { return v; });
     u32* dst = out + (size_t)blockIdx.x * N + 4096u * w + 16u * c16 + 4u * g;
 #pragma unroll
     for (int t = 0; t < 16; ++t) store4_nt(dst + 256 * t, d[t]);
@@ -258,8 +258,14 @@ __global__ __launch_bounds__(64 * W) TCFFT_MFMA_BUDGET void k_dif(const u32* in,
 // carried by its stage-1 twiddle recurrence (FP32, before rounding).
 // x and y may alias (in place), so neither is __restrict__: a workgroup reads
 // its signal completely before its first store of y.
+// VALU instructions and memory share the bound (VALU busy 71% of the time), so
+// the wave index is scalar (addresses on the SALU) and the DFT-16 operands of
+// one sign are built from one set of cosines.  With SPEC the kernel runs best
+// at two waves per SIMD: a training step of 256 channels x 8192 x 32 takes 441
+// us (447 before these), 459 with three, 473 with one and a half.  128
+// channels x 4096 x 100: 329 -> 326.5, 64 x 16384 x 50: 411.7 -> 403.9.
 template <int W, bool CONJ, bool SPEC>
-__global__ __launch_bounds__(64 * W) TCFFT_MFMA_BUDGET void k_conv(const u32* x, const u32* __restrict__ h_rev,
+__global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(2, SPEC ? 2 : 8))) void k_conv(const u32* x, const u32* __restrict__ h_rev,
                                                  u32* y, u32* __restrict__ spec, u32 channels,
                                                  float scale, const float2* __restrict__ w4096,
                                                  const float2* __restrict__ wn_hi, const float2* __restrict__ wn_lo,
@@ -267,7 +273,7 @@ __global__ __launch_bounds__(64 * W) TCFFT_MFMA_BUDGET void k_conv(const u32* x,
     extern __shared__ u32 lds[];
     constexpr u32 N = 4096u * W;
     const u32 sig = blockIdx.x;
-    const int lane = lane_id(), w = threadIdx.x >> 6;
+    const int lane = lane_id(), w = W == 1 ? 0 : __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
     const int c16 = lane & 15, g = lane >> 4;
     Dif4096Tw dtw;
     dif4096_tw_load<W>(dtw, lane, w4096, (u32)w, wn_hi, wn_lo, wn_lo_bits);
@@ -289,7 +295,7 @@ __global__ __launch_bounds__(64 * W) TCFFT_MFMA_BUDGET void k_conv(const u32* x,
     {
         const Dft16Op op = make_dft16(lane, -1);
         u32 sq[4];
-        dif4096<-1, W>(d, dtw, op, [&](int t, int i, cf v) -> cf {
+        dif4096<-1, W>(d, dtw, op, lane, [&](int t, int i, cf v) -> cf {
             const cf h = unpack(hq[t & 3][i]);
             if (i == 3 && t + 4 < 16) load4(hq[t & 3], hp + 256 * (t + 4));
             if constexpr (SPEC) {
