@@ -298,6 +298,27 @@ __device__ __forceinline__ void st_at_nt(void* base, u32 off_bytes, T v) {
     __builtin_nontemporal_store(v, reinterpret_cast<T*>(reinterpret_cast<char*>(base) + off_bytes));
 }
 
+// The same with the base held in SGPRs, for rows a run-time step apart: there
+// the compiler otherwise adds the lane's offset once and then each row's to
+// that sum, a 64-bit VALU addition per access (130 of 2258 VALU instructions in
+// a split column pass; fft32 of 8 x 2^20 56.9 -> 56.3 us, 2D 1024 x 1024 x 8
+// 54.15 -> 53.8).  The 2^16 split pass and k_cols_big, which issue their loads
+// sooner the other way, were 1% slower with it.
+#define TCFFT_GLOBAL __attribute__((address_space(1)))
+__device__ __forceinline__ TCFFT_GLOBAL char* row_base(const void* base) {
+    TCFFT_GLOBAL char* p = (TCFFT_GLOBAL char*)const_cast<void*>(base);
+    asm("" : "+s"(p));
+    return p;
+}
+template <class T>
+__device__ __forceinline__ T ld_row_nt(const void* base, u32 off_bytes) {
+    return __builtin_nontemporal_load((const TCFFT_GLOBAL T*)(row_base(base) + off_bytes));
+}
+template <class T>
+__device__ __forceinline__ void st_row_nt(void* base, u32 off_bytes, T v) {
+    __builtin_nontemporal_store(v, (TCFFT_GLOBAL T*)(row_base(base) + off_bytes));
+}
+
 // Small radix-T DFT in FP32 registers (T = 2, 4, 8), in place on v[0..T).
 template <int T>
 __device__ __forceinline__ void small_dft(cf* v, int sign);

@@ -1067,7 +1067,7 @@ __global__ __launch_bounds__(64 * W) TCFFT_MFMA_BUDGET void k_split_colsw(const 
         for (int r0 = 0; r0 < 16; ++r0)
 #pragma unroll
             for (int j = 0; j < 4; ++j) {
-                const f32x2 v = ld_at_nt<f32x2>(ub + ((size_t)(W * (r0 + 16 * j)) << a.q_log2), off);
+                const f32x2 v = ld_row_nt<f32x2>(ub + ((size_t)(W * (r0 + 16 * j)) << a.q_log2), off);
                 dr[r0][j] = v[0];
                 di[r0][j] = v[1];
             }
@@ -1149,8 +1149,8 @@ __global__ __launch_bounds__(64 * W) TCFFT_MFMA_BUDGET void k_split_colsw(const 
                     // row k0 + 16 (4g + i) + 256 k2 (the 64 g part is the lane's)
 #pragma unroll
                     for (int k2 = 0; k2 < W; ++k2)
-                        st_at_nt<f32x2>(ob + ((size_t)(8u * r + tt + 16u * i + 256u * k2) << a.qlo_log2), off,
-                                        f32x2{v[k2].x, v[k2].y});
+                        st_row_nt<f32x2>(ob + ((size_t)(8u * r + tt + 16u * i + 256u * k2) << a.qlo_log2), off,
+                                         f32x2{v[k2].x, v[k2].y});
                 }
             }
         }
