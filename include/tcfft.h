@@ -129,6 +129,8 @@ int tcfft_exec_natural_noalloc(tcfft_plan plan, const void *in, void *out, int d
  * overlap), 16-byte aligned; n_lines is independent of the plan's batch.
  * Allocates nothing; graph-capturable. */
 int tcfft_permute_to_dropin(tcfft_plan plan, const void *in, void *out, int n_lines, void *stream);
+/* The same on FP32 complex input (8 bytes a point), rounded to nearest fp16. */
+int tcfft_permute_to_dropin_f32(tcfft_plan plan, const void *in, void *out, int n_lines, void *stream);
 
 /* Split precision (no counterpart in the reference; config "FP16 hi+lo of
  * FP32 inputs"): FP32 complex input and output (interleaved float re/im,

@@ -47,6 +47,7 @@ EXPORTS = (
     "tcfft_plan_create_r2c_1d", "tcfft_exec_r2c", "tcfft_exec_c2r", "tcfft_permute_to_dropin",
     "tcfft_exec_natural_noalloc", "tcfft_multi_exec_natural", "tcfft_plan_prepare_split", "tcfft_query_split",
     "tcfft_exec_r2c_adjoint", "tcfft_exec_c2r_adjoint", "tcfft_conv_filter_grad_natural",
+    "tcfft_permute_to_dropin_f32",
 )
 NOALLOC_SCRATCH_BYTES = 64 << 20  # TCFFT_NOALLOC_SCRATCH_BYTES
 OPT_SPLIT_CHUNK = 1
@@ -111,6 +112,7 @@ def lib():
         L.tcfft_plan_create_r2c_1d.argtypes = [ctypes.POINTER(_vp), ctypes.c_int, ctypes.c_int]
         L.tcfft_exec_r2c.argtypes = [_vp, _vp, _vp, _vp]
         L.tcfft_permute_to_dropin.argtypes = [_vp, _vp, _vp, ctypes.c_int, _vp]
+        L.tcfft_permute_to_dropin_f32.argtypes = [_vp, _vp, _vp, ctypes.c_int, _vp]
         L.tcfft_exec_c2r.argtypes = [_vp, _vp, _vp, _vp]
         L.tcfft_exec_r2c_adjoint.argtypes = [_vp, _vp, _vp, _vp]
         L.tcfft_exec_c2r_adjoint.argtypes = [_vp, _vp, _vp, _vp]
@@ -236,6 +238,11 @@ class _Plan:
         natural-order data into the order exec consumes, on the device."""
         _check(lib().tcfft_permute_to_dropin(self._h, _vp(in_ptr), _vp(out_ptr), n_lines, _vp(stream)),
                "tcfft_permute_to_dropin")
+
+    def permute_to_dropin_f32(self, in_ptr: int, out_ptr: int, n_lines: int, stream: int = 0):
+        """permute_to_dropin of FP32 complex lines, rounded to fp16."""
+        _check(lib().tcfft_permute_to_dropin_f32(self._h, _vp(in_ptr), _vp(out_ptr), n_lines, _vp(stream)),
+               "tcfft_permute_to_dropin_f32")
 
     def exec_split(self, in_ptr: int, out_ptr: int, direction: int = FORWARD, stream: int = 0):
         """FP32 complex in/out (natural order), FP16 hi/lo MFMA split precision:

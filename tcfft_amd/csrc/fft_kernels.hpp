@@ -178,6 +178,9 @@ struct GatherTile {
 };
 hipError_t launch_gather_tiled_1d(const uint32_t* in, uint32_t* out, uint32_t n_log2, uint32_t total,
                                   const RevSpec& spec, const GatherTile& gt, hipStream_t st);
+// The same on FP32 complex input, rounded to fp16.
+hipError_t launch_gather_tiled_1d(const float2* in, uint32_t* out, uint32_t n_log2, uint32_t total,
+                                  const RevSpec& spec, const GatherTile& gt, hipStream_t st);
 
 // Single-pass transform of N = 4096*W (W = 2, 4, 8, 16) on natural-order
 // input, in -> out (in place allowed when nx_log2 = 0); 2D as launch_rows_nat.

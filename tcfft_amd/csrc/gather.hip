@@ -4,6 +4,7 @@
 // radix reversal that tcfft_doit_half.cpp:6-29 builds on the host: with p's
 // digits p_0 (radix r_0, least significant) ... p_{m-1}, the index is
 // p_{m-1} + r_{m-1}*(p_{m-2} + r_{m-2}*(... + r_1*p_0)).
+#include "fft_device.hpp"
 #include "fft_kernels.hpp"
 
 namespace tcfft {
@@ -39,7 +40,18 @@ __device__ __forceinline__ uint32_t rev_index(uint32_t p, const RevSpec& s) {
 // Each thread moves 4 consecutive elements with one 16-byte load (4
 // consecutive rev) and one 16-byte store (4 consecutive p).  LDS word
 // tau ^ ((tau >> a) & (2^a-1)) spreads both phases over the banks.
-__global__ __launch_bounds__(256) void k_gather_tiled(const uint32_t* __restrict__ in, uint32_t* __restrict__ out,
+// In is uint32_t (fp16 complex) or float2, rounded to fp16 on the way: the
+// FFT-conv layer's filter, whose conversion in a pass of its own took as long
+// as the permutation (5.9 us each for 256 x 8192; layer forward of 200 x 8192
+// over 30 batch entries 129.6 -> 124.7 us, 20 x 8192 over 4 24.9 -> 20.8).
+__device__ __forceinline__ uint4 load4_words(const uint32_t* p) { return *reinterpret_cast<const uint4*>(p); }
+__device__ __forceinline__ uint4 load4_words(const float2* p) {
+    const float4 a = reinterpret_cast<const float4*>(p)[0], b = reinterpret_cast<const float4*>(p)[1];
+    return make_uint4(pack(a.x, a.y), pack(a.z, a.w), pack(b.x, b.y), pack(b.z, b.w));
+}
+
+template <class In>
+__global__ __launch_bounds__(256) void k_gather_tiled(const In* __restrict__ in, uint32_t* __restrict__ out,
                                                       uint32_t n_log2, RevSpec spec, GatherTile gt) {
     __shared__ uint32_t tile[4096];
     __shared__ uint32_t pos_hi[64], rev_lo[64];
@@ -75,7 +87,7 @@ __global__ __launch_bounds__(256) void k_gather_tiled(const uint32_t* __restrict
         // e .. e+3: consecutive input indices (the low b bits of rev)
         const uint32_t hi = e >> gt.b;  // tau's low a bits
         const uint32_t src = rev_block | (e & bmask) | rev_lo[hi & amask];
-        const uint4 v = *reinterpret_cast<const uint4*>(in + base + src);
+        const uint4 v = load4_words(in + base + src);
         const uint32_t t0 = ((e & bmask) << gt.a) | hi;
         tile[lds_word(t0)] = v.x;
         tile[lds_word(t0 + (1u << gt.a))] = v.y;
@@ -95,13 +107,23 @@ __global__ __launch_bounds__(256) void k_gather_tiled(const uint32_t* __restrict
     }
 }
 
-hipError_t launch_gather_tiled_1d(const uint32_t* in, uint32_t* out, uint32_t n_log2, uint32_t total,
-                                  const RevSpec& spec, const GatherTile& gt, hipStream_t st) {
+template <class In>
+static hipError_t launch_gather_t(const In* in, uint32_t* out, uint32_t n_log2, uint32_t total, const RevSpec& spec,
+                                  const GatherTile& gt, hipStream_t st) {
     if (gt.a + gt.b > 12 || gt.a + gt.b > n_log2 || gt.a > 6 || gt.b > 6 || gt.a < 2 || gt.b < 2)
         return hipErrorInvalidValue;
     const uint32_t blocks = total >> (gt.a + gt.b);
-    hipLaunchKernelGGL(k_gather_tiled, dim3(blocks), dim3(256), 0, st, in, out, n_log2, spec, gt);
+    hipLaunchKernelGGL(k_gather_tiled<In>, dim3(blocks), dim3(256), 0, st, in, out, n_log2, spec, gt);
     return hipGetLastError();
+}
+
+hipError_t launch_gather_tiled_1d(const uint32_t* in, uint32_t* out, uint32_t n_log2, uint32_t total,
+                                  const RevSpec& spec, const GatherTile& gt, hipStream_t st) {
+    return launch_gather_t(in, out, n_log2, total, spec, gt, st);
+}
+hipError_t launch_gather_tiled_1d(const float2* in, uint32_t* out, uint32_t n_log2, uint32_t total,
+                                  const RevSpec& spec, const GatherTile& gt, hipStream_t st) {
+    return launch_gather_t(in, out, n_log2, total, spec, gt, st);
 }
 
 }  // namespace tcfft

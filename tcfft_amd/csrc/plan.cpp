@@ -1243,6 +1243,25 @@ bool aligned16(const void* ptr) { return ptr && !((uintptr_t)ptr & 15u); }
 
 }  // namespace
 
+template <class In>
+static int permute_to_dropin(tcfft_plan plan, const void* in, void* out, int n_lines, void* stream) {
+    if (!valid(plan)) return TCFFT_INVALID_PLAN;
+    const Layout& L = plan->lay;
+    if (L.dims != 1) return TCFFT_INVALID_PLAN;
+    if (n_lines < 1 || (long)L.n * n_lines >= (1L << 31)) return TCFFT_INVALID_BATCH;
+    const uintptr_t a = (uintptr_t)in, b = (uintptr_t)out;
+    const size_t points = (size_t)L.n * (size_t)n_lines;
+    if (!in || !out || (a & 15u) || (b & 15u)) return TCFFT_INVALID_POINTER;
+    if (a < b + points * 4u && b < a + points * sizeof(In)) return TCFFT_INVALID_POINTER;  // overlap
+    tcfft::GatherTile gt{};
+    if (!gather_tile(L.rad_y, gt)) return TCFFT_INVALID_VALUE;
+    DeviceGuard guard(plan->device);
+    const hipError_t e = tcfft::launch_gather_tiled_1d((const In*)in, (uint32_t*)out, (uint32_t)ilog2((uint32_t)L.n),
+                                                       (uint32_t)points, rev_spec(L.rad_y), gt, (hipStream_t)stream);
+    if (e != hipSuccess) return hip_fail(e);
+    return TCFFT_SUCCESS;
+}
+
 extern "C" {
 
 int tcfft_exec_dif(tcfft_plan plan, const void* in, void* out, int direction, void* stream) {
@@ -1616,23 +1635,11 @@ int exec_natural_staged(tcfft_plan plan, const void* in, void* out, int directio
 extern "C" {
 
 int tcfft_permute_to_dropin(tcfft_plan plan, const void* in, void* out, int n_lines, void* stream) {
-    if (!valid(plan)) return TCFFT_INVALID_PLAN;
-    const Layout& L = plan->lay;
-    if (L.dims != 1) return TCFFT_INVALID_PLAN;
-    if (n_lines < 1 || (long)L.n * n_lines >= (1L << 31)) return TCFFT_INVALID_BATCH;
-    const uintptr_t a = (uintptr_t)in, b = (uintptr_t)out;
-    const size_t bytes = (size_t)L.n * (size_t)n_lines * 4u;
-    if (!in || !out || (a & 15u) || (b & 15u)) return TCFFT_INVALID_POINTER;
-    if (a < b + bytes && b < a + bytes) return TCFFT_INVALID_POINTER;  // overlap
-    tcfft::GatherTile gt{};
-    if (!gather_tile(L.rad_y, gt)) return TCFFT_INVALID_VALUE;
-    DeviceGuard guard(plan->device);
-    const hipError_t e = tcfft::launch_gather_tiled_1d((const uint32_t*)in, (uint32_t*)out,
-                                                       (uint32_t)ilog2((uint32_t)L.n),
-                                                       (uint32_t)((size_t)L.n * (size_t)n_lines),
-                                                       rev_spec(L.rad_y), gt, (hipStream_t)stream);
-    if (e != hipSuccess) return hip_fail(e);
-    return TCFFT_SUCCESS;
+    return permute_to_dropin<uint32_t>(plan, in, out, n_lines, stream);
+}
+
+int tcfft_permute_to_dropin_f32(tcfft_plan plan, const void* in, void* out, int n_lines, void* stream) {
+    return permute_to_dropin<float2>(plan, in, out, n_lines, stream);
 }
 
 int tcfft_gen_rev(int n, const int* radices, int n_radices, int* rev) {

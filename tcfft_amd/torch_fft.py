@@ -309,9 +309,13 @@ class _FusedConv(torch.autograd.Function):
         stream = _stream(x.device)
         # the filter into the digit-reversed order on the device (LDS-tiled,
         # copy speed; a torch gather reads 16x the bytes for this permutation)
-        h16 = weight.detach().half().contiguous()
-        h_rev = torch.empty_like(h16)
-        plan.permute_to_dropin(h16.data_ptr(), h_rev.data_ptr(), C, stream)
+        w = weight.detach()
+        h_rev = torch.empty(w.shape, dtype=torch.float16, device=w.device)
+        if w.dtype == torch.float32 and w.is_contiguous() and w.data_ptr() % 16 == 0:
+            plan.permute_to_dropin_f32(w.data_ptr(), h_rev.data_ptr(), C, stream)
+        else:
+            h16 = w.half().contiguous()
+            plan.permute_to_dropin(h16.data_ptr(), h_rev.data_ptr(), C, stream)
         y = torch.empty_like(x)
         # the spectrum of x is kept only when the filter gradient will be needed
         # (grad mode is off inside forward, so the caller passes it in)
