@@ -308,7 +308,10 @@ class _FusedConv(torch.autograd.Function):
         plan = _plan(n, signals, x.device)
         stream = _stream(x.device)
         # the filter into the digit-reversed order on the device (LDS-tiled,
-        # copy speed; a torch gather reads 16x the bytes for this permutation)
+        # copy speed; a torch gather reads 16x the bytes for this permutation);
+        # FP32 lines that the kernel can load in 16-byte pieces are rounded on
+        # the way, which saves a launch and a pass (forward of 20 x 8192 over 4
+        # batch entries 24.9 -> 20.8 us)
         w = weight.detach()
         h_rev = torch.empty(w.shape, dtype=torch.float16, device=w.device)
         if w.dtype == torch.float32 and w.is_contiguous() and w.data_ptr() % 16 == 0:
