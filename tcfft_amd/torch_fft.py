@@ -249,7 +249,13 @@ class _RFFT(torch.autograd.Function):
 
     @staticmethod
     def backward(ctx, g):
-        return _c2r(g.half(), ctx.n, adjoint=True)
+        # g may be a part of a larger buffer (torch.cat hands its inputs'
+        # gradients out as views), contiguous but at any element offset; the
+        # kernel reads whole bins of 4 bytes
+        g = g.half().contiguous()
+        if g.data_ptr() % 4:
+            g = g.clone()
+        return _c2r(g, ctx.n, adjoint=True)
 
 
 class _C2R(torch.autograd.Function):
