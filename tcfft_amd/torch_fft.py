@@ -251,8 +251,8 @@ class _RFFT(torch.autograd.Function):
     def backward(ctx, g):
         # g may be a part of a larger buffer (torch.cat hands its inputs'
         # gradients out as views), contiguous but at any element offset; the
-        # kernel reads whole bins of 4 bytes
-        g = g.half().contiguous()
+        # kernel reads whole bins of 4 bytes, and the sign as it is stored
+        g = g.half().contiguous().resolve_neg()
         if g.data_ptr() % 4:
             g = g.clone()
         return _c2r(g, ctx.n, adjoint=True)
@@ -320,7 +320,7 @@ class _FusedConv(torch.autograd.Function):
         # batch entries 24.9 -> 20.8 us)
         w = weight.detach()
         h_rev = torch.empty(w.shape, dtype=torch.float16, device=w.device)
-        if w.dtype == torch.float32 and w.is_contiguous() and w.data_ptr() % 16 == 0:
+        if w.dtype == torch.float32 and w.is_contiguous() and w.data_ptr() % 16 == 0 and not w.is_neg():
             plan.permute_to_dropin_f32(w.data_ptr(), h_rev.data_ptr(), C, stream)
         else:
             h16 = w.half().contiguous()
