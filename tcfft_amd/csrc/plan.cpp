@@ -222,6 +222,13 @@ struct tcfft_plan_s {
     // 2D 1024^2 x 8: 14.7 against 15.1)
     int rows_waves = 0;
     int rows_tiles = 0;  // tiles per wave of a row first pass (rows_nt; 0 = by the grid)
+    // The schedule options as the caller set them.  The tuner, which times
+    // tcfft_exec, changes only the fields above: the natural-order row passes
+    // have other optima (256 x 16384: 8 tiles win the drop-in call, 8.0 us
+    // against 8.7 with 4; natural order 10.8 with 8, 9.5 with 4)
+    struct {
+        int delay = -1, groups = 3, waves = 0, tiles = 0;
+    } set;
     int cols_delay = 1;   // start delay of the radix-256*W column pass (3 groups; 2D 1024^2 x 8: 36.0 -> 33.8 us)
     int split_delay = 2;  // start delay of the split-precision passes (3 groups; 2^16 x 256: 110.6 -> 106.6 us)
     // first pass's output stores of a multi-pass plan: -1 = cached while the
@@ -530,15 +537,15 @@ tcfft::StartSched nat_big_sched(const tcfft_plan_s* p, int W, uint32_t lines) {
 // only when the grid is at most one 4-wave workgroup per CU (4096 x 1024:
 // 10.0 -> 9.2 us); with more workgroups per CU they desynchronise by
 // themselves and a delay only costs time (1024 x 8192: 15.9 -> 16.2 us).
-// Waves per workgroup of a contiguous-row first pass: the plan's setting, or
+// Waves per workgroup of a contiguous-row first pass: the plan's `setting`, or
 // by default 4 for 4096-point lines over at least 32 waves per CU and 1
 // otherwise.  Measured (rotated buffers): 4096 x 1024 7.7 us with one wave
 // against 8.6 with four; even at 2048-4096 lines; four ahead from 8192
 // lines (47.7 against 48.6 us) to 65536 (352 against 369 us); for 2048-point
 // and shorter lines one wave stays ahead at every batch (2048 x 131072: 369
 // against 403 us).
-uint32_t rows_wg(const tcfft_plan_s* p, const Pass& ps) {
-    if (p->rows_waves > 0) return (uint32_t)p->rows_waves;
+uint32_t rows_wg(const tcfft_plan_s* p, const Pass& ps, int setting) {
+    if (setting > 0) return (uint32_t)setting;
     const uint32_t waves = (ps.n_tiles + 15u) / 16u;
     return ps.radix == 16 && waves >= 32u * (uint32_t)p->cus ? 4u : 1u;
 }
@@ -558,16 +565,16 @@ uint32_t rows_wg(const tcfft_plan_s* p, const Pass& ps) {
 // 256 x 16384 9.02 / 8.04 / 8.68; at two waves per SIMD or more, 16 (2D
 // 1024^2 x 8 31.3 us against 34.0 at 8 and 36.0 at 4; 1024 x 8192 14.2
 // against 16.7 and 18.3).
-uint32_t rows_nt(const tcfft_plan_s* p, const Pass& ps) {
+uint32_t rows_nt(const tcfft_plan_s* p, const Pass& ps, int setting) {
     const uint32_t T = (uint32_t)ps.radix;
     if (ps.has_epi) return 16u;
     if (T >= 16) {
-        if (p->rows_tiles > 0) return (uint32_t)p->rows_tiles;
+        if (setting > 0) return (uint32_t)setting;
         const uint32_t lines = ps.n_tiles / 16u, cus = (uint32_t)p->cus;
         return lines <= cus ? 4u : lines <= 4u * cus ? 8u : 16u;
     }
     const uint32_t lo = T <= 4 ? 4u : 8u;
-    if (p->rows_tiles > 0) return std::max((uint32_t)p->rows_tiles, lo);
+    if (setting > 0) return std::max((uint32_t)setting, lo);
     const uint32_t want = 8u * (uint32_t)p->cus;  // two waves per SIMD
     for (uint32_t nt = 16u; nt > lo; nt /= 2)
         if ((ps.n_tiles + nt - 1u) / nt >= want) return nt;
@@ -585,10 +592,10 @@ uint32_t rows_nt(const tcfft_plan_s* p, const Pass& ps) {
 // 28.7).
 uint32_t rows_nt_nat(const tcfft_plan_s* p, const Pass& ps) {
     if (ps.radix < 16) {
-        const uint32_t nt = rows_nt(p, ps);
-        return ps.radix == 1 && nt == 8u && !p->rows_tiles ? 4u : nt;
+        const uint32_t nt = rows_nt(p, ps, p->set.tiles);
+        return ps.radix == 1 && nt == 8u && !p->set.tiles ? 4u : nt;
     }
-    if (p->rows_tiles > 0) return (uint32_t)p->rows_tiles;
+    if (p->set.tiles > 0) return (uint32_t)p->set.tiles;
     return ps.n_tiles / 16u <= 2u * (uint32_t)p->cus ? 4u : 8u;
 }
 
@@ -596,8 +603,16 @@ uint32_t rows_nt_nat(const tcfft_plan_s* p, const Pass& ps) {
 // rows that fill the chip, whose stores go to permuted lines (2D 1024 x 1024
 // x 8 29.4 us against 30.7 with one; 1D 1024 x 16384 26.7 against 26.1).
 uint32_t rows_wg_nat(const tcfft_plan_s* p, const Pass& ps) {
-    if (p->rows_waves > 0) return (uint32_t)p->rows_waves;
-    return p->lay.dims == 2 && (ps.n_tiles + 15u) / 16u >= 4u * (uint32_t)p->cus ? 4u : rows_wg(p, ps);
+    if (p->set.waves > 0) return (uint32_t)p->set.waves;
+    return p->lay.dims == 2 && (ps.n_tiles + 15u) / 16u >= 4u * (uint32_t)p->cus ? 4u : rows_wg(p, ps, 0);
+}
+
+// Start schedule of the natural-order pass: the caller's, or none.  The pass
+// has no load phase of its own to stagger: with a delay of 1, 1024 x 64 takes
+// 3.37 us against 2.50 without, 4096 x 256 5.17 and 4.74, 1024 x 4096 8.8 and
+// 8.4, 2048 x 2048 9.6 and 8.9, 2D 32 x 2048 x 64 16.8 and 15.9.
+tcfft::StartSched rows_nat_sched(const tcfft_plan_s* p) {
+    return tcfft::StartSched{(uint32_t)std::max(p->set.delay, 0), (uint32_t)p->set.groups, 0u};
 }
 
 // Start schedule of a contiguous-row first pass run with nt tiles per wave.
@@ -660,10 +675,11 @@ int run_passes(tcfft_plan_s* p, uint32_t* buf, int sign, hipStream_t st, size_t 
         const EpiParams* epi = ps.has_epi ? &ps.epi : nullptr;
         hipError_t e;
         if (ps.kind == 0) {
-            tcfft::StartSched sc = rows_sched(p, ps, rows_nt(p, ps));
+            const uint32_t nt = rows_nt(p, ps, p->rows_tiles);
+            tcfft::StartSched sc = rows_sched(p, ps, nt);
             sc.cached_out = cached_out(p, i, nsig);
-            e = tcfft::launch_rows(ps.radix, buf, ps.n_tiles, sign, p->w4096, epi, sc, rows_wg(p, ps), rows_nt(p, ps),
-                                   st);
+            e = tcfft::launch_rows(ps.radix, buf, ps.n_tiles, sign, p->w4096, epi, sc,
+                                   rows_wg(p, ps, p->rows_waves), nt, st);
         } else if (ps.kind == 2) {
             tcfft::StartSched sc = big_sched(p, ps.radix, ps.n_tiles);
             sc.cached_out = cached_out(p, i, nsig);
@@ -1343,7 +1359,7 @@ int tcfft_plan_set_option(tcfft_plan plan, int option, int value) {
         return TCFFT_SUCCESS;
     case TCFFT_OPT_BIG_DELAY:
         if (value < -1 || value > 64) return TCFFT_INVALID_VALUE;
-        plan->big_delay = value;
+        plan->big_delay = plan->set.delay = value;
         return TCFFT_SUCCESS;
     case TCFFT_OPT_COLS_DELAY:
         if (value < 0 || value > 64) return TCFFT_INVALID_VALUE;
@@ -1351,7 +1367,7 @@ int tcfft_plan_set_option(tcfft_plan plan, int option, int value) {
         return TCFFT_SUCCESS;
     case TCFFT_OPT_BIG_GROUPS:
         if (value < 1 || value > 8) return TCFFT_INVALID_VALUE;
-        plan->big_groups = value;
+        plan->big_groups = plan->set.groups = value;
         return TCFFT_SUCCESS;
     case TCFFT_OPT_SPLIT_DELAY:
         if (value < 0 || value > 64) return TCFFT_INVALID_VALUE;
@@ -1359,7 +1375,7 @@ int tcfft_plan_set_option(tcfft_plan plan, int option, int value) {
         return TCFFT_SUCCESS;
     case TCFFT_OPT_ROWS_WAVES:
         if (value != 0 && value != 1 && value != 2 && value != 4) return TCFFT_INVALID_VALUE;
-        plan->rows_waves = value;
+        plan->rows_waves = plan->set.waves = value;
         return TCFFT_SUCCESS;
     case TCFFT_OPT_FIRST_CACHED:
         if (value < -1 || value > 1) return TCFFT_INVALID_VALUE;
@@ -1367,7 +1383,7 @@ int tcfft_plan_set_option(tcfft_plan plan, int option, int value) {
         return TCFFT_SUCCESS;
     case TCFFT_OPT_ROWS_TILES:
         if (value != 0 && value != 4 && value != 8 && value != 16) return TCFFT_INVALID_VALUE;
-        plan->rows_tiles = value;
+        plan->rows_tiles = plan->set.tiles = value;
         return TCFFT_SUCCESS;
     case TCFFT_OPT_MALL_CHUNK:
         if (value != 0 && (value < 16 || value > 65536)) return TCFFT_INVALID_VALUE;
@@ -1580,7 +1596,7 @@ int exec_natural_staged(tcfft_plan plan, const void* in, void* out, int directio
             Pass fp = first;
             fp.n_tiles = (uint32_t)((uint64_t)first.n_tiles / B * ns);
             const uint32_t nt = fused_rows ? rows_nt_nat(plan, fp) : 16u;
-            tcfft::StartSched sc = fused_rows ? rows_sched(plan, fp, nt) : nat_big_sched(plan, fp.radix, fp.n_tiles);
+            tcfft::StartSched sc = fused_rows ? rows_nat_sched(plan) : nat_big_sched(plan, fp.radix, fp.n_tiles);
             sc.cached_out = cached_out(plan, 0, ns);
             const uint32_t* ci = rsrc + per * s0;
             uint32_t* co = (uint32_t*)out + per * s0;

@@ -1,0 +1,35 @@
+"""What tcfft_plan_autotune and tcfft_multi_autotune choose, they choose by
+timing the drop-in call: it must not reach the natural-order kernels, which
+have other optima.  The launches of a tuned plan's natural-order call are
+compared with an untuned plan's."""
+import pytest
+
+import tcfft_amd
+from launches import launches
+
+torch = pytest.importorskip("torch")
+pytestmark = pytest.mark.gpu
+
+
+def natural_launches(plan, x, out, params=None):
+    return launches(lambda st: plan.exec_natural(x.data_ptr(), out.data_ptr(), tcfft_amd.FORWARD, st), params)
+
+
+# shapes whose drop-in optimum (tiles per wave, waves per workgroup) is not the
+# natural-order one: 256-point lines (8 tiles against 4), 2D rows (1 wave
+# against 4)
+@pytest.mark.parametrize("shape", [(256, 16384), (1024, 1024, 8), (2048, 8192)])
+def test_tuned_rows_keep_the_natural_launch(shape):
+    x = (torch.rand(*(shape[::-1] if len(shape) == 2 else shape), 2, device="cuda") * 2 - 1).half()
+    out = torch.empty_like(x)
+    make = tcfft_amd.Plan1D if len(shape) == 2 else tcfft_amd.Plan2D
+    plain, tuned = make(*shape), make(*shape)
+    scratch = x.clone()
+    tuned.autotune(scratch.data_ptr())
+    a, b = (natural_launches(p, x, out, {0: (6,)})[0] for p in (plain, tuned))
+    assert b.key == a.key and b.words == [0]  # parameter 6: the start schedule, its delay first
+    # a caller's own choice holds for both calls
+    tuned.set_option(tcfft_amd.OPT_ROWS_WAVES, 2)
+    assert natural_launches(tuned, x, out)[0].threads == 128
+    plain.destroy()
+    tuned.destroy()
