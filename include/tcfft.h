@@ -239,7 +239,7 @@ int tcfft_conv_filter_grad_natural(tcfft_plan plan, int channels, const void *x_
  * but leave compute units idle; at 2^16 x 256 the whole batch is fastest).
  * TCFFT_OPT_BIG_DELAY (-1..64, default -1 = per-kernel default; the
  * natural-order 65536-point kernel then runs 5 groups with delay 3, the
- * natural-order pass over lines of 256..4096 points none) and
+ * natural-order passes over lines of 256..4096 and 2^17..2^20 points none) and
  * TCFFT_OPT_BIG_GROUPS (1..8, default 3): start schedule of the first pass
  * (contiguous lines of up to 65536 points); the workgroups resident at
  * launch form GROUPS groups and group k starts k * DELAY quanta (1024 GPU
@@ -298,9 +298,9 @@ int tcfft_plan_set_option(tcfft_plan plan, int option, int value);
  * 256 MiB buffer that the call allocates and frees, so that the data is
  * timed cold, as a caller's previous work leaves it; the four fastest
  * candidates are timed again in three alternating rounds before the choice.
- * The choices are made for tcfft_exec; the natural-order pass over lines of
- * 256..4096 points, whose optima are others, keeps the options as the caller
- * set them and their defaults.
+ * The choices are made for tcfft_exec; the natural-order passes over lines of
+ * 256..4096 and 2^17..2^20 points, whose optima are others, keep the options
+ * as the caller set them and their defaults.
  * On return `data` holds what it held on entry (if the copy cannot be
  * allocated, transforms of itself, and the timed runs see those).  No
  * reference counterpart (the reference has one fixed launch per size). */

@@ -224,8 +224,8 @@ struct tcfft_plan_s {
     int rows_tiles = 0;  // tiles per wave of a row first pass (rows_nt; 0 = by the grid)
     // The schedule options as the caller set them.  The tuner, which times
     // tcfft_exec, changes only the fields above: the natural-order row passes
-    // have other optima (256 x 16384: 8 tiles win the drop-in call, 8.0 us
-    // against 8.7 with 4; natural order 10.8 with 8, 9.5 with 4)
+    // and k_lines_nat have other optima (256 x 16384: 8 tiles win the drop-in
+    // call, 8.0 us against 8.7 with 4; natural order 10.8 with 8, 9.5 with 4)
     struct {
         int delay = -1, groups = 3, waves = 0, tiles = 0;
     } set;
@@ -607,11 +607,12 @@ uint32_t rows_wg_nat(const tcfft_plan_s* p, const Pass& ps) {
     return p->lay.dims == 2 && (ps.n_tiles + 15u) / 16u >= 4u * (uint32_t)p->cus ? 4u : rows_wg(p, ps, 0);
 }
 
-// Start schedule of the natural-order pass: the caller's, or none.  The pass
-// has no load phase of its own to stagger: with a delay of 1, 1024 x 64 takes
-// 3.37 us against 2.50 without, 4096 x 256 5.17 and 4.74, 1024 x 4096 8.8 and
-// 8.4, 2048 x 2048 9.6 and 8.9, 2D 32 x 2048 x 64 16.8 and 15.9.
-tcfft::StartSched rows_nat_sched(const tcfft_plan_s* p) {
+// Start schedule of the natural-order row pass, and of k_lines_nat: the
+// caller's, or none.  The row pass has no load phase of its own to stagger:
+// with a delay of 1, 1024 x 64 takes 3.37 us against 2.50 without, 4096 x 256
+// 5.17 and 4.74, 1024 x 4096 8.8 and 8.4, 2048 x 2048 9.6 and 8.9, 2D 32 x
+// 2048 x 64 16.8 and 15.9.
+tcfft::StartSched nat_sched(const tcfft_plan_s* p) {
     return tcfft::StartSched{(uint32_t)std::max(p->set.delay, 0), (uint32_t)p->set.groups, 0u};
 }
 
@@ -1596,7 +1597,7 @@ int exec_natural_staged(tcfft_plan plan, const void* in, void* out, int directio
             Pass fp = first;
             fp.n_tiles = (uint32_t)((uint64_t)first.n_tiles / B * ns);
             const uint32_t nt = fused_rows ? rows_nt_nat(plan, fp) : 16u;
-            tcfft::StartSched sc = fused_rows ? rows_nat_sched(plan) : nat_big_sched(plan, fp.radix, fp.n_tiles);
+            tcfft::StartSched sc = fused_rows ? nat_sched(plan) : nat_big_sched(plan, fp.radix, fp.n_tiles);
             sc.cached_out = cached_out(plan, 0, ns);
             const uint32_t* ci = rsrc + per * s0;
             uint32_t* co = (uint32_t*)out + per * s0;
@@ -1626,9 +1627,9 @@ int exec_natural_staged(tcfft_plan plan, const void* in, void* out, int directio
         L.passes[1].radix <= 16) {
         return for_chunks(plan, [&](uint32_t s0, uint32_t ns) -> int {
             const size_t off = (size_t)L.n * s0;
-            // no stagger by default: 2^20 x 16 66 us with the 65536-point
+            // no stagger but the caller's: 2^20 x 16 66 us with the 65536-point
             // kernel's schedule, 59 without, 2^17 x 128 59 and 53
-            tcfft::StartSched sc{plan->big_delay > 0 ? (uint32_t)plan->big_delay : 0u, (uint32_t)plan->big_groups, 0u};
+            tcfft::StartSched sc = nat_sched(plan);
             sc.cached_out = cached_out(plan, 0, ns);
             const hipError_t e = tcfft::launch_nat_two_pass(L.passes[1].radix, src + off, (uint32_t*)out + off, ns,
                                                             direction, plan->w4096, first.epi, sc, st);

@@ -33,3 +33,18 @@ def test_tuned_rows_keep_the_natural_launch(shape):
     assert natural_launches(tuned, x, out)[0].threads == 128
     plain.destroy()
     tuned.destroy()
+
+
+@pytest.mark.parametrize("n,batch", [(1 << 17, 128), (1 << 20, 16)])
+def test_tuned_two_pass_lines_start_together(n, batch):
+    """k_lines_nat runs without a start delay (the first word of its parameter
+    6, the schedule) unless the caller sets one."""
+    x = (torch.rand(batch, n, 2, device="cuda") * 2 - 1).half()
+    out = torch.empty_like(x)
+    plan = tcfft_amd.Plan1D(n, batch)
+    scratch = x.clone()
+    plan.autotune(scratch.data_ptr())
+    assert natural_launches(plan, x, out, {0: (6,)})[0].words == [0]
+    plan.set_option(tcfft_amd.OPT_BIG_DELAY, 2)
+    assert natural_launches(plan, x, out, {0: (6,)})[0].words == [2]
+    plan.destroy()
