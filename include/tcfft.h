@@ -328,7 +328,9 @@ int tcfft_multi_exec(tcfft_multi plan, void *data, int direction, void *stream);
  * Allocates nothing; graph-capturable. */
 int tcfft_multi_exec_natural(tcfft_multi plan, const void *in, void *out, int direction, void *stream);
 /* Schedule: grid = persistent workgroups (0 = one per task), order = task
- * order (0 largest sizes first, 1 interleaved, 2 smallest first). */
+ * order (0 largest sizes first, 1 interleaved, 2 smallest first).
+ * tcfft_multi_exec_natural walks a list of order 0 from its end when it has
+ * more tasks than the GPU has compute units. */
 int tcfft_multi_set_schedule(tcfft_multi plan, int grid, int order);
 /* Start delay of the resident workgroups (0..64; 0 = none): they form 3
  * groups by their index within an XCD and group k starts k * delay quanta of

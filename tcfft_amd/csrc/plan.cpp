@@ -1704,7 +1704,7 @@ struct tcfft_multi_s {
     tcfft::MultiTables tb{};
     uint32_t grid = 256;
     int order = 0;
-    bool order_set = false;  // the caller (or the tuner) chose the task order
+    uint32_t cus = 256;  // compute units of the device
     int delay = 0;  // start delay of the resident workgroups (3 groups, quanta of 1024 cycles)
     std::vector<void*> allocs;
 };
@@ -1805,6 +1805,9 @@ int tcfft_multi_create(tcfft_multi* plan, int n_signals, const int* sizes) {
     int rc = TCFFT_SUCCESS;
     hipError_t e = hipGetDevice(&p->device);
     if (e != hipSuccess) rc = hip_fail(e);
+    int cus = 0;
+    if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, p->device) == hipSuccess && cus > 0)
+        p->cus = (uint32_t)cus;
     multi_build_tasks(p, 0);
     void* d = nullptr;
     if (!rc) rc = multi_alloc(p, p->tasks.size() * sizeof(tcfft::MultiTask), &d);
@@ -1872,7 +1875,6 @@ int tcfft_multi_set_schedule(tcfft_multi plan, int grid, int order) {
     if (grid < 0 || order < 0 || order > 2) return TCFFT_INVALID_VALUE;
     DeviceGuard guard(plan->device);
     plan->grid = (uint32_t)grid;
-    plan->order_set = true;
     if (order != plan->order) {
         plan->order = order;
         multi_build_tasks(plan, order);
@@ -1901,12 +1903,16 @@ int tcfft_multi_exec_natural(tcfft_multi plan, const void* in, void* out, int di
     if (in != out && a < b + bytes && b < a + bytes) return TCFFT_INVALID_POINTER;  // partial overlap
     if (direction != TCFFT_FORWARD && direction != TCFFT_INVERSE) return TCFFT_INVALID_VALUE;
     DeviceGuard guard(plan->device);
-    // Until an order is chosen, a list of more than a task per CU is walked
-    // from its end: the small signals' tasks first, whose different lengths
-    // spread the workgroups' phases (natural order, 2048 signals 68.9 -> 65.1
-    // us, 4096 139.7 -> 125.2; fewer tasks want the longest first, 300 signals
-    // 25.5 against 25.9; the drop-in call gains nothing).
-    const bool reverse = !plan->order_set && plan->tasks.size() > plan->grid;
+    // Order 0 with more than a task per CU is walked from its end: the small
+    // signals' tasks first, whose different lengths spread the workgroups'
+    // phases.  Natural order, largest first -> smallest first: 2048 signals
+    // (480 tasks) 68.5 -> 63.6 us on a grid of 256, 102.6 -> 96.9 on 128, 68.0
+    // -> 63.9 on 512; 4096 signals 131.8 -> 122.1, but 190.1 -> 193.1 on 128;
+    // 1100 signals 35.9 -> 35.4.  With a task per CU or fewer the longest go
+    // first (700 signals 26.6 against 26.9).  The drop-in call gains nothing
+    // from it.  A property of the list alone, so that setting the current
+    // schedule again changes nothing.
+    const bool reverse = plan->order == 0 && plan->tasks.size() > plan->cus;
     hipError_t e = tcfft::launch_multi_nat((const uint32_t*)in, (uint32_t*)out, plan->d_tasks,
                                            (uint32_t)plan->tasks.size(), plan->d_offsets, plan->grid, direction,
                                            plan->w4096, plan->tb, reverse,

@@ -2,6 +2,7 @@
 timing the drop-in call: it must not reach the natural-order kernels, which
 have other optima.  The launches of a tuned plan's natural-order call are
 compared with an untuned plan's."""
+import numpy as np
 import pytest
 
 import tcfft_amd
@@ -47,4 +48,33 @@ def test_tuned_two_pass_lines_start_together(n, batch):
     assert natural_launches(plan, x, out, {0: (6,)})[0].words == [0]
     plan.set_option(tcfft_amd.OPT_BIG_DELAY, 2)
     assert natural_launches(plan, x, out, {0: (6,)})[0].words == [2]
+    plan.destroy()
+
+
+def test_uneven_natural_walk_is_kept():
+    """A list of more than a task per compute unit in the default order is
+    walked from its end (parameter 7 of k_multi_nat) whatever the grid, and
+    also after the current schedule is set again or tuned."""
+    rng = np.random.default_rng(3)
+    sizes = 2 ** rng.integers(8, 17, 2048)
+    plan = tcfft_amd.MultiPlan(sizes)
+    assert plan.n_tasks > 256
+    x = (torch.rand(int(sizes.sum()), 2, device="cuda") * 2 - 1).half()
+    out = torch.empty_like(x)
+
+    def reverse(p=plan):
+        return natural_launches(p, x, out, {0: (7,)})[0].words[0]
+
+    assert reverse() == 1
+    plan.set_schedule(*plan.schedule()[:2])
+    assert reverse() == 1
+    for grid, order, want in ((0, 0, 1), (512, 0, 1), (128, 0, 1), (256, 2, 0), (256, 1, 0), (256, 0, 1)):
+        plan.set_schedule(grid, order)
+        assert reverse() == want, (grid, order)
+    scratch = x.clone()
+    _, order, _ = plan.autotune(scratch.data_ptr())
+    assert reverse() == (order == 0)
+    few = tcfft_amd.MultiPlan(sizes[:300])
+    assert few.n_tasks <= 256 and reverse(few) == 0
+    few.destroy()
     plan.destroy()
