@@ -98,8 +98,9 @@ int tcfft_exec(tcfft_plan plan, void *data, int direction, void *stream);
 /* Natural-order input and output; the result equals tcfft_exec on the input
  * permuted by the caller-side gen_rev (tcfft_doit_half.cpp:40-46), bit for
  * bit.  The digit reversal runs in the first pass's load for lines (1D, or
- * 2D rows) of up to 65536 points and 1D lines of 2^17..2^20 points of a plan
- * with the default radix split, else as one extra tiled reversal pass.  in == out is allowed; in and out must not otherwise
+ * 2D rows) of up to 65536 points and, from two to six signals up, 1D lines of
+ * 2^17..2^20 points of a plan with the default radix split, else as one extra
+ * tiled reversal pass.  in == out is allowed; in and out must not otherwise
  * overlap.  The 2D in-place case and the 1D in-place case above 65536
  * points stage the input in a device workspace of the buffer's size that such
  * plans allocate at creation (2D plans, 1D plans whose first pass does not

@@ -1622,11 +1622,34 @@ int exec_natural_staged(tcfft_plan plan, const void* in, void* out, int directio
         int rc = stage(src);
         if (rc) return rc;
     }
-    // 2^17..2^20 points: two passes that read natural order themselves
-    if (L.passes.size() == 2 && first.kind == 2 && first.radix == 16 && first.has_epi && L.passes[1].kind == 1 &&
-        L.passes[1].radix <= 16) {
-        return for_chunks(plan, [&](uint32_t s0, uint32_t ns) -> int {
-            const size_t off = (size_t)L.n * s0;
+    // 2^17..2^20 points (n = 65536*R): two passes that read natural order
+    // themselves, or, for the fewest signals, the reversal and the plan's own
+    // passes.  k_lines_nat's R workgroups a signal each pull 256 KiB through
+    // one CU, which a small grid waits for when the input is not in L2; where
+    // they are a multiple of 16, the two that share 128-byte lines run on one
+    // XCD.  Input in the MALL, reversal + plan / two passes: 2^17 x 1 25.6 /
+    // 26.6 us, x 4 26.6 / 27.0, x 5 27.3 / 27.2, x 8 28.3 / 25.3; 2^18 x 1 26.2 /
+    // 28.9, x 3 27.7 / 29.4, x 4 28.5 / 27.1, x 5 30.2 / 30.2; 2^19 x 1 27.3 /
+    // 31.8, x 2 29.0 / 29.5, x 3 32.0 / 33.7, x 4 34.0 / 33.6, x 5 36.6 / 36.8;
+    // 2^20 x 1 29.1 / 33.1, x 2 34.1 / 37.4, x 3 38.8 / 39.5, x 4 45.5 / 41.0.
+    // Between the split pass and this transform of a real-input plan, r2c and
+    // c2r of twice the points: 2^17 x 4 30.3 / 29.9 and 29.6 / 29.8, x 5 31.6 /
+    // 30.3 and 30.6 / 30.3; 2^18 x 3 32.3 / 32.5 and 31.5 / 32.8, x 4 33.9 / 30.8
+    // and 32.8 / 29.2; 2^19 x 1 31.1 / 34.4 and 30.7 / 34.5, x 2 34.9 / 33.3 and
+    // 33.8 / 31.3, x 3 40.2 / 38.3 and 38.5 / 39.4; 2^20 x 1 33.8 / 36.4 and 33.5 /
+    // 34.7, x 2 43.1 / 42.8 and 40.4 / 38.7, x 3 51.2 / 47.6 and 46.1 / 42.6.
+    const bool two_pass = L.passes.size() == 2 && first.kind == 2 && first.radix == 16 && first.has_epi &&
+                          L.passes[1].kind == 1 && L.passes[1].radix <= 16;
+    auto enough = [&](uint32_t ns) {
+        const uint32_t R = (uint32_t)L.passes[1].radix;
+        if (plan->real_n) return ns >= (R == 2u ? 5u : R == 4u ? 4u : 2u);
+        return ns >= (R <= 4u ? 5u : R == 8u ? 6u : 4u) || (R <= 8u && ns * R % 16u == 0u);
+    };
+    // per batch chunk (chunk_signals)
+    const tcfft::RevSpec spec = rev_spec(L.rad_y);
+    return for_chunks(plan, [&](uint32_t s0, uint32_t ns) -> int {
+        const size_t off = (size_t)L.n * s0;
+        if (two_pass && enough(ns)) {
             // no stagger but the caller's: 2^20 x 16 66 us with the 65536-point
             // kernel's schedule, 59 without, 2^17 x 128 59 and 53
             tcfft::StartSched sc = nat_sched(plan);
@@ -1634,12 +1657,7 @@ int exec_natural_staged(tcfft_plan plan, const void* in, void* out, int directio
             const hipError_t e = tcfft::launch_nat_two_pass(L.passes[1].radix, src + off, (uint32_t*)out + off, ns,
                                                             direction, plan->w4096, first.epi, sc, st);
             return e == hipSuccess ? TCFFT_SUCCESS : hip_fail(e);
-        });
-    }
-    // per batch chunk (chunk_signals): the reversal, then the passes
-    const tcfft::RevSpec spec = rev_spec(L.rad_y);
-    return for_chunks(plan, [&](uint32_t s0, uint32_t ns) -> int {
-        const size_t off = (size_t)L.n * s0;
+        }
         hipError_t e = tcfft::launch_gather_tiled_1d(src + off, (uint32_t*)out + off, (uint32_t)ilog2((uint32_t)L.n),
                                                      (uint32_t)((size_t)L.n * ns), spec, gt, st);
         if (e != hipSuccess) return hip_fail(e);
