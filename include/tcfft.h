@@ -271,7 +271,8 @@ int tcfft_conv_filter_grad_natural(tcfft_plan plan, int channels, const void *x_
  * and four waves per line).  The default is the largest that still gives
  * every SIMD two waves (16 on all but small batches); for 4096-point lines
  * 4 up to one line per CU, 8 up to four, 16 above, and on natural-order
- * input 4 up to one line per CU, 16 from 4 to 8 lines per CU, 8 otherwise.
+ * input 4 up to two lines per CU, 8 above (16 for most 2D shapes of 6 to 15
+ * lines per CU).
  * None of these options changes results. */
 enum tcfft_option {
     TCFFT_OPT_SPLIT_CHUNK = 1,

@@ -2045,9 +2045,16 @@ static hipError_t launch_rows_half_nat_t(const u32* in, u32* out, u32 n_tiles, c
     const size_t lds = (DIRECT ? 4096u : 8192u) * sizeof(u32);
     auto k = k_rows_half_nat<SIGN, CACHED, WPL, DIRECT>;
     const KernelInfo ki = kernel_info(k, 64 * WPL, lds);
-    // whole lines through LDS above 16 lines per CU (see the kernel)
+    // whole lines through LDS above 16 lines per CU (see the kernel).  2D, whose
+    // stores are permuted, also at 3 to 4 and at 16 lines per CU (16 x 4096 x 48
+    // 14.1 us against 14.4 direct, x 64 17.0 and 17.8, x 256 48.2 and 49.3, 1024 x
+    // 4096 20.8 and 21.3; x 40 13.2 and 12.6, x 80 20.1 and 19.9), except for nx =
+    // 128..512 (128 x 4096 x 8 19.2 and 18.4, 512 x 4096 x 2 21.7 and 20.9; see
+    // rows_nt_nat)
     if constexpr (WPL == 2 && DIRECT) {
-        if (lines > 16u * ki.cus)
+        const bool permuted = nx_log2 != 0 && (nx_log2 < 7 || nx_log2 > 9);
+        if (lines > 16u * ki.cus ||
+            (permuted && (lines == 16u * ki.cus || (lines >= 3u * ki.cus && lines <= 4u * ki.cus))))
             return launch_rows_half_nat_t<SIGN, CACHED, WPL, false>(in, out, n_tiles, w4096, nx_log2, xpos, sched, st);
     }
     if (ki.lds_status != hipSuccess) return ki.lds_status;

@@ -585,7 +585,14 @@ uint32_t rows_nt(const tcfft_plan_s* p, const Pass& ps, int setting) {
 // up to two lines per CU, two above (out of place, random input; one / two /
 // four waves per line: 4096 x 256 6.7 / 5.4 / 5.0 us, 4096 x 512 7.5 / 6.2 /
 // 5.4, 4096 x 1024 8.4 / 7.8 / 8.2, 4096 x 2048 12.9 / 12.0 / 13.9, 4096 x
-// 4096 27.3 / 22.7 / 24.0, 4096 x 16384 95.6 / 90.7 / 107).  256-point lines:
+// 4096 27.3 / 22.7 / 24.0, 4096 x 16384 95.6 / 90.7 / 107).  2D lines go to
+// permuted places: one wave per line from 6 to below 16 lines per CU (whole
+// transforms, one / two waves: 16 x 4096 x 96 22.9 / 23.4 us, x 128 27.6 / 28.9,
+// x 192 36.6 / 39.3, x 256 48.7 / 48.2, x 384 69.7 / 68.7; 1024 x 4096 x 2 31.9 /
+// 33.3, x 3 39.9 / 43.7), except for nx = 128..512, where two stay ahead (128 x
+// 4096 x 16 28.4 / 26.7, 256 x 4096 x 16 51.2 / 48.2, 512 x 4096 x 4 32.8 /
+// 30.6; the same at nx = 2..64 and at 1024, 2048; why these three differ was not
+// found).  256-point lines:
 // 16 or 4, never 8 (256 x 16384 9.5 us with 4, 10.7 with 8; 256 x 65536 27.4
 // with 4, 26.9 with 16).  Else as rows_nt (1024 x 1024 5.8 / 4.7 / 4.6 us with
 // 16 / 8 / 4 tiles, 1024 x 4096 9.5 / 8.7 / 9.9, 1024 x 16384 26.1 / 25.9 /
@@ -596,7 +603,10 @@ uint32_t rows_nt_nat(const tcfft_plan_s* p, const Pass& ps) {
         return ps.radix == 1 && nt == 8u && !p->set.tiles ? 4u : nt;
     }
     if (p->set.tiles > 0) return (uint32_t)p->set.tiles;
-    return ps.n_tiles / 16u <= 2u * (uint32_t)p->cus ? 4u : 8u;
+    const uint32_t lines = ps.n_tiles / 16u, cus = (uint32_t)p->cus;
+    const bool mid_nx = p->lay.nx >= 128 && p->lay.nx <= 512;
+    if (p->lay.dims == 2 && !mid_nx && lines >= 6u * cus && lines < 16u * cus) return 16u;
+    return lines <= 2u * cus ? 4u : 8u;
 }
 
 // Waves per workgroup of the natural-order pass: as rows_wg, but four for 2D
