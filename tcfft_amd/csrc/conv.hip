@@ -230,7 +230,11 @@ __global__ __launch_bounds__(64 * W) TCFFT_MFMA_BUDGET void k_dif(const u32* in,
                                                 const float2* __restrict__ wn_lo, u32 wn_lo_bits) {
     extern __shared__ u32 lds[];
     constexpr u32 N = 4096u * W;
-    const int lane = lane_id(), w = W == 1 ? 0 : __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+    // a scalar wave index pays off at four waves (14.6 against 14.9 us for 16384 x
+    // 400), not at two (26.9 against 26.0 us for 8192 x 1600, 76.4 and 75.1 for x
+    // 6400)
+    const int lane = lane_id(), wave = threadIdx.x >> 6;
+    const int w = W == 4 ? __builtin_amdgcn_readfirstlane(wave) : W == 2 ? wave : 0;
     const int c16 = lane & 15, g = lane >> 4;
     Dif4096Tw dtw;
     dif4096_tw_load<W>(dtw, lane, w4096, (u32)w, wn_hi, wn_lo, wn_lo_bits);
