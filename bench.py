@@ -455,10 +455,10 @@ def bench_split_shapes(torch, tcfft_amd, reps):
         ms = graph_time(torch, lambda i, st: plan.exec_split(ins[i % len(ins)].data_ptr(),
                                                              outs[i % len(ins)].data_ptr(), tcfft_amd.FORWARD, st),
                         reps, 3)
-        # algorithmic bytes, each point read and written once: the pass list of
-        # query_split is not what the exec runs (it merges passes)
-        res[name] = {"ms": round(ms, 5), "rel_l2_vs_fp64": err,
-                     "hbm_frac": round(16.0 * per * batch / (ms * 1e-3) / 1e9 / PEAK_HBM_GBS, 4)}
+        npass = len(tcfft_amd.query_split_exec(dims, a, b, batch))
+        frac = 16.0 * per * batch / (ms * 1e-3) / 1e9 / PEAK_HBM_GBS  # each point read and written once
+        res[name] = {"ms": round(ms, 5), "passes": npass, "rel_l2_vs_fp64": err, "hbm_frac": round(frac, 4),
+                     "hbm_frac_per_pass": round(npass * frac, 4)}
         plan.destroy()
         del ins, outs
     return res

@@ -158,9 +158,10 @@ int tcfft_exec_split(tcfft_plan plan, const void *in, void *out, int direction, 
  * counterpart in the reference. */
 int tcfft_plan_prepare_split(tcfft_plan plan);
 
-/* The split-precision pass list tcfft_plan_prepare_split starts from for a shape
+/* The split-precision decomposition of a shape into passes of at most 256 rows
  * (dims 1: n_or_nx = n, ny ignored; dims 2: nx x ny), computed on the host
- * without a device.  Pass i fills desc[5i .. 5i+4] = {R, log2 Q, log2 Qlo,
+ * without a device; what tcfft_exec_split runs where a kernel takes several of
+ * them at once is tcfft_query_split_exec's list.  Pass i fills desc[5i .. 5i+4] = {R, log2 Q, log2 Qlo,
  * log2 M or 0, units}: each signal seen as R rows x Q columns, the R-point
  * DFT down every column, output k of column q = q_hi*Qlo + q_lo times
  * W_M^{q_hi k} (0: no twiddle) stored at q_hi*R*Qlo + k*Qlo + q_lo; units =
@@ -168,6 +169,10 @@ int tcfft_plan_prepare_split(tcfft_plan plan);
  * two-pass kernel): *n_passes = 0.  capacity < passes: TCFFT_INVALID_VALUE
  * with *n_passes set.  No counterpart in the reference. */
 int tcfft_query_split(int dims, int n_or_nx, int ny, int n_batch, int *desc, int capacity, int *n_passes);
+/* The passes tcfft_exec_split runs on a prepared plan of the shape, in the same
+ * form: R up to 4096, and log2 Q = log2 Qlo = 0 for a pass over whole
+ * contiguous lines of R points (units = lines). */
+int tcfft_query_split_exec(int dims, int n_or_nx, int ny, int n_batch, int *desc, int capacity, int *n_passes);
 
 /* Real-input transforms (no counterpart in the reference, whose callers feed
  * real data as complex with zero imaginary parts, e.g. the generator of

@@ -47,7 +47,7 @@ EXPORTS = (
     "tcfft_plan_create_r2c_1d", "tcfft_exec_r2c", "tcfft_exec_c2r", "tcfft_permute_to_dropin",
     "tcfft_exec_natural_noalloc", "tcfft_multi_exec_natural", "tcfft_plan_prepare_split", "tcfft_query_split",
     "tcfft_exec_r2c_adjoint", "tcfft_exec_c2r_adjoint", "tcfft_conv_filter_grad_natural",
-    "tcfft_permute_to_dropin_f32",
+    "tcfft_permute_to_dropin_f32", "tcfft_query_split_exec",
 )
 NOALLOC_SCRATCH_BYTES = 64 << 20  # TCFFT_NOALLOC_SCRATCH_BYTES
 OPT_SPLIT_CHUNK = 1
@@ -103,6 +103,7 @@ def lib():
         L.tcfft_plan_prepare_split.argtypes = [_vp]
         L.tcfft_query_split.argtypes = [ctypes.c_int, ctypes.c_int, ctypes.c_int, ctypes.c_int, _i32p, ctypes.c_int,
                                         _i32p]
+        L.tcfft_query_split_exec.argtypes = L.tcfft_query_split.argtypes
         L.tcfft_plan_set_option.argtypes = [_vp, ctypes.c_int, ctypes.c_int]
         L.tcfft_plan_autotune.argtypes = [_vp, _vp, _vp, _i32p, _i32p, ctypes.POINTER(ctypes.c_float)]
         L.tcfft_plan_create_1d_split.argtypes = [ctypes.POINTER(_vp), ctypes.c_int, ctypes.c_int, ctypes.c_int]
@@ -179,15 +180,26 @@ def query_2d(nx: int, ny: int, batch: int = 1):
     return [int(v) for v in rx[: nrx.value]], [int(v) for v in ry[: nry.value]], npass.value
 
 
-def query_split(dims: int, n_or_nx: int, ny: int = 0, batch: int = 1):
-    """Split-precision pass list of a shape (tcfft_query_split): one dict per
-    pass with R, q_log2, qlo_log2, m_log2 (0 = no twiddle) and units."""
+def _split_passes(name: str, dims: int, n_or_nx: int, ny: int, batch: int):
     desc = np.zeros(5 * 16, dtype=np.int32)
     npass = ctypes.c_int()
-    _check(lib().tcfft_query_split(dims, n_or_nx, ny, batch, desc.ctypes.data_as(_i32p), 16, ctypes.byref(npass)),
-           f"tcfft_query_split(dims={dims}, n_or_nx={n_or_nx}, ny={ny}, batch={batch})")
+    _check(getattr(lib(), name)(dims, n_or_nx, ny, batch, desc.ctypes.data_as(_i32p), 16, ctypes.byref(npass)),
+           f"{name}(dims={dims}, n_or_nx={n_or_nx}, ny={ny}, batch={batch})")
     keys = ("R", "q_log2", "qlo_log2", "m_log2", "units")
     return [dict(zip(keys, (int(v) for v in desc[5 * i: 5 * i + 5]))) for i in range(npass.value)]
+
+
+def query_split(dims: int, n_or_nx: int, ny: int = 0, batch: int = 1):
+    """Split-precision decomposition of a shape into passes of at most 256 rows
+    (tcfft_query_split): one dict per pass with R, q_log2, qlo_log2, m_log2 (0
+    = no twiddle) and units."""
+    return _split_passes("tcfft_query_split", dims, n_or_nx, ny, batch)
+
+
+def query_split_exec(dims: int, n_or_nx: int, ny: int = 0, batch: int = 1):
+    """The passes exec_split runs, in the same form; q_log2 = 0 for a pass over
+    whole contiguous lines of R points (tcfft_query_split_exec)."""
+    return _split_passes("tcfft_query_split_exec", dims, n_or_nx, ny, batch)
 
 
 class _Plan:

@@ -950,14 +950,15 @@ int tcfft_query_2d(int nx, int ny, int n_batch, int* radices_x, int* n_radices_x
     return copy_radices(lay.rad_y, radices_y, capacity, n_radices_y);
 }
 
-int tcfft_query_split(int dims, int n_or_nx, int ny, int n_batch, int* desc, int capacity, int* n_passes) {
+static int query_split_list(decltype(&split_steps_of) list, int dims, int n_or_nx, int ny, int n_batch, int* desc,
+                            int capacity, int* n_passes) {
     if (!n_passes || (capacity > 0 && !desc)) return TCFFT_INVALID_POINTER;
     Layout lay;
     int rc = dims == 1 ? build_layout_1d(n_or_nx, n_batch, lay)
                        : dims == 2 ? build_layout_2d(n_or_nx, ny, n_batch, lay) : TCFFT_INVALID_VALUE;
     if (rc) return rc;
     std::vector<tcfft_plan_s::SplitStep> steps;
-    rc = split_steps_of(dims, n_or_nx, ny, n_batch, steps);
+    rc = list(dims, n_or_nx, ny, n_batch, steps);
     if (rc) return rc;
     *n_passes = (int)steps.size();
     if ((int)steps.size() > capacity) return TCFFT_INVALID_VALUE;
@@ -971,6 +972,14 @@ int tcfft_query_split(int dims, int n_or_nx, int ny, int n_batch, int* desc, int
         d[4] = (int)s.a.units;
     }
     return TCFFT_SUCCESS;
+}
+
+int tcfft_query_split(int dims, int n_or_nx, int ny, int n_batch, int* desc, int capacity, int* n_passes) {
+    return query_split_list(split_steps_of, dims, n_or_nx, ny, n_batch, desc, capacity, n_passes);
+}
+
+int tcfft_query_split_exec(int dims, int n_or_nx, int ny, int n_batch, int* desc, int capacity, int* n_passes) {
+    return query_split_list(split_exec_steps_of, dims, n_or_nx, ny, n_batch, desc, capacity, n_passes);
 }
 
 int tcfft_exec(tcfft_plan plan, void* data, int direction, void* stream) {
