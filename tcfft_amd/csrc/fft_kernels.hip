@@ -1438,7 +1438,6 @@ __global__ __launch_bounds__(64 * W) TCFFT_MFMA_BUDGET void k_big_nat(
     constexpr u32 N = 4096u * W;
     start_delay(sched);
     const int lane = lane_id();
-    const int c16 = lane & 15, g = lane >> 4;
     const u32 w = (u32)__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
     const u32 sig = blockIdx.x;
     BigTw bt;
@@ -1722,7 +1721,6 @@ __global__ __launch_bounds__(64 * W) TCFFT_MFMA_BUDGET void k_r2c_big(
     constexpr u32 L = 4096u * W;
     start_delay(sched);
     const int lane = lane_id();
-    const int c16 = lane & 15, g = lane >> 4;
     const u32 w = (u32)__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
     const u32 sig = blockIdx.x;
     BigTw bt;
@@ -1779,7 +1777,6 @@ __global__ __launch_bounds__(64 * W) TCFFT_MFMA_BUDGET void k_c2r_big(
     constexpr u32 L = 4096u * W;
     start_delay(sched);
     const int lane = lane_id();
-    const int c16 = lane & 15, g = lane >> 4;
     const u32 w = (u32)__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
     const u32 sig = blockIdx.x;
     BigTw bt;
@@ -2501,7 +2498,6 @@ __device__ __forceinline__ void multi_big_nat(const u32* in, u32* out, const Mul
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int grp = wave / W, w = wave % W;
     const int lane = lane_id();
-    const int c16 = lane & 15, g = lane >> 4;
     // a group without a signal (last task of a class) reads the task's first
     // signal, so that every load stays in bounds, and stores nothing
     const bool active = grp < (int)tk.count;

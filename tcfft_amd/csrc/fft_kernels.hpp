@@ -69,7 +69,7 @@ hipError_t launch_split_65536(const float2* in, float2* mid, float2* out, uint32
 // columns (element (r, q) at r*Q + q); the R-point DFT down every column,
 // output k of column q = q_hi*Qlo + q_lo times W_M^{q_hi k} (M = R*Q/Qlo;
 // m_mask = 0: no twiddle), stored at q_hi*R*Qlo + k*Qlo + q_lo.  Qlo = 1 is
-// the row store (row = true); otherwise Qlo >= 16.  R = 16..256 on MFMA,
+// the row store (row = true, R >= 64); otherwise Qlo >= 16.  R = 16..256 on MFMA,
 // R = 512..2048 in a workgroup (with a twiddle only as row store),
 // R = 2, 4, 8 (no twiddle, Qlo = Q) on VALU.  src != dst unless Qlo = Q.
 struct SplitPassArgs {

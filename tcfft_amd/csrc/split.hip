@@ -1260,12 +1260,9 @@ static hipError_t launch_pass_s(int R, bool row, const float2* src, float2* dst,
     case 2: return row ? hipErrorInvalidValue : launch_small_t<2, SIGN>(src, dst, a, st);
     case 4: return row ? hipErrorInvalidValue : launch_small_t<4, SIGN>(src, dst, a, st);
     case 8: return row ? hipErrorInvalidValue : launch_small_t<8, SIGN>(src, dst, a, st);
-    case 16:
-        return row ? launch_pass_t<16, true, SIGN>(src, dst, a, w4096, sched, st)
-                   : launch_pass_t<16, false, SIGN>(src, dst, a, w4096, sched, st);
-    case 32:
-        return row ? launch_pass_t<32, true, SIGN>(src, dst, a, w4096, sched, st)
-                   : launch_pass_t<32, false, SIGN>(src, dst, a, w4096, sched, st);
+    // contiguous axes start with 64 rows or more (shorter ones are k_split_rows)
+    case 16: return row ? hipErrorInvalidValue : launch_pass_t<16, false, SIGN>(src, dst, a, w4096, sched, st);
+    case 32: return row ? hipErrorInvalidValue : launch_pass_t<32, false, SIGN>(src, dst, a, w4096, sched, st);
     case 64:
         return row ? launch_pass_t<64, true, SIGN>(src, dst, a, w4096, sched, st)
                    : launch_pass_t<64, false, SIGN>(src, dst, a, w4096, sched, st);
