@@ -349,39 +349,41 @@ __global__ __launch_bounds__(256) void k_conv_wgrad(const u32* __restrict__ xs, 
 // order: position p = d0 + 16*d1 + 256*d2 + 4096*d3 goes to index d3 + W*(d2 +
 // 16*d1 + 256*d0).  Bound by the two spectra's reads, so the reordering
 // happens on the FP32 sums in LDS on their way out.  A workgroup owns the
-// positions with D adjacent d1: reads in runs of 16*D words (16*W runs, d2 and
-// d3), writes in 16 runs (d0) of 16*W*D indices.  A thread sums four adjacent
-// words of S runs.  LDS element of (d0, j = d3 + W*d2 + 16*W*(d1 mod D)):
-// 16*W*D*d0 + (j ^ d0), 8 bytes each.  Measured at 256 channels x 8192 over 32
-// batch entries: sums in digit-reversed order 92 us and a gather of them 23
-// (8-byte reads 64 KiB apart); 92.5 in one.
-template <int W, int D>
-__global__ __launch_bounds__(256) void k_conv_wgrad_nat(const u32* __restrict__ xs, const u32* __restrict__ gs,
-                                                        float2* __restrict__ gh, u32 channels, u32 batch,
-                                                        float scale) {
-    static_assert(D == 1 || D == 4, "one or four d1 per workgroup");
-    constexpr u32 N = 4096u * W, ROW = 16u * W * D;
-    constexpr int THREADS = D == 4 ? 256 : 64 * W, S = D == 4 ? W : 1;
+// positions with four adjacent d1 (reads in runs of 64 words, whole cache
+// lines) and Q adjacent d2, of every d3: 4*(16/Q) workgroups a channel.  It
+// writes 64 runs (d0, d1) of Q*W indices.  A thread sums four adjacent words of
+// S runs (d3), U batch entries' loads in flight.  LDS element of (d0, j = d3 +
+// W*d2 + W*Q*(d1 mod 4)): 4*W*Q*d0 + (j ^ d0), 8 bytes each.  Measured at 256
+// channels x 8192 over 32 batch entries: sums in digit-reversed order 92 us and
+// a gather of them 23 (8-byte reads 64 KiB apart); 92.5 in one.
+template <int W, int Q, int S, int U>
+__global__ __launch_bounds__(16 * Q * W / S) void k_conv_wgrad_nat(const u32* __restrict__ xs,
+                                                                 const u32* __restrict__ gs,
+                                                                 float2* __restrict__ gh, u32 channels, u32 batch,
+                                                                 float scale) {
+    static_assert(16 % Q == 0 && W % S == 0 && W * Q >= 4, "whole runs; the swizzle stays in a row");
+    constexpr u32 N = 4096u * W, RUN = W * Q, ROW = 4u * RUN;
+    constexpr int THREADS = 16 * Q * W / S;
     __shared__ float2 tile[16 * ROW];
-    const u32 tid = threadIdx.x;
-    const u32 ch = blockIdx.x / (16u / D), d1h = blockIdx.x % (16u / D);
-    const u32 q = tid % (4u * D), d2 = tid / (4u * D) & 15u, d3 = D == 4 ? 0u : tid >> 6;
-    const size_t base = (size_t)ch * N + 16u * D * d1h + 256u * d2 + 4096u * d3 + 4u * q;
+    const u32 tid = threadIdx.x, part = blockIdx.x % (64u / Q);
+    const u32 ch = blockIdx.x / (64u / Q), d1h = part / (16u / Q), d2h = part % (16u / Q);
+    const u32 q = tid % 16u, d2 = tid / 16u % Q, d3 = tid / (16u * Q) * S;
+    const size_t base = (size_t)ch * N + 64u * d1h + 256u * (Q * d2h + d2) + 4096u * d3 + 4u * q;
     const size_t step = (size_t)channels * N;
     cf acc[S][4] = {};
-    // U batch entries' loads in flight per thread, then one at a time
+    // U batch entries, then one at a time
     auto sum = [&](auto u_const, u32 b) {
-        constexpr int U = decltype(u_const)::value;
-        u32 x[U][S][4], g[U][S][4];
+        constexpr int NB = decltype(u_const)::value;
+        u32 x[NB][S][4], g[NB][S][4];
 #pragma unroll
-        for (int u = 0; u < U; ++u)
+        for (int u = 0; u < NB; ++u)
 #pragma unroll
             for (int s = 0; s < S; ++s) {
                 load4_nt(x[u][s], xs + base + (b + u) * step + 4096u * s);
                 load4_nt(g[u][s], gs + base + (b + u) * step + 4096u * s);
             }
 #pragma unroll
-        for (int u = 0; u < U; ++u)
+        for (int u = 0; u < NB; ++u)
 #pragma unroll
             for (int s = 0; s < S; ++s)
 #pragma unroll
@@ -391,24 +393,23 @@ __global__ __launch_bounds__(256) void k_conv_wgrad_nat(const u32* __restrict__ 
                     acc[s][i].y += a.x * c.y - a.y * c.x;
                 }
     };
-    constexpr u32 U = D == 1 ? 8 : 8 / W;
     u32 b = 0;
-    for (; b + U <= batch; b += U) sum(std::integral_constant<int, (int)U>{}, b);
+    for (; b + U <= batch; b += U) sum(std::integral_constant<int, U>{}, b);
     for (; b < batch; ++b) sum(std::integral_constant<int, 1>{}, b);
-    // words 4q + i: d0 = 4*(q & 3) + i, d1 mod D = q >> 2
+    // words 4q + i: d0 = 4*(q & 3) + i, d1 mod 4 = q >> 2
 #pragma unroll
     for (int s = 0; s < S; ++s)
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
-            const u32 d0 = 4u * (q & 3u) + i, j = d3 + (u32)s + W * d2 + 16u * W * (q >> 2);
+            const u32 d0 = 4u * (q & 3u) + i, j = d3 + (u32)s + W * d2 + RUN * (q >> 2);
             tile[ROW * d0 + (j ^ d0)] = make_float2(acc[s][i].x * scale, acc[s][i].y * scale);
         }
     __syncthreads();
-    float2* const o = gh + (size_t)ch * N + ROW * d1h;
+    float2* const o = gh + (size_t)ch * N + 64u * W * d1h + RUN * d2h;
 #pragma unroll
-    for (u32 e = tid; e < 16u * ROW; e += THREADS) {
-        const u32 d0 = e / ROW, j = e % ROW;
-        o[256u * W * d0 + j] = tile[ROW * d0 + (j ^ d0)];
+    for (u32 k = 0; k < 16u * ROW / THREADS; ++k) {
+        const u32 e = tid + k * THREADS, d0 = e / ROW, j = e % ROW;
+        o[256u * W * d0 + 16u * W * (j / RUN) + j % RUN] = tile[ROW * d0 + (j ^ d0)];
     }
 }
 
@@ -489,17 +490,23 @@ hipError_t launch_conv_wgrad(const uint32_t* xs, const uint32_t* gs, float2* gh,
     return hipGetLastError();
 }
 
-// Four d1 per workgroup (256-byte reads) when that gives at least a workgroup
-// per CU, else one (64-byte reads, four times the workgroups).
+// Every d2 in a workgroup and all d3 in a thread (long runs to write) when that
+// gives at least a workgroup per CU, else four d2 and one d3, four times the
+// workgroups and W times their threads.  Channels x batch entries, the former /
+// the latter / sums in digit-reversed order and a gather: n = 16384, 1 x 100 148 /
+// 22.4 / 39.1 us, 32 x 32 53.7 / 24.7 / 34.6, 128 x 8 28.1 / 30.2 / 43.1; n = 8192,
+// 16 x 64 27.2 / 16.7 / 41.0, 48 x 16 12.2 / 10.9 / 21.9, 64 x 16 13.4 / 14.2 / 23.0;
+// n = 4096, 1 x 100 29.0 / 20.7 / 20.7, 32 x 32 12.2 / 9.9 / 19.2, 63 x 16 8.7 /
+// 8.8 / 15.9.
 template <int W>
 static void launch_wgrad_nat_t(const u32* xs, const u32* gs, float2* gh, u32 channels, u32 batch, float scale, u32 cus,
                                hipStream_t st) {
     if (4u * channels >= cus)
-        hipLaunchKernelGGL((k_conv_wgrad_nat<W, 4>), dim3(4u * channels), dim3(256), 0, st, xs, gs, gh, channels,
-                           batch, scale);
+        hipLaunchKernelGGL((k_conv_wgrad_nat<W, 16, W, 8 / W>), dim3(4u * channels), dim3(256), 0, st, xs, gs, gh,
+                           channels, batch, scale);
     else
-        hipLaunchKernelGGL((k_conv_wgrad_nat<W, 1>), dim3(16u * channels), dim3(64 * W), 0, st, xs, gs, gh, channels,
-                           batch, scale);
+        hipLaunchKernelGGL((k_conv_wgrad_nat<W, 4, 1, 4>), dim3(16u * channels), dim3(64 * W), 0, st, xs, gs, gh,
+                           channels, batch, scale);
 }
 
 hipError_t launch_conv_wgrad_nat(int W, const uint32_t* xs, const uint32_t* gs, float2* gh, uint32_t channels,
