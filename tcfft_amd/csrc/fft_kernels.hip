@@ -1869,9 +1869,9 @@ static KernelInfo kernel_info(K kernel, int threads, size_t lds) {
 }
 
 // Waves per workgroup of the kernels whose waves each own a 16 KiB LDS slice
-// (k_r2c, k_c2r): four, or one when the grid has fewer than four
-// waves per CU, where four-wave workgroups would leave most CUs idle
-// (1024 x 1024 natural order: 64 workgroups on 256 CUs).
+// (k_r2c, k_c2r): four, or one when the grid has fewer than four waves per CU,
+// where four-wave workgroups would leave most CUs idle (rfft of 64 x 8192: 16
+// workgroups on 256 CUs; 10.2 -> 9.05 us).
 template <class K>
 static u32 slice_wg(K kernel, u32 waves) {
     const KernelInfo k4 = kernel_info(kernel, 256, 4 * 4096 * sizeof(u32));

@@ -404,7 +404,10 @@ int split_steps_of(int dims, int n_or_nx, int ny, int batch, std::vector<tcfft_p
 // kernel holds more than a pass of the list:
 //   a contiguous axis of 256..4096 points: whole lines (k_split_rows);
 //   1D 2^17..2^22 points: two passes of radix 256..2048 instead of three;
-//   a strided axis of 512..2048 points: one pass (k_split_colsw).
+//   a strided axis of 512..2048 points: one pass (k_split_colsw), at every
+//   grid: whole calls with the list's two passes there / with one, 512 x 256 x 1
+//   34.0 / 13.1 us, x 16 40.9 / 22.4, 1024 x 256 x 1 30.8 / 15.8, 2048 x 256 x 1 31.6 /
+//   22.6, x 4 40.9 / 29.0, 2048 x 1024 x 4 80.2 / 57.7 (both without a start delay).
 int split_exec_steps_of(int dims, int n_or_nx, int ny, int batch, std::vector<tcfft_plan_s::SplitStep>& steps) {
     std::vector<tcfft_plan_s::SplitStep> list;
     const int rc = split_steps_of(dims, n_or_nx, ny, batch, list);
@@ -513,7 +516,9 @@ bool valid(tcfft_plan p) { return p && p->magic == kMagic; }
 // 27.66, no stagger 28.13; natural order 5 groups delay 3 37.40 us, 7 groups
 // delay 2 37.11, 3 groups delay 2 38.59.
 // A grid of less than one wave per SIMD has nothing to stagger (natural order,
-// 8192 x 100: 8.9 us with the delay, 7.1 without; 16384 x 64 10.6 and 9.8).
+// 8192 x 100: 8.9 us with the delay, 7.1 without; 16384 x 64 10.6 and 9.8;
+// drop-in behind a copy of its input, 8192 x 128 10.6 and 8.9, 16384 x 64 11.5
+// and 10.3, 32768 x 32 16.1 and 14.9, the first pass of 2^20 x 2 32.0 and 30.2).
 tcfft::StartSched big_sched(const tcfft_plan_s* p, int W, uint32_t lines) {
     const bool small = (uint64_t)lines * (uint32_t)W < 4u * (uint64_t)p->cus;
     const int delay = p->big_delay >= 0 ? p->big_delay : small ? 0 : (W == 4 || W == 8 ? 1 : 2);
@@ -583,20 +588,19 @@ uint32_t rows_nt(const tcfft_plan_s* p, const Pass& ps, int setting) {
 
 // The same for the natural-order pass.  4096-point lines: four waves per line
 // up to two lines per CU, two above (out of place, random input; one / two /
-// four waves per line: 4096 x 256 6.7 / 5.4 / 5.0 us, 4096 x 512 7.5 / 6.2 /
-// 5.4, 4096 x 1024 8.4 / 7.8 / 8.2, 4096 x 2048 12.9 / 12.0 / 13.9, 4096 x
-// 4096 27.3 / 22.7 / 24.0, 4096 x 16384 95.6 / 90.7 / 107).  2D lines go to
+// four waves per line: 4096 x 256 5.9 / 4.9 / 4.8 us, 4096 x 512 6.7 / 6.5 /
+// 5.8, 4096 x 1024 9.0 / 7.7 / 8.0, 4096 x 2048 13.2 / 12.0 / 13.8, 4096 x
+// 4096 27.0 / 22.8 / 23.9, 4096 x 16384 96 / 93 / 110).  2D lines go to
 // permuted places: one wave per line from 6 to below 16 lines per CU (whole
 // transforms, one / two waves: 16 x 4096 x 96 22.9 / 23.4 us, x 128 27.6 / 28.9,
 // x 192 36.6 / 39.3, x 256 48.7 / 48.2, x 384 69.7 / 68.7; 1024 x 4096 x 2 31.9 /
 // 33.3, x 3 39.9 / 43.7), except for nx = 128..512, where two stay ahead (128 x
 // 4096 x 16 28.4 / 26.7, 256 x 4096 x 16 51.2 / 48.2, 512 x 4096 x 4 32.8 /
 // 30.6; the same at nx = 2..64 and at 1024, 2048; why these three differ was not
-// found).  256-point lines:
-// 16 or 4, never 8 (256 x 16384 9.5 us with 4, 10.7 with 8; 256 x 65536 27.4
-// with 4, 26.9 with 16).  Else as rows_nt (1024 x 1024 5.8 / 4.7 / 4.6 us with
-// 16 / 8 / 4 tiles, 1024 x 4096 9.5 / 8.7 / 9.9, 1024 x 16384 26.1 / 25.9 /
-// 28.7).
+// found).  256-point lines: 16 or 4, never 8 (256 x 16384 9.4 us with 4, 10.5
+// with 8; 256 x 65536 26.9 with 4, 35 with 8, 26.8 with 16).  Else as rows_nt
+// (1024 x 1024 5.6 / 4.4 / 4.2 us with 16 / 8 / 4 tiles, 1024 x 4096 9.3 / 8.4 /
+// 9.7, 1024 x 16384 25.7 / 25.7 / 28.8).
 uint32_t rows_nt_nat(const tcfft_plan_s* p, const Pass& ps) {
     if (ps.radix < 16) {
         const uint32_t nt = rows_nt(p, ps, p->set.tiles);
