@@ -518,7 +518,7 @@ bool valid(tcfft_plan p) { return p && p->magic == kMagic; }
 // A grid of less than one wave per SIMD has nothing to stagger (natural order,
 // 8192 x 100: 8.9 us with the delay, 7.1 without; 16384 x 64 10.6 and 9.8;
 // drop-in behind a copy of its input, 8192 x 128 10.6 and 8.9, 16384 x 64 11.5
-// and 10.3, 32768 x 32 16.1 and 14.9, the first pass of 2^20 x 2 32.0 and 30.2).
+// and 10.3, 32768 x 32 16.1 and 14.9, both passes of 2^20 x 2 32.0 and 30.2).
 tcfft::StartSched big_sched(const tcfft_plan_s* p, int W, uint32_t lines) {
     const bool small = (uint64_t)lines * (uint32_t)W < 4u * (uint64_t)p->cus;
     const int delay = p->big_delay >= 0 ? p->big_delay : small ? 0 : (W == 4 || W == 8 ? 1 : 2);
